@@ -225,6 +225,8 @@ def bench_uneven(ctx, torch, stream, n, steps, log):
         def label(cd):
             if cd["layout"] == "lane":
                 return "lane" + (" (lower bound, pruned)" if cd.get("pruned") else "")
+            if cd.get("windowed"):
+                return "windowed"
             return (f'{cd["rows_per_lane"]}x{cd["lanes"]}'
                     f'{" persistent" if cd["persistent"] else " static"}')
         # every candidate's time on the bucket's sample (ms), for the record

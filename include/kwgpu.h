@@ -154,7 +154,7 @@ int kwgpu_fd1d_price_device(kwgpu_ctx* ctx, const kwgpu_option* d_opts, size_t n
  * grids included, on device-resident options, prices and status, asynchronous on
  * `stream`; here params->x_dims / params->t_dims, when set, are HOST arrays of n sizes.
  * The PDE order, the sizes and the bucket counters of the batch live in a fixed device
- * scratch array of the library (12 MiB per device, held until the process ends): at most
+ * scratch array of the library (24 MiB per device, held until the process ends): at most
  * 1048576 options (more returns KWGPU_ERR_INVALID), wave layout only (x_dim <= 2048, else
  * KWGPU_ERR_UNSUPPORTED). No graph and no side stream: the grid-size buckets run one
  * after another on `stream`. Calls on one context are ordered; calls from different
@@ -204,7 +204,8 @@ int kwgpu_fd1d_greeks(kwgpu_ctx* ctx, const kwgpu_option* opts, size_t n,
  * batch (x-points rounded up to a power of two, 64 .. 2048), times on a sample of the
  * bucket's options each wave-layout variant that holds it (rows per lane x lanes per
  * option: 4, 2 or 1 options per wave, or two waves per option), with a static and with
- * a persistent grid, and in FP64 also the lane layout; keeps the fastest per (bucket,
+ * a persistent grid, and in FP64 also the lane layout and (theta 1/2, over 128 points) the
+ * windowed march, which such grids take untuned; keeps the fastest per (bucket,
  * precision) in the context, which later calls use. `report` (may be NULL) receives a
  * JSON object with every timing. Device pointers as for kwgpu_fd1d_price_device (the
  * sampled options' prices are written); synchronous.

@@ -1,0 +1,135 @@
+// fd1d_plan.h -- which rows of an option's grid its FD march has to carry.
+//
+// The mesh spans +-scale sigma sqrt(T) around the strike (50 standard deviations by
+// default), and most of its rows have a solution that is known beforehand:
+//   * out of the money, beyond a few standard deviations, it is 0: truncating it at
+//     distance b from the strike changes the price at a spot by the share of paths that
+//     reach b and come back to the payoff, exp(-2 b (b - x*) / (sigma^2 T)) of the price
+//     by the reflection principle, whatever the drift (a bridge does not see it);
+//   * in the money, past the exercise boundary b(T), every step ends projected onto the
+//     payoff, so those rows are constant in time. b(tau) moves away from the strike as tau
+//     grows, so rows past b(T) are pinned at every step.
+// Rows are counted as positions from the in-the-money edge of the mesh: position i is row
+// i of a put's grid and row N - 1 - i of a call's, and xi = log(S/K) for a put, -log(S/K)
+// for a call grows with the position. In xi a call is a put with the drift reversed.
+//
+// The window [lo, end) found here is an estimate of where both start to hold, with
+// margins; the march checks the in-the-money cut after its last step and an option whose
+// boundary went past it is solved again on its whole grid. Options outside the rule's
+// domain keep their whole grid (lo = 0, end = N).
+//
+// Host and device code; only the C library's mathematics, so that it can be checked on
+// the CPU.
+#pragma once
+
+#include <math.h>
+
+#include "kwgpu.h"
+
+#ifndef KWGPU_HD
+#define KWGPU_HD __host__ __device__ inline
+#endif
+
+namespace kwgpu {
+
+struct Window {
+    int lo, end;  // positions; lo > 0: the rows before it are pinned to the payoff
+};
+
+// Positions of pinned rows eliminated in front of the window in set-up (fd1d_window.h).
+constexpr int kPinnedRows = 256;
+constexpr int kWindowMinSteps = 64;
+
+// log of the critical spot of an American put with unit strike, rate r > 0 and yield q, in
+// Barone-Adesi & Whaley's approximation: the root of
+//     f(S) = (1 - S) - E(S) + (1 - e^{-qT} Phi(-d1(S))) S / lambda
+// by three Newton steps from their starting value between the perpetual critical spot and
+// min(1, r / q). In FP32: the result only places a cut that is checked afterwards. Over
+// 320000 options (vol 2-150 %, T 0.005-30 years) 36 are off by more than 0.02; a bisection
+// to the last digit costs some 20 evaluations of f and was half the planning time.
+KWGPU_HD float critical_log_spot(float t, float z, float r, float q) {
+    const float z2 = z * z, st = z * sqrtf(t), n = 2.0f * (r - q) / z2 - 1.0f;
+    const float lam = 0.5f * (-n - sqrtf(n * n - 8.0f * r / (z2 * expm1f(-r * t))));
+    const float perp = 0.5f * (-n - sqrtf(n * n + 8.0f * r / z2));
+    const float eq = expf(-q * t), er = expf(-r * t), drift = (r - q + 0.5f * z2) * t;
+    const float lowest = perp / (perp - 1.0f), top = q > r ? r / q : 1.0f;
+    const float h = ((r - q) * t - 2.0f * st) / (1.0f - lowest);
+    float s = lowest + (top - lowest) * expf(h < 0.0f ? h : 0.0f);
+    s = fminf(fmaxf(s, 1e-3f), top);
+    for (int it = 0; it < 3; ++it) {
+        const float d1 = (logf(s) + drift) / st;
+        const float n1 = 1.0f - 0.5f * eq * erfcf(d1 * 0.70710678f);  // 1 - e^{-qT} Phi(-d1)
+        const float n2 = 0.5f * er * erfcf((d1 - st) * 0.70710678f);
+        const float f = (1.0f - s) - (n2 - s * (1.0f - n1)) + n1 * s / lam;
+        const float df = n1 * (1.0f / lam - 1.0f) +
+                         eq * 0.39894228f * expf(-0.5f * d1 * d1) / (lam * st);
+        s = fminf(fmaxf(s - f / df, 0.5f * s), fminf(top, 2.0f * s));
+    }
+    return logf(s);
+}
+
+// The window of option o on an N-point grid marched `steps` steps at theta = 1/2. `far`:
+// the largest xi at which the option's price is asked for (0 or less: at or in the money).
+//
+// Out of the money the bound is b (b - far) >= 18 sigma^2 T, i.e. a relative truncation
+// error of e^-36 = 2e-16. Where the steps are few Crank-Nicolson's tails are heavier than
+// the Gaussian's: at 64 steps the exponent 36 loses 2 n (y^3/3 + ...), y = 36 / (2 n), 0.9.
+//
+// In the money the cut lies 0.04 in log S and 3 rows past the approximate critical spot:
+// about 10 rows of 1024 for a boundary that went past it in none of some 13000 random
+// windows (vol 1-200 %, T 0.005-30 years, rates -3-25 %) at 0.05 and 4, in 1 at 0.03 and 3
+// and in 19 at 0.02 and 2. It needs
+//   * kPinnedRows rows to forget the approximate value they are started from: with
+//     a = theta dt (sigma^2 / 2) / dx^2 at the cut, an error shrinks by about
+//     e^{-1/sqrt(a)} per row, and a <= 150 leaves 1e-9 of an error of O(dt^2);
+//   * early exercise to be worth something: while q > r the boundary never comes nearer than
+//     log(r / q) to the strike, and past 4.5 sigma sqrt(T) the premium is below about 1e-9 of
+//     the price. Such an option keeps the rows its European twin keeps, and with them the
+//     same arithmetic, so that rounding cannot price it below the twin (on 32768 options at
+//     1024 x 1024 the two had differed by up to 9e-11, the smallest such ratio 5.1);
+//   * for a call, the unprojected edge row to be forgotten as well: its value can be
+//     e^{scale sigma sqrt(T)}, 22 sigma sqrt(T) decades, and a row with a < 0.1 takes off
+//     at least one.
+KWGPU_HD Window window_of(const kwgpu_option& o, int N, int steps, double density, double scale,
+                          double far) {
+    Window w{0, N};
+    const double s = o.z * sqrt(o.t), s2 = s * s;
+    const double mu = o.r - o.q - 0.5 * o.z * o.z;
+    // the domain: a march long enough to pay for a second set-up, no overflow anywhere on
+    // the mesh, a drift within a few standard deviations, ordinary rates
+    if (!(steps >= kWindowMinSteps && N >= 128 && s > 0.0 && scale * s <= 150.0 && scale >= 10.0 &&
+          fabs(mu) * o.t <= 3.0 * s && fabs(o.r) <= 1.0 && fabs(o.q) <= 1.0 && far < 1e6))
+        return w;
+    const double Y = asinh(scale * s / density), h = 2.0 * Y / (N - 1);  // mesh step in y
+    const double per = 1.0 / h;
+    {
+        const double u = far > 0.0 ? far : 0.0;
+        const double b = 0.5 * (u + sqrt(u * u + 4.0 * 18.0 * s2));
+        // the mesh must resolve a standard deviation there
+        if (!(sqrt(b * b + density * density) * h <= 0.5 * s)) return w;
+        const double at = (asinh(b / density) + Y) * per;
+        const int e = (int)ceil(at) + 3;
+        if (e < N) w.end = e;
+    }
+    // the put that the option is in xi
+    const double r = o.w < 0 ? o.r : o.q, q = o.w < 0 ? o.q : o.r;
+    if (!o.e || !(r > 0.0)) return w;
+    if (q > r && log(q / r) > 4.5 * s) return w;
+    const double xb = (double)critical_log_spot((float)o.t, (float)o.z, (float)r, (float)q) - 0.04;
+    if (!(xb > -6.9)) return w;  // nor when it is no number
+    const double at = (asinh(xb / density) + Y) * per;
+    const int lo = (int)floor(at) - 3;
+    if (lo < 16 || lo >= w.end - 8) return w;
+    const double dx = sqrt(xb * xb + density * density) * h;
+    const double a1 = 0.25 * s2 / steps;  // a at dx = 1
+    if (!(a1 <= 150.0 * dx * dx)) return w;
+    if (!(o.w < 0)) {
+        const double xa = sqrt(a1 / 0.1) * per;  // about where a = 0.1
+        const double from = xa > -xb ? xa : -xb;
+        if (!((Y - asinh(from / density)) * per >= 22.0 * s + 20.0)) return w;
+    }
+    w.lo = lo;
+    return w;
+}
+
+}  // namespace kwgpu

@@ -28,6 +28,9 @@
 // w_j = g_j - u_j w_{j+1}, B^{-1} V = D^{-1} w, so with a_j = 1 / (theta d_j)
 //     V'_j = a_j w_j - ((1-theta)/theta) V_j              (= a_j w_j - V_j at theta 1/2).
 //
+// FP64 at theta 1/2 marches each option on its window of rows where its grid has more rows
+// than it needs (fd1d_plan.h, fd1d_window.h); what follows holds for both forms.
+//
 // FP64 march: 6 instructions per point and step at theta 1/2 (1 forward, 1 backward,
 // 2 carry fix-ups, 1 correction, 1 projection) plus the scans amortised over M rows.
 // The state, a, l, u and the forward fix-up live in VGPRs; the backward fix-up and the
@@ -44,6 +47,7 @@
 
 #include <algorithm>
 
+#include "fd1d_plan.h"
 #include "kwgpu_internal.h"
 
 namespace kwgpu {
@@ -63,6 +67,7 @@ constexpr int kRowShr = 0x110;   // + n, n in 1..15
 constexpr int kRowShl = 0x100;   // + n
 constexpr int kRowBcast15 = 0x142;
 constexpr int kRowBcast31 = 0x143;
+constexpr int kRowNewBcast = 0x150;  // + n: every lane of a row reads its lane n
 constexpr int kWaveShr1 = 0x138;
 constexpr int kWaveShl1 = 0x130;
 
@@ -120,6 +125,7 @@ struct Lanes {
 
 template <class T>
 struct ScanMul {
+    // (a windowed march's scans, fd1d_window.h, take other windows: see win_fwd_scan)
     T F1, F2, F4, F8, FB15, FB31;  // forward, window products of the lanes' P
     T G1, G2, G4, G8;              // backward, window products of the lanes' Q
     T X16, X32, X48;               // backward across rows: L = 64, nonzero only in the
@@ -141,6 +147,14 @@ struct Pde {
     kwgpu_option opt;
     bool live, solve;
     int N, steps, j0;
+};
+
+// Where a windowed march (fd1d_window.h) begins: the position of its first row and the
+// relation x_{lo-1} = alpha + beta x_lo that the pinned rows before it leave (0, 0 when
+// there are none); k0 is set by setup: what alpha adds to the first row's right-hand side.
+struct Edge {
+    int lo;
+    double alpha, beta, k0;
 };
 
 template <int M, int L, int W>
@@ -175,6 +189,11 @@ __device__ __forceinline__ Pde pde_of(const FdBatch& b, int group, const Lanes& 
     d.steps = d.solve ? td - 1 : 0;
     d.j0 = t.ls * M;
     return d;
+}
+
+// payoff at xi (fd1d_plan.h) in units of K
+__device__ __forceinline__ double payoff_xi(const PdeParams& p, double xi) {
+    return p.call ? fmax(0.0, exp(-xi) - 1.) : fmax(0.0, 1. - exp(xi));
 }
 
 // ---- set-up: grid, operator rows, payoff, LU factors, carry coefficients (FP64) ----
@@ -271,11 +290,14 @@ __device__ __forceinline__ Map2 select_map(bool p, const Map2& x, const Map2& y)
 // TF is the type the march takes the factors, fix-ups and scan multipliers in: double
 // for the FP64 march; float for the FP32-mixed one, which gets each as it is produced
 // (so no FP64 copy of the factor arrays stays live beside the FP32 one).
-template <int M, int L, int W, class TF>
+// WIN: the rows are positions d.j0 .. of a windowed march in xi (d.P's drift has xi's
+// sign), behind `edge`.
+template <int M, int L, int W, bool WIN = false, class TF>
 __device__ __forceinline__ void setup(const FdBatch& b, const Pde& d, const Lanes& t, double* qp,
                                       double (&xv)[M], TF (&ap)[M], TF (&lo)[M],
                                       TF (&up)[M], TF (&R)[M], TF (&Q)[M],
-                                      double (&blv)[M], double (&buv)[M], ScanMul<TF>& sm) {
+                                      double (&blv)[M], double (&buv)[M], ScanMul<TF>& sm,
+                                      Edge* edge = nullptr) {
     using Gm = Geo<M, L, W>;
     constexpr int LT = Gm::LT;
     const PdeParams& P = d.P;
@@ -314,9 +336,21 @@ __device__ __forceinline__ void setup(const FdBatch& b, const Pde& d, const Lane
             ru = rcp(xd - xc);
             rm = rcp(xd - xb);
             b_row_rcp(P, th, j, rl, ru, rm, blv[i], bv[i], buv[i]);
-            xv[i] = j < N ? payoff(P, xc) : 0.0;
+            if constexpr (WIN)
+                xv[i] = j < N ? payoff_xi(P, xc) : 0.0;
+            else
+                xv[i] = j < N ? payoff(P, xc) : 0.0;
             xb = xc;
             xc = xd;
+        }
+    }
+    if constexpr (WIN) {
+        // behind pinned rows the first row's pivot is b + bl beta (an entering pivot of 1
+        // after an upper entry of -beta) and its right-hand side V - bl alpha
+        edge->k0 = 0.0;
+        if (t.ls == 0) {
+            bu_prev = -edge->beta;
+            edge->k0 = -blv[0] * edge->alpha;
         }
     }
 
@@ -381,6 +415,12 @@ __device__ __forceinline__ void setup(const FdBatch& b, const Pde& d, const Lane
     qp[gl] = d0;
     __syncthreads();
     up[M - 1] = (TF)(buv[M - 1] * (t.ls + 1 < LT ? rcp(qp[gl + 1]) : 1.0));
+    if constexpr (WIN) {
+        // no carry enters a window: 0 from the pinned side (alpha is in k0), and x = 0
+        // beyond its end
+        lo[0] = t.ls == 0 ? TF(0) : lo[0];
+        up[M - 1] = t.ls == LT - 1 ? TF(0) : up[M - 1];
+    }
 
     // Carry propagation coefficients: g_j = ghat_j + Pc_j g_in,
     // w_j = what_j + R_j g_in + Q_j w_in.
@@ -409,6 +449,27 @@ __device__ __forceinline__ void setup(const FdBatch& b, const Pde& d, const Lane
         const double w2 = Pl * dpp<kRowShr + 1>(Pl);  // Pl over lanes l-1 .. l
         const double w4 = w2 * dpp<kRowShr + 2>(w2);  // l-3 .. l
         const double w8 = w4 * dpp<kRowShr + 4>(w4);  // l-7 .. l
+        if constexpr (WIN) {
+            // quads first, then quads into rows: prefixes (Pl) and suffixes (Ql) within a quad
+            const int qd = t.lane & 3;
+            double a = Pl, z = Ql, x;
+            x = dpp<kRowShr + 1>(a); a = qd >= 1 ? a * x : a;
+            x = dpp<kRowShr + 2>(a); a = qd >= 2 ? a * x : a;
+            x = dpp<kRowShl + 1>(z); z = qd <= 2 ? z * x : z;
+            x = dpp<kRowShl + 2>(z); z = qd <= 1 ? z * x : z;
+            sm.F1 = qd >= 1 ? Pl : 0.0;
+            sm.F2 = qd >= 2 ? w2 : 0.0;
+            sm.F4 = a;  // taken by the second quad of a half row
+            x = dpp<kRowShr + 4>(a);  // lane 15 of a row: lane 11's
+            const double a11 = dpp<kRowNewBcast + 15>(x);
+            sm.F8 = pr >= 12 ? a * a11 : a;  // ... and by a row's second half
+            sm.G1 = qd <= 2 ? Ql : 0.0;
+            const double q2 = Ql * dpp<kRowShl + 1>(Ql);  // (outside any select, see below)
+            sm.G2 = qd <= 1 ? q2 : 0.0;
+            sm.G4 = z;
+            const double z4 = dpp<kRowNewBcast + 4>(z);
+            sm.G8 = pr < 4 ? z * z4 : z;
+        } else {
         sm.F1 = (TF)(pr >= 1 ? Pl : 0.0);
         sm.F2 = (TF)(pr >= 2 ? w2 : 0.0);
         sm.F4 = (TF)(pr >= 4 ? w4 : 0.0);
@@ -420,6 +481,7 @@ __device__ __forceinline__ void setup(const FdBatch& b, const Pde& d, const Lane
         sm.G2 = (TF)(pr + 2 <= 15 ? v2 : 0.0);
         sm.G4 = (TF)(pr + 4 <= 15 ? v4 : 0.0);
         sm.G8 = (TF)(pr + 8 <= 15 ? v8 : 0.0);
+        }
         // row-inclusive prefix of Pl and suffix of Ql
         double ip = Pl, sq = Ql;
         {
@@ -443,6 +505,10 @@ __device__ __forceinline__ void setup(const FdBatch& b, const Pde& d, const Lane
         sm.X16 = (TF)((w64 && wrow == 0) || (w32 && (wrow & 1) == 0) ? sq : 0.0);
         sm.X32 = (TF)(w64 && wrow == 1 ? sq : 0.0);
         sm.X48 = (TF)(w64 && wrow == 2 ? sq : 0.0);
+        if constexpr (WIN) {
+            sm.X16 = sq;  // rows 0 and 2 take the next row's first lane
+            sm.X32 = wrow == 1 ? sq : wrow == 0 ? sq * rs1 : 0.0;  // rows 0, 1 take lane 32
+        }
         // two-wave groups: Pl over wave 1's lanes 0..l (carry of wave 0's last lane into
         // wave 1) and Ql over wave 0's lanes l..63 (carry of wave 1's first lane back)
         if constexpr (W == 2) {
@@ -521,6 +587,67 @@ __device__ __forceinline__ T bwd_scan(T cb, const ScanMul<T>& sm, const Lanes& t
         cb = fma(sm.X16, src, cb);
     }
     return cb;
+}
+
+// The scans of a windowed march: the same inclusive scans in fewer instructions. gfx950 has
+// one DPP control for 64-bit operands, row_newbcast (every lane of a row reads one lane of
+// it), and v_fmac_f64 takes it; a Kogge-Stone stage costs two 32-bit DPP moves and an FMA.
+// So only the two stages within a quad of lanes are Kogge-Stone; quads are then joined into
+// half rows and rows by broadcasting the last lane of the lower part (Sklansky's scheme),
+// one v_fmac_f64 for each source, the taking lanes selected by the instruction's bank and
+// row masks. 34 instructions for the two scans of 64 lanes instead of 43, 32 instead of 38
+// and two branches for 32, 26 instead of 32 for 16.
+template <int LANE, int ROWS, int BANKS, bool LAST = false>
+__device__ __forceinline__ double fmac_newbcast(double acc, double src, double mul) {
+    // acc += src[LANE of the row] * mul in the lanes of the given rows and quads. A DPP read
+    // wants two wait states after the VALU write of its register: waited for here before the
+    // read and, where a DPP move follows (LAST), after the write, as the compiler does not
+    // look into the assembly.
+    if constexpr (LAST)
+        asm("s_nop 1\n\t"
+            "v_fmac_f64_dpp %0, %1, %2 row_newbcast:%3 row_mask:%4 bank_mask:%5\n\t"
+            "s_nop 1"
+            : "+v"(acc)
+            : "v"(src), "v"(mul), "n"(LANE), "n"(ROWS), "n"(BANKS));
+    else
+        asm("s_nop 1\n\t"
+            "v_fmac_f64_dpp %0, %1, %2 row_newbcast:%3 row_mask:%4 bank_mask:%5"
+            : "+v"(acc)
+            : "v"(src), "v"(mul), "n"(LANE), "n"(ROWS), "n"(BANKS));
+    return acc;
+}
+template <int L>
+__device__ __forceinline__ double win_fwd_scan(double c, const ScanMul<double>& sm) {
+    c = fma(sm.F1, dpp<kRowShr + 1>(c), c);
+    const double s2 = dpp<kRowShr + 2>(c);
+    c = fma(sm.F2, s2, c);
+    c = fmac_newbcast<3, 0xF, 0x2>(c, c, sm.F4);
+    c = fmac_newbcast<11, 0xF, 0x8>(c, c, sm.F4);
+    c = fmac_newbcast<7, 0xF, 0xC, true>(c, c, sm.F8);
+    double s = s2;  // rows outside a broadcast's mask keep a finite value of their own option
+    if constexpr (L >= 32) {
+        s = dpp<kRowBcast15, 0xA>(c, s);
+        c = fma(sm.FB15, s, c);
+    }
+    if constexpr (L == 64) {
+        s = dpp<kRowBcast31, 0xC>(c, s);
+        c = fma(sm.FB31, s, c);
+    }
+    return c;
+}
+template <int L>
+__device__ __forceinline__ double win_bwd_scan(double c, const ScanMul<double>& sm) {
+    c = fma(sm.G1, dpp<kRowShl + 1>(c), c);
+    c = fma(sm.G2, dpp<kRowShl + 2>(c), c);
+    c = fmac_newbcast<4, 0xF, 0x1>(c, c, sm.G4);
+    c = fmac_newbcast<12, 0xF, 0x4>(c, c, sm.G4);
+    c = fmac_newbcast<8, 0xF, 0x3, true>(c, c, sm.G8);
+    if constexpr (L >= 32) {
+        // rows 0 and 2 take the first lane of the next row: one lane down, then across the row
+        c = fmac_newbcast<15, 0x5, 0xF, true>(c, dpp<kWaveShl1>(c), sm.X16);
+    }
+    if constexpr (L == 64) c = fma(sm.X32, readlane<32>(c), c);
+    return c;
 }
 
 // Carries of one step: forward scan of `c` (the lanes' local last values) giving each
@@ -636,13 +763,15 @@ __device__ __forceinline__ void interpolate(const FdBatch& b, const Pde& d, cons
 // a single FMA a_j w_j - V_j. Steps [0, wmin) are taken by every segment of the
 // workgroup, steps [wmin, wsteps) only by segments whose own march (`steps`) lasts that
 // long (several options per workgroup).
-template <int M, int L, int W, bool HALF>
+// WIN: a windowed march, whose first row's right-hand side takes k0.
+template <int M, int L, int W, bool HALF, bool WIN = false>
 __device__ __forceinline__ void march_f64(double (&xv)[M], const double (&ap)[M],
                                           const double (&lo)[M], const double (&up)[M],
                                           const double (&R)[M], const double2* qpv,
                                           const ScanMul<double>& sm, const Lanes& t,
                                           bool first_lane, bool last_lane, double* xchg,
-                                          int wmin, int wsteps, int steps, double c_th) {
+                                          int wmin, int wsteps, int steps, double c_th,
+                                          double k0 = 0.0) {
     constexpr int NT = Geo<M, L, W>::NT;
     constexpr bool ONE = Geo<M, L, W>::G == 1;  // one option per workgroup
     // LDS reads of the (Q, payoff) pairs in flight ahead of the row updates. Measured on
@@ -651,10 +780,16 @@ __device__ __forceinline__ void march_f64(double (&xv)[M], const double (&ap)[M]
     // where the extra registers turn into spill reloads inside the step loop; the
     // 256- and 512-point kernels (4 and 2 options per wave) 2.69 and 5.34 ms at 0, 2.88
     // and 6.33 at 3.
-    constexpr int PF0 = W == 2 ? KWGPU_PF2 : ONE ? KWGPU_PF1 : KWGPU_PFG;
+    // Windowed marches hold fewer scan multipliers and no branch, and have the registers for
+    // it at every width. 16384 options, 512 steps, on 256- and 512-point grids (16-lane
+    // options mostly) and on 1024 points (32- and 64-lane ones): 741, 1088 and 1840 us with
+    // the pairs read at the point of use, 566, 890 and 1525 us read 4 ahead; 2 to 8 ahead
+    // differ by less than 3 %.
+    constexpr int PF0 = WIN ? (ONE ? 3 : 4) : W == 2 ? KWGPU_PF2 : ONE ? KWGPU_PF1 : KWGPU_PFG;
     constexpr int PF = PF0 < M ? PF0 : M - 1;  // 0: each pair read where it is used
     const int wv = __builtin_amdgcn_readfirstlane(t.wv);  // wave of a W = 2 group
     double g[M];
+    auto first = [&](double v) { return WIN ? v + k0 : v; };  // the first row's V
     // backward substitution of g in place and the step's carries: g_in (forward) and
     // w_in (backward) of this lane
     auto carries = [&](int step, double& gin, double& win) {
@@ -679,6 +814,11 @@ __device__ __forceinline__ void march_f64(double (&xv)[M], const double (&ap)[M]
             const double2 ab = qpv[M * NT + t.gl];
             gin = fma(ab.x, u, gin);
             win = fma(ab.y, u, win);
+        } else if constexpr (WIN) {
+            gin = dpp<kWaveShr1>(win_fwd_scan<L>(c, sm));
+            if constexpr (L < 64) gin = first_lane ? 0.0 : gin;
+            win = dpp<kWaveShl1>(win_bwd_scan<L>(fma(R[0], gin, g[0]), sm));
+            if constexpr (L < 64) win = last_lane ? 0.0 : win;
         } else {
             gin = fwd_carry<L, W>(c, sm, t, first_lane, xchg);
             win = bwd_carry<L, W>(fma(R[0], gin, g[0]), sm, t, last_lane, xchg);
@@ -689,7 +829,7 @@ __device__ __forceinline__ void march_f64(double (&xv)[M], const double (&ap)[M]
     // the substitution is a dependent chain of M FMAs, the row updates are independent
     // of each other, so interleaved they fill the chain's latency.
     if (wmin > 0) {
-        g[0] = xv[0];
+        g[0] = first(xv[0]);
 #pragma unroll
         for (int i = 1; i < M; ++i) g[i] = fma(-lo[i], g[i - 1], xv[i]);
     }
@@ -716,14 +856,14 @@ __device__ __forceinline__ void march_f64(double (&xv)[M], const double (&ap)[M]
             w = fma(qv.x, win, w);
             const double v = HALF ? fma(ap[i], w, -xv[i]) : fma(ap[i], w, -c_th * xv[i]);
             xv[i] = vmax(v, qv.y);
-            g[i] = i == 0 ? xv[0] : fma(-lo[i], g[i - 1], xv[i]);  // next step's
+            g[i] = i == 0 ? first(xv[0]) : fma(-lo[i], g[i - 1], xv[i]);  // next step's
         }
     }
     // Steps only the longer segments take (several options per workgroup): lanes whose
     // own march is done keep their values.
     if constexpr (!ONE) {
         for (int step = wmin; step < wsteps; ++step) {
-            g[0] = xv[0];
+            g[0] = first(xv[0]);
 #pragma unroll
             for (int i = 1; i < M; ++i) g[i] = fma(-lo[i], g[i - 1], xv[i]);
             double gin, win;
@@ -917,6 +1057,8 @@ void fd1d_wave(FdBatch b, int* queue, int ngroups) {
     }
 }
 
+#include "fd1d_window.h"
+
 __global__ void zero_counters(int* c, int n) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i < n) c[i] = 0;
@@ -1006,6 +1148,32 @@ hipError_t launch_fd1d_wave(const FdBatch& b, int max_x_dim, int precision, hipS
                             int* queue) {
     if (!wave_layout_fits(max_x_dim, precision)) return hipErrorInvalidValue;
     return launch_fd1d_wave_variant(b, default_wave_variant(max_x_dim), precision, s, queue);
+}
+
+hipError_t launch_fd1d_lone(const FdBatch& b, hipStream_t s) {
+    if (b.m <= 0) return hipSuccess;
+    if (b.theta != 0.5) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(fd1d_lone, dim3(b.m), dim3(64), 0, s, b);
+    return hipGetLastError();
+}
+
+hipError_t launch_fd1d_windowed(const FdBatch& b, const WindowScratch& w, int n_big,
+                                hipStream_t s) {
+    if (b.m <= 0) return hipSuccess;
+    if (b.theta != 0.5 || !w.rec || !w.list || !w.counts) return hipErrorInvalidValue;
+    if (n_big == 0 && b.m <= kLoneMax) return launch_fd1d_lone(b, s);
+    int* cursor = w.counts + kWindowCounters / 2;
+    const unsigned nb = (unsigned)((b.m + 255) / 256);
+    if (hipError_t e = launch_zero_counters(w.counts, kWindowCounters, s)) return e;
+    hipLaunchKernelGGL(plan_windows, dim3(nb), dim3(256), 0, s, b, w.rec, w.counts);
+    hipLaunchKernelGGL(list_windows, dim3(nb), dim3(256), 0, s, b, (const int*)w.rec,
+                       (const int*)w.counts, cursor, w.list);
+    hipLaunchKernelGGL(fd1d_windowed, dim3(b.m), dim3(64), 0, s, b, (const int*)w.rec, w.counts,
+                       w.list);
+    if (n_big > 0)
+        hipLaunchKernelGGL(fd1d_window_big, dim3(n_big), dim3(128), 0, s, b, (const int*)w.counts,
+                           (const uint32_t*)w.list);
+    return hipGetLastError();
 }
 
 hipError_t launch_zero_counters(int* c, int n, hipStream_t s) {

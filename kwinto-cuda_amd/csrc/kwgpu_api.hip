@@ -15,6 +15,7 @@
 #include <tuple>
 #include <vector>
 
+#include "fd1d_plan.h"
 #include "kwgpu_internal.h"
 
 namespace {
@@ -26,33 +27,37 @@ struct DevBuf {
 
 }  // namespace
 
-// Kernel choice for one grid-size bucket: a wave-layout variant (or -1 for the lane
-// layout) and whether its grid is persistent.
+// Kernel choice for one grid-size bucket: a wave-layout variant, kLane for the lane layout
+// or kWindowed for the windowed march, and whether its grid is persistent.
+constexpr int kLane = -1, kWindowed = -2;
 struct Choice {
-    int variant = -1;
+    int variant = kLane;
     bool persist = true;
 };
 
 // One launch of an uneven batch: PDEs order[begin, begin + count) of one bucket.
 struct Bucket {
-    int cap;         // grid-size bucket: power of two >= x_dim (64 .. 2048), or kLaneCap
+    int cap;         // grid-size bucket: power of two >= x_dim (64 .. 2048), kLaneCap, or
+                     // kWindowCap for all PDEs of the windowed march together
     Choice ch;
     size_t begin, count;
     int max_x;
     int prec = KWGPU_FP64;  // the march's precision for this bucket's PDEs
+    int big = 0;            // kWindowCap: how many have over 1024 x-points
 };
 
-constexpr int kLaneCap = 1 << 30;
+constexpr int kLaneCap = 1 << 30, kWindowCap = 1 << 29;
 constexpr int kSide = 4;  // side streams an uneven batch forks onto
 
 // Device scratch of kwgpu_fd1d_price_device_noalloc: one uneven batch's PDE order, its
-// per-option x and t points, and its bucket counters, for at most kNoAllocMaxOptions
-// options (12 MiB + 256 B, held by every device the library runs on until the process
-// ends). Host code never uses the name: it takes the device address from
+// per-option x and t points, the windowed march's records and list (two entries an option),
+// and the bucket counters, for at most kNoAllocMaxOptions options (24 MiB + 512 B, held by
+// every device the library runs on until the process ends). Host code never uses the name: it takes the device address from
 // hipGetSymbolAddress, once per device, when a context is created there.
 constexpr size_t kNoAllocMaxOptions = size_t(1) << 20;
 constexpr int kNoAllocCounters = 64;
-__device__ __align__(256) uint32_t scratch[3 * kNoAllocMaxOptions + kNoAllocCounters];
+__device__ __align__(256) uint32_t
+    scratch[6 * kNoAllocMaxOptions + kNoAllocCounters + kwgpu::kWindowCounters];
 constexpr int kMaxDevices = 64;
 uint32_t* g_scratch[kMaxDevices] = {};  // device address of `scratch`, per device
 std::mutex g_scratch_mu;
@@ -75,6 +80,8 @@ struct kwgpu_ctx {
     hipStream_t stream = nullptr;
     std::string err;
     DevBuf opts, prices, status, rep, off, list, order, xd, td, ws, counters;
+    DevBuf window;     // the windowed march's counters, records (of wrecs PDEs) and list
+    size_t wrecs = 0;
     // autotuned choices per (bucket, precision), and per precision whether an uneven
     // batch's buckets run one after another on the caller's stream (true) or
     // concurrently on the side streams (false, the default)
@@ -85,6 +92,7 @@ struct kwgpu_ctx {
     hipEvent_t ev_fork = nullptr, ev_join[kSide] = {};
     bool plan_valid = false;
     uint64_t plan_key = 0;              // hash of everything but the sizes
+    unsigned plan_slots = 0;            // which grid sizes' PDEs it puts in the windowed bucket
     std::vector<int32_t> plan_x, plan_t;  // the sizes the plan was made for (compared exactly)
     std::vector<uint8_t> plan_p;          // ... and the per-PDE precisions (empty: one for all)
     int plan_prec = -1, plan_layout = -1;  // ... and the precision and layout it bucketed for
@@ -176,15 +184,50 @@ int bucket_of(int x, int precision, int layout) {
     return c;
 }
 
-Choice choice_for(const kwgpu_ctx* c, int cap, int precision, int layout) {
+// The windowed march is the default wherever it is built: FP64 at theta 1/2 and over 128
+// x-points (a smaller grid's window saves no wave: the narrowest class holds 128 rows).
+bool windowed_fits(int cap, int precision, double theta) {
+    return cap >= 256 && cap <= 2048 && precision == KWGPU_FP64 && theta == 0.5;
+}
+
+Choice choice_for(const kwgpu_ctx* c, int cap, int precision, int layout, double theta) {
     Choice ch;
     if (cap == kLaneCap) return ch;  // lane layout
+    const bool windowed = windowed_fits(cap, precision, theta);
     auto it = c->tuned.find({cap, precision});
-    if (it != c->tuned.end() && !(layout == KWGPU_LAYOUT_WAVE_REG && it->second.variant < 0))
+    if (it != c->tuned.end() && !(layout == KWGPU_LAYOUT_WAVE_REG && it->second.variant == kLane) &&
+        !(it->second.variant == kWindowed && !windowed))
         return it->second;
-    ch.variant = kwgpu::default_wave_variant(cap);
-    ch.persist = true;
+    ch.variant = windowed ? kWindowed : kwgpu::default_wave_variant(cap);
+    ch.persist = !windowed;
     return ch;
+}
+
+// Scratch of a windowed launch of m PDEs of a batch of n (the records are by PDE), `big` of
+// the m with over 1024 x-points, in one allocation: counters, records, list.
+int ensure_window(kwgpu_ctx* c, size_t n, size_t m, size_t big) {
+    c->wrecs = std::max(c->wrecs, n);
+    if (ensure(c->window, (kwgpu::kWindowCounters + c->wrecs + m + big) * sizeof(int)) != hipSuccess) {
+        c->wrecs = 0;
+        return fail(c, KWGPU_ERR_NOMEM, "kwgpu: window scratch allocation failed");
+    }
+    return KWGPU_OK;
+}
+
+kwgpu::WindowScratch window_scratch(const kwgpu_ctx* c) {
+    int* counts = (int*)c->window.p;
+    int* rec = counts + kwgpu::kWindowCounters;
+    return {rec, (uint32_t*)(rec + c->wrecs), counts};
+}
+
+// A stream under capture takes no scratch of the context: the captured launch may be
+// replayed beside the context's other solves and after its buffers have grown. (The
+// stand-in runtime of the host tests has no such call.)
+extern "C" hipError_t hipStreamIsCapturing(hipStream_t, hipStreamCaptureStatus*) __attribute__((weak));
+bool capturing(hipStream_t s) {
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    if (!hipStreamIsCapturing || hipStreamIsCapturing(s, &st) != hipSuccess) return false;
+    return st != hipStreamCaptureStatusNone;
 }
 
 uint64_t fnv(uint64_t h, const void* p, size_t n) {
@@ -210,8 +253,33 @@ uint64_t fnv_batch(uint64_t h, const FdBatch& b) {
 
 uint64_t fnv_bucket(uint64_t h, const Bucket& k) {
     const int persist = k.ch.persist ? 1 : 0;
-    return fnv_fields(h, k.cap, k.ch.variant, persist, k.begin, k.count, k.max_x, k.prec);
+    return fnv_fields(h, k.cap, k.ch.variant, persist, k.begin, k.count, k.max_x, k.prec, k.big);
 }
+
+// The buckets of an uneven batch by slot number: 0 the windowed march's PDEs, of every grid
+// size whose choice it is; then capacities 64 .. 2048 and the lane layout in FP64, then in
+// FP32-mixed.
+struct Slots {
+    static constexpr int kCaps = 7, kCount = 1 + 2 * kCaps;
+    int layout;
+    unsigned mask = 0;  // bit k: FP64 PDEs of capacity 64 << k are windowed
+    Slots(const kwgpu_ctx* c, int layout_, double theta) : layout(layout_) {
+        for (int k = 0; k + 1 < kCaps; ++k)
+            if (choice_for(c, 64 << k, KWGPU_FP64, layout, theta).variant == kWindowed) mask |= 1u << k;
+    }
+    int of(int x, int prec) const {
+        const int c = bucket_of(x, prec, layout);
+        const int k = c == kLaneCap ? kCaps - 1 : 31 - __builtin_clz((unsigned)c) - 6;
+        if (prec == KWGPU_FP64 && (mask >> k & 1)) return 0;
+        return 1 + (prec == KWGPU_FP32_MIXED ? kCaps : 0) + k;
+    }
+    int cap(int slot) const {
+        if (slot == 0) return kWindowCap;
+        const int k = (slot - 1) % kCaps;
+        return k == kCaps - 1 ? kLaneCap : 64 << k;
+    }
+    int prec(int slot) const { return slot <= kCaps ? KWGPU_FP64 : KWGPU_FP32_MIXED; }
+};
 
 int lane_launch(kwgpu_ctx* c, FdBatch bb, int max_x, int precision, hipStream_t s, double* ws) {
     if (precision != KWGPU_FP64)
@@ -244,7 +312,10 @@ int launch_buckets(kwgpu_ctx* c, const FdBatch& b, const std::vector<Bucket>& pl
         FdBatch bb = b;
         bb.order = (const uint32_t*)c->order.p + k.begin;
         bb.m = (int)k.count;
-        if (k.ch.variant < 0) {
+        if (k.ch.variant == kWindowed) {
+            if ((e = kwgpu::launch_fd1d_windowed(bb, window_scratch(c), k.big, ss)))
+                return hip_fail(c, e, "kwgpu: windowed kernel launch");
+        } else if (k.ch.variant < 0) {
             double* ws = (double*)c->ws.p + ws_off;
             ws_off += kwgpu::lane_workspace_doubles(bb.m, k.max_x);
             if (int rc = lane_launch(c, bb, k.max_x, k.prec, ss, ws)) return rc;
@@ -296,8 +367,11 @@ void drop_graph(kwgpu_ctx* c) {
 // a persistent grid takes the longest first; each bucket's kernel (autotuned variant)
 // runs on its own side stream. The whole launch sequence is captured once into a
 // hipGraph and replayed while the batch (sizes, buffers, parameters) is unchanged.
+//
+// whole: every PDE's march carries its whole grid (no windowed march).
 int run_fd_on(kwgpu_ctx* c, FdBatch b, const int32_t* pde_x, const int32_t* pde_t, int precision,
-              int layout, hipStream_t s, const uint8_t* pde_prec) {
+              int layout, hipStream_t s, const uint8_t* pde_prec, bool whole) {
+    const double theta = whole ? 0.0 : b.theta;  // as the choice of a march sees it
     // per-PDE precisions go through the planned path, with the uniform sizes spelled out
     std::vector<int32_t> ux, ut;
     if (pde_prec && !pde_x) {
@@ -338,7 +412,23 @@ int run_fd_on(kwgpu_ctx* c, FdBatch b, const int32_t* pde_x, const int32_t* pde_
 
     if (uniform) {
         const int cap = bucket_of(b.x_dim, precision, layout);
-        Choice ch = choice_for(c, cap, precision, layout);
+        Choice ch = choice_for(c, cap, precision, layout, theta);
+        if (ch.variant == kWindowed) {
+            const bool lone = b.m <= kwgpu::kLoneMax && b.x_dim <= 1024;
+            if (b.t_dim - 1 >= kwgpu::kWindowMinSteps && lone) {
+                if (hipError_t e = kwgpu::launch_fd1d_lone(b, s); e != hipSuccess)
+                    return hip_fail(c, e, "kwgpu: windowed kernel launch");
+                return KWGPU_OK;
+            }
+            if (b.t_dim - 1 >= kwgpu::kWindowMinSteps && !capturing(s)) {
+                const int big = b.x_dim > 1024 ? b.m : 0;
+                if (int rc = ensure_window(c, b.m, b.m, big)) return rc;
+                if (hipError_t e = kwgpu::launch_fd1d_windowed(b, window_scratch(c), big, s))
+                    return hip_fail(c, e, "kwgpu: windowed kernel launch");
+                return KWGPU_OK;
+            }
+            ch.variant = kwgpu::default_wave_variant(cap);
+        }
         if (ch.variant < 0) {
             const size_t need = kwgpu::lane_workspace_doubles(b.m, b.x_dim) * sizeof(double);
             if (c->ws.cap < need) drop_graph(c);  // a captured graph may hold the old buffer
@@ -353,33 +443,32 @@ int run_fd_on(kwgpu_ctx* c, FdBatch b, const int32_t* pde_x, const int32_t* pde_
     }
 
     const int m = b.m;
-    // buckets in ascending capacity (64 .. 2048, then the lane layout), FP64 ones first,
-    // then FP32-mixed ones: counts and widest grid, without sorting the PDEs
-    constexpr int kSlots = 7;
-    auto slot_of = [&](int p) {
-        const int cap = bucket_of(pde_x[p], precision, layout);
-        const int k = cap == kLaneCap ? kSlots - 1 : 31 - __builtin_clz((unsigned)cap) - 6;
-        return prec_of(p) == KWGPU_FP32_MIXED ? kSlots + k : k;
-    };
+    // buckets: the FP64 PDEs of every grid size that takes the windowed march as one, then
+    // ascending capacity (64 .. 2048, then the lane layout), FP64 ones first, then
+    // FP32-mixed ones: counts and widest grid, without sorting the PDEs
+    const Slots slots(c, layout, theta);
+    auto slot_of = [&](int p) { return slots.of(pde_x[p], prec_of(p)); };
     std::vector<Bucket> plan;
-    if (same_sizes) {
+    // (a plan made under other kernel choices has other buckets: its key differs)
+    if (same_sizes && c->plan_slots == slots.mask) {
         plan = c->plan;
-        for (Bucket& k : plan) k.ch = choice_for(c, k.cap, k.prec, layout);
+        for (Bucket& k : plan)
+            if (k.cap != kWindowCap) k.ch = choice_for(c, k.cap, k.prec, layout, theta);
     } else {
-        size_t count[2 * kSlots] = {};
-        int widest[2 * kSlots] = {};
+        size_t count[Slots::kCount] = {};
+        int widest[Slots::kCount] = {}, big = 0;
         for (int p = 0; p < m; ++p) {
             const int k = slot_of(p);
             ++count[k];
             widest[k] = std::max(widest[k], pde_x[p]);
+            big += k == 0 && pde_x[p] > 1024;
         }
         size_t begin = 0;
-        for (int k = 0; k < 2 * kSlots; ++k) {
+        for (int k = 0; k < Slots::kCount; ++k) {
             if (!count[k]) continue;
-            const int kc = k % kSlots;
-            const int cap = kc == kSlots - 1 ? kLaneCap : 64 << kc;
-            const int pr = k < kSlots ? KWGPU_FP64 : KWGPU_FP32_MIXED;
-            plan.push_back(Bucket{cap, choice_for(c, cap, pr, layout), begin, count[k], widest[k], pr});
+            const int cap = slots.cap(k), pr = slots.prec(k);
+            const Choice ch = k == 0 ? Choice{kWindowed, false} : choice_for(c, cap, pr, layout, theta);
+            plan.push_back(Bucket{cap, ch, begin, count[k], widest[k], pr, k == 0 ? big : 0});
             begin += count[k];
         }
     }
@@ -390,12 +479,14 @@ int run_fd_on(kwgpu_ctx* c, FdBatch b, const int32_t* pde_x, const int32_t* pde_
     key = fnv_fields(key, precision);
     for (const Bucket& k : plan) key = fnv_bucket(key, k);
     const auto sit = c->serial.find(precision);
-    const int serial = sit != c->serial.end() && sit->second ? 1 : 0;
+    // (one bucket has nothing to run beside)
+    const int serial = plan.size() == 1 || (sit != c->serial.end() && sit->second) ? 1 : 0;
     key = fnv_fields(key, serial);
 
     // ... and the context buffers a captured graph would reference
     auto with_buffers = [&](uint64_t k) {
-        const void* bufs[3] = {c->order.p, c->counters.p, c->ws.p};
+        const kwgpu::WindowScratch w = window_scratch(c);
+        const void* bufs[5] = {c->order.p, c->counters.p, c->ws.p, w.counts, w.list};
         return fnv(k, bufs, sizeof(bufs));
     };
     if (int rc = ensure_side_streams(c)) return rc;
@@ -403,8 +494,11 @@ int run_fd_on(kwgpu_ctx* c, FdBatch b, const int32_t* pde_x, const int32_t* pde_
     if (rebuild) {
         drop_graph(c);
         size_t ws = 0;
-        for (const Bucket& k : plan)
-            if (k.ch.variant < 0) ws += kwgpu::lane_workspace_doubles((int)k.count, k.max_x);
+        for (const Bucket& k : plan) {
+            if (k.ch.variant == kLane) ws += kwgpu::lane_workspace_doubles((int)k.count, k.max_x);
+            if (k.ch.variant == kWindowed)
+                if (int rc = ensure_window(c, m, k.count, k.big)) return rc;
+        }
         if (ensure(c->order, sizeof(uint32_t) * m) != hipSuccess ||
             ensure(c->counters, sizeof(int) * plan.size()) != hipSuccess ||
             (ws && ensure(c->ws, ws * sizeof(double)) != hipSuccess))
@@ -423,6 +517,7 @@ int run_fd_on(kwgpu_ctx* c, FdBatch b, const int32_t* pde_x, const int32_t* pde_
             (e = hipStreamSynchronize(s)))
             return hip_fail(c, e, "kwgpu: order upload");
         c->plan = plan;
+        c->plan_slots = slots.mask;
         c->plan_key = key;
         c->plan_x.assign(pde_x, pde_x + m);
         c->plan_t.assign(pde_t, pde_t + m);
@@ -469,11 +564,11 @@ int run_fd_on(kwgpu_ctx* c, FdBatch b, const int32_t* pde_x, const int32_t* pde_
 // context's PDE order, counters and lane workspace that this one rewrites; its own end
 // is recorded for the next.
 int run_fd(kwgpu_ctx* c, FdBatch b, const int32_t* pde_x, const int32_t* pde_t, int precision,
-           int layout, hipStream_t s, const uint8_t* pde_prec = nullptr) {
+           int layout, hipStream_t s, const uint8_t* pde_prec = nullptr, bool whole = false) {
     if (c->done_stream && c->done_stream != s)
         if (hipError_t e = hipStreamWaitEvent(s, c->ev_done, 0); e != hipSuccess)
             return hip_fail(c, e, "kwgpu: order after the previous solve");
-    const int rc = run_fd_on(c, b, pde_x, pde_t, precision, layout, s, pde_prec);
+    const int rc = run_fd_on(c, b, pde_x, pde_t, precision, layout, s, pde_prec, whole);
     if (hipError_t e = hipEventRecord(c->ev_done, s); e != hipSuccess)
         return rc ? rc : hip_fail(c, e, "kwgpu: solve event");
     c->done_stream = s;
@@ -551,7 +646,7 @@ void group_pdes(const kwgpu_option* opts, size_t n, const int32_t* xd, const int
 // Host-pointer FD price with the reference's PDE compression; results are left in
 // the device buffers `d_prices` / `d_status` (sized n). Returns KWGPU_OK or an error.
 int fd_price_host(kwgpu_ctx* c, const kwgpu_option* opts, size_t n, const kwgpu_fd1d_params* p,
-                  DevBuf& d_opts, DevBuf& d_prices, DevBuf& d_status) {
+                  DevBuf& d_opts, DevBuf& d_prices, DevBuf& d_status, bool whole = false) {
     hipStream_t s = c->stream;
     // PDE compression, src/Pricer/kwFd1d.cpp:28-65: options equal in (t, r, q, z, e, w)
     // -- and, for uneven batches, in grid size -- share one solve.
@@ -632,7 +727,7 @@ int fd_price_host(kwgpu_ctx* c, const kwgpu_option* opts, size_t n, const kwgpu_
     }
     const int rc = run_fd(c, b, pde_x.empty() ? nullptr : pde_x.data(),
                           pde_t.empty() ? nullptr : pde_t.data(), p->precision, p->layout, s,
-                          pprec.empty() ? nullptr : pprec.data());
+                          pprec.empty() ? nullptr : pprec.data(), whole);
     // the host vectors above must outlive every copy queued from them
     e = hipStreamSynchronize(s);
     if (rc) return rc;
@@ -687,7 +782,7 @@ int ctx_device(kwgpu_ctx* c) { return c ? c->device : 0; }
 // KWGPU_FP64 or KWGPU_FP32_MIXED; null: params->precision for all): one plan, one graph.
 int fd_price_device_prec(kwgpu_ctx* c, const kwgpu_option* d_opts, size_t n,
                          const kwgpu_fd1d_params* p, double* d_prices, int32_t* d_status,
-                         void* stream, const uint8_t* host_prec) {
+                         void* stream, const uint8_t* host_prec, bool whole) {
     if (!c) return KWGPU_ERR_INVALID;
     c->err.clear();
     if (int rc = check_params(c, p)) return rc;
@@ -709,7 +804,7 @@ int fd_price_device_prec(kwgpu_ctx* c, const kwgpu_option* d_opts, size_t n,
     b.prices = d_prices;
     b.status = d_status;
     if (!p->x_dims && !p->t_dims)
-        return run_fd(c, b, nullptr, nullptr, p->precision, p->layout, s, host_prec);
+        return run_fd(c, b, nullptr, nullptr, p->precision, p->layout, s, host_prec, whole);
     // grouping needs the sizes on the host: pinned staging owned by the context
     if (c->hsizes_cap < 2 * n) {
         if (c->hsizes) (void)hipHostFree(c->hsizes);
@@ -733,7 +828,7 @@ int fd_price_device_prec(kwgpu_ctx* c, const kwgpu_option* d_opts, size_t n,
         return hip_fail(c, e, "kwgpu: t_dims download");
     if ((e = hipStreamSynchronize(s)) != hipSuccess) return hip_fail(c, e, "kwgpu: sync");
     if (int rc = check_dims(c, hx, ht, n)) return rc;
-    return run_fd(c, b, hx, ht, p->precision, p->layout, s, host_prec);
+    return run_fd(c, b, hx, ht, p->precision, p->layout, s, host_prec, whole);
 }
 }  // namespace kwgpu
 
@@ -794,7 +889,7 @@ void kwgpu_destroy(kwgpu_ctx* c) {
     (void)hipEventDestroy(c->ev_done);
     if (c->hsizes) (void)hipHostFree(c->hsizes);
     for (DevBuf* b : {&c->opts, &c->prices, &c->status, &c->rep, &c->off, &c->list, &c->order,
-                      &c->xd, &c->td, &c->ws, &c->counters})
+                      &c->xd, &c->td, &c->ws, &c->counters, &c->window})
         free_buf(*b);
     (void)hipStreamDestroy(c->stream);
     delete c;
@@ -960,7 +1055,12 @@ int kwgpu_fd1d_greeks(kwgpu_ctx* c, const kwgpu_option* opts, size_t n,
     if (p->x_dims) p9.x_dims = xd.data();
     if (p->t_dims) p9.t_dims = td.data();
     const size_t n9 = n * kSets;
-    if (int rc = fd_price_host(c, all.data(), n9, &p9, c->opts, c->prices, c->status)) return rc;
+    // Whole grids: rho divides a difference of two prices by 2 b r, which for rates near 0
+    // turns any other rounding of the march into leading digits (300 options with rates down
+    // to 3e-4: 7e-10 of rho between the two marches), and windows save nothing here that a
+    // book of this size is bound by
+    if (int rc = fd_price_host(c, all.data(), n9, &p9, c->opts, c->prices, c->status, true))
+        return rc;
     std::vector<double> v(n9);
     std::vector<int32_t> st(n9);
     hipError_t e;
@@ -1025,7 +1125,9 @@ int kwgpu_fd1d_price_device_noalloc(kwgpu_ctx* c, const kwgpu_option* d_opts, si
     uint32_t* d_order = base;
     int32_t* d_x = reinterpret_cast<int32_t*>(base + kNoAllocMaxOptions);
     int32_t* d_t = reinterpret_cast<int32_t*>(base + 2 * kNoAllocMaxOptions);
-    int* d_counters = reinterpret_cast<int*>(base + 3 * kNoAllocMaxOptions);
+    int* d_counters = reinterpret_cast<int*>(base + 6 * kNoAllocMaxOptions);
+    const kwgpu::WindowScratch ws{reinterpret_cast<int*>(base + 3 * kNoAllocMaxOptions),
+                                  base + 4 * kNoAllocMaxOptions, d_counters + kNoAllocCounters};
     FdBatch b{};
     b.opts = d_opts;
     b.m = (int)n;
@@ -1036,31 +1138,38 @@ int kwgpu_fd1d_price_device_noalloc(kwgpu_ctx* c, const kwgpu_option* d_opts, si
     b.theta = p->theta;
     b.prices = d_prices;
     b.status = d_status;
-    // buckets: (x-points rounded up to a power of two) in ascending order, PDEs by
-    // t-points descending within each (ties by index), as for uneven batches elsewhere
+    // the buckets of uneven batches elsewhere, PDEs by t-points descending within each (ties
+    // by index)
     std::vector<Bucket> plan;
     hipError_t e = hipSuccess;
     if (!hx && !ht) {
         const int cap = bucket_of(p->x_dim, p->precision, p->layout);
-        plan.push_back(Bucket{cap, choice_for(c, cap, p->precision, p->layout), 0, n, p->x_dim,
-                              p->precision});
+        Choice ch = choice_for(c, cap, p->precision, p->layout, p->theta);
+        if (ch.variant == kWindowed && p->t_dim - 1 < kwgpu::kWindowMinSteps)
+            ch = Choice{kwgpu::default_wave_variant(cap), true};
+        plan.push_back(Bucket{cap, ch, 0, n, p->x_dim, p->precision, p->x_dim > 1024 ? (int)n : 0});
     } else {
+        const Slots slots(c, p->layout, p->theta);
         auto gx = [&](size_t i) { return hx ? hx[i] : p->x_dim; };
         auto gt = [&](size_t i) { return ht ? ht[i] : p->t_dim; };
         std::vector<uint32_t> ord(n);
         std::iota(ord.begin(), ord.end(), 0u);
-        std::vector<int> cap(n);
-        for (size_t i = 0; i < n; ++i) cap[i] = bucket_of(gx(i), p->precision, p->layout);
+        std::vector<int> slot(n);
+        for (size_t i = 0; i < n; ++i) slot[i] = slots.of(gx(i), p->precision);
         std::sort(ord.begin(), ord.end(), [&](uint32_t a, uint32_t z) {
-            return std::make_tuple(cap[a], -gt(a), a) < std::make_tuple(cap[z], -gt(z), z);
+            return std::make_tuple(slot[a], -gt(a), a) < std::make_tuple(slot[z], -gt(z), z);
         });
         for (size_t k = 0; k < n;) {
             size_t k1 = k;
-            int widest = 0;
-            while (k1 < n && cap[ord[k1]] == cap[ord[k]]) widest = std::max(widest, gx(ord[k1++]));
-            const int cp = cap[ord[k]];
-            plan.push_back(Bucket{cp, choice_for(c, cp, p->precision, p->layout), k, k1 - k,
-                                  widest, p->precision});
+            int widest = 0, big = 0;
+            for (; k1 < n && slot[ord[k1]] == slot[ord[k]]; ++k1) {
+                widest = std::max(widest, gx(ord[k1]));
+                big += gx(ord[k1]) > 1024;
+            }
+            const int sl = slot[ord[k]], cp = slots.cap(sl);
+            const Choice ch = sl == 0 ? Choice{kWindowed, false}
+                                      : choice_for(c, cp, p->precision, p->layout, p->theta);
+            plan.push_back(Bucket{cp, ch, k, k1 - k, widest, p->precision, sl == 0 ? big : 0});
             k = k1;
         }
         std::vector<int32_t> fx, ft;
@@ -1085,9 +1194,11 @@ int kwgpu_fd1d_price_device_noalloc(kwgpu_ctx* c, const kwgpu_option* d_opts, si
         FdBatch bb = b;
         if (bb.order) bb.order += k.begin;
         bb.m = (int)k.count;
-        if ((e = kwgpu::launch_fd1d_wave_variant(bb, k.ch.variant, k.prec, s,
-                                                 k.ch.persist ? d_counters + i : nullptr)))
-            return hip_fail(c, e, "kwgpu_fd1d_price_device_noalloc: launch");
+        e = k.ch.variant == kWindowed
+                ? kwgpu::launch_fd1d_windowed(bb, ws, k.big, s)
+                : kwgpu::launch_fd1d_wave_variant(bb, k.ch.variant, k.prec, s,
+                                                  k.ch.persist ? d_counters + i : nullptr);
+        if (e) return hip_fail(c, e, "kwgpu_fd1d_price_device_noalloc: launch");
     }
     if ((e = hipEventRecord(c->ev_done, s))) return hip_fail(c, e, "kwgpu: solve event");
     c->done_stream = s;
@@ -1164,10 +1275,14 @@ int kwgpu_fd1d_autotune(kwgpu_ctx* c, const kwgpu_option* d_opts, size_t n,
             bool pruned = false;  // ms is a lower bound; the candidate was not run
         };
         std::vector<Cand> cands;
+        if (windowed_fits(cap, prec, p->theta)) {
+            if ((rc = ensure_window(c, n, S, bx > 1024 ? S : 0))) break;
+            cands.push_back({Choice{kWindowed, false}, 0.f});
+        }
         for (int v = 0; v < kwgpu::wave_variant_count(); ++v)
             if (kwgpu::wave_variant(v).capacity() == cap)
                 for (bool per : {false, true}) cands.push_back({Choice{v, per}, 0.f});
-        if (prec == KWGPU_FP64) cands.push_back({Choice{-1, false}, 0.f});
+        if (prec == KWGPU_FP64) cands.push_back({Choice{kLane, false}, 0.f});
         // the lane layout streams its state through HBM and runs ~100x slower than the
         // wave variants: it is timed on the first kLaneSample sampled options and scaled
         constexpr size_t kLaneSample = 256;
@@ -1184,10 +1299,10 @@ int kwgpu_fd1d_autotune(kwgpu_ctx* c, const kwgpu_option* d_opts, size_t n,
             pts_max = std::max(pts_max, pts);
         }
         for (auto& cd : cands) {
-            if (cd.ch.variant < 0 && pts_min > 0.0) {
+            if (cd.ch.variant == kLane && pts_min > 0.0) {
                 float best_wave = 0.f;
                 for (const auto& w : cands)
-                    if (w.ch.variant >= 0 && (best_wave == 0.f || w.ms < best_wave)) best_wave = w.ms;
+                    if (w.ch.variant != kLane && (best_wave == 0.f || w.ms < best_wave)) best_wave = w.ms;
                 FdBatch bp = bb;
                 bp.m = 1;
                 bp.order = (const uint32_t*)sample.p + kmin;
@@ -1212,7 +1327,13 @@ int kwgpu_fd1d_autotune(kwgpu_ctx* c, const kwgpu_option* d_opts, size_t n,
                 }
             }
             auto run = [&]() -> int {
-                if (cd.ch.variant < 0) {
+                if (cd.ch.variant == kWindowed) {
+                    if (hipError_t e2 = kwgpu::launch_fd1d_windowed(bb, window_scratch(c),
+                                                                    bx > 1024 ? (int)S : 0, s))
+                        return hip_fail(c, e2, "kwgpu_fd1d_autotune: launch");
+                    return KWGPU_OK;
+                }
+                if (cd.ch.variant == kLane) {
                     if (ensure(ws, kwgpu::lane_workspace_doubles(bl.m, bx) * sizeof(double)))
                         return fail(c, KWGPU_ERR_NOMEM, "kwgpu_fd1d_autotune: workspace");
                     return lane_launch(c, bl, bx, prec, s, (double*)ws.p);
@@ -1228,7 +1349,7 @@ int kwgpu_fd1d_autotune(kwgpu_ctx* c, const kwgpu_option* d_opts, size_t n,
             };
             if ((rc = run())) break;  // warm-up
             // the median of three timed runs (one for the lane layout, which is slow)
-            const int reps = cd.ch.variant < 0 ? 1 : 3;
+            const int reps = cd.ch.variant == kLane ? 1 : 3;
             float t[3] = {0.f, 0.f, 0.f};
             for (int r = 0; r < reps && !rc; ++r) {
                 if ((e = hipEventRecord(e0, s))) { rc = hip_fail(c, e, "event"); break; }
@@ -1240,12 +1361,12 @@ int kwgpu_fd1d_autotune(kwgpu_ctx* c, const kwgpu_option* d_opts, size_t n,
             if (rc) break;
             if (reps == 3) std::sort(t, t + 3);
             cd.ms = reps == 3 ? t[1] : t[0];
-            if (cd.ch.variant < 0) cd.ms *= (float)S / (float)bl.m;
+            if (cd.ch.variant == kLane) cd.ms *= (float)S / (float)bl.m;
         }
         if (rc) break;
         // a later candidate must be faster by 2 % to displace an earlier one: within
-        // that margin sample timings are noise, and the order puts the 16-row,
-        // static-grid variant first
+        // that margin sample timings are noise, and the order puts the windowed march,
+        // then the 16-row, static-grid variant first
         const Cand* best = &cands[0];
         for (const auto& cd : cands)
             if (cd.ms < 0.98f * best->ms) best = &cd;
@@ -1258,7 +1379,12 @@ int kwgpu_fd1d_autotune(kwgpu_ctx* c, const kwgpu_option* d_opts, size_t n,
         js += buf;
         for (size_t k = 0; k < cands.size(); ++k) {
             const auto& cd = cands[k];
-            if (cd.ch.variant < 0) {
+            if (cd.ch.variant == kWindowed) {
+                std::snprintf(buf, sizeof(buf),
+                              "%s{\"layout\": \"wave\", \"rows_per_lane\": 0, \"lanes\": 0, \"waves\": 0, "
+                              "\"persistent\": false, \"windowed\": true, \"ms\": %.4f}",
+                              k ? ", " : "", cd.ms);
+            } else if (cd.ch.variant == kLane) {
                 std::snprintf(buf, sizeof(buf), "%s{\"layout\": \"lane\", \"ms\": %.4f, \"pruned\": %s}",
                               k ? ", " : "", cd.ms, cd.pruned ? "true" : "false");
             } else {
@@ -1343,6 +1469,7 @@ int kwgpu_tune_load(kwgpu_ctx* c, const char* path) {
             c->serial[prec] = v != 0;
             continue;
         }
+        if (v == kWindowed && !windowed_fits(cap, prec, 0.5)) continue;
         if (v >= kwgpu::wave_variant_count() || (v >= 0 && kwgpu::wave_variant(v).capacity() != cap)) continue;
         if (v < 0 && prec != KWGPU_FP64) continue;
         c->tuned[{cap, prec}] = Choice{v, per != 0};

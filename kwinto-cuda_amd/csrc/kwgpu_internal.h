@@ -175,10 +175,11 @@ namespace kwgpu {
 // Context internals shared by the C-ABI translation units (kwgpu_api.hip).
 int ctx_fail(kwgpu_ctx* c, int code, const std::string& msg);
 hipStream_t ctx_stream(kwgpu_ctx* c);
-// kwgpu_fd1d_price_device with an optional per-option precision (host array of n).
+// kwgpu_fd1d_price_device with an optional per-option precision (host array of n); whole:
+// every march carries its whole grid (no windowed march).
 int fd_price_device_prec(kwgpu_ctx* c, const kwgpu_option* d_opts, size_t n,
                          const kwgpu_fd1d_params* p, double* d_prices, int32_t* d_status,
-                         void* stream, const uint8_t* host_prec);
+                         void* stream, const uint8_t* host_prec, bool whole = false);
 int ctx_device(kwgpu_ctx* c);
 
 // Wave layout, FP64 / FP32-mixed. Returns hipErrorInvalidValue when x_dim does not fit.
@@ -199,6 +200,21 @@ int default_wave_variant(int max_x_dim);  // -1 when the grid does not fit
 hipError_t launch_fd1d_wave_variant(const FdBatch& b, int variant, int precision, hipStream_t s,
                                     int* queue = nullptr);
 bool wave_layout_fits(int x_dim, int precision);
+// FP64 at theta 1/2 on each PDE's window of rows (fd1d_window.h), x_dim <= 2048. Device
+// scratch of the caller: a record per PDE number (all that b.order may name), a list of
+// b.m + n_big entries and kWindowCounters counters. n_big: how many of the b.m PDEs have over
+// 1024 x-points.
+constexpr int kWindowCounters = 32;
+struct WindowScratch {
+    int* rec;
+    uint32_t* list;
+    int* counts;
+};
+hipError_t launch_fd1d_windowed(const FdBatch& b, const WindowScratch& w, int n_big,
+                                hipStream_t s);
+// The same for at most kLoneMax PDEs, x_dim <= 1024, without scratch: one PDE a wave.
+constexpr int kLoneMax = 2048;
+hipError_t launch_fd1d_lone(const FdBatch& b, hipStream_t s);
 // Lane layout (any grid size).
 hipError_t launch_fd1d_lane(const FdBatch& b, hipStream_t s);
 size_t lane_workspace_doubles(int m, int max_x_dim);

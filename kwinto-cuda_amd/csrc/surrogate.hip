@@ -2008,7 +2008,10 @@ int kwgpu_surrogate_labels(kwgpu_ctx* ctx, const kwgpu_option* d_opts, size_t n,
     kwgpu_fd1d_params p = *fd;
     p.x_dims = nx;
     p.t_dims = nt;
-    int rc = kwgpu::fd_price_device_prec(ctx, d_nodes, n2, &p, fdp, fst, st, nullptr);
+    // Whole grids: a fit amplifies the last digits of its labels (the windowed march's other
+    // rounding, 1e-12 of a price, became 4e-5 of the weights in eight Adam steps), and a fit
+    // is to stay the same for a seed. The labels are about 2 % of a fit's time.
+    int rc = kwgpu::fd_price_device_prec(ctx, d_nodes, n2, &p, fdp, fst, st, nullptr, true);
     if (rc == KWGPU_OK) {
         hipLaunchKernelGGL(node_premium_kernel, dim3(nblk(n, 256)), dim3(256), 0, st, d_nodes, n,
                            fdp, fst, ok, d_premium, d_keep);
