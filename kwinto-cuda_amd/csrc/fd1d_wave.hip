@@ -60,7 +60,7 @@ namespace {
 #define KWGPU_PF2 0  // two-wave groups: read at the point of use (any buffer costs spills)
 #endif
 #ifndef KWGPU_PFG
-#define KWGPU_PFG 0  // several options per wave
+#define KWGPU_PFG 4  // several options per wave
 #endif
 
 constexpr int kRowShr = 0x110;   // + n, n in 1..15
@@ -548,6 +548,26 @@ __device__ __forceinline__ int group_steps(const Pde& d, const Lanes& t, double*
     }
 }
 
+template <int LANE, int ROWS, int BANKS, bool LAST = false>
+__device__ __forceinline__ double fmac_newbcast(double acc, double src, double mul) {
+    // acc += src[LANE of the row] * mul in the lanes of the given rows and quads. A DPP read
+    // wants two wait states after the VALU write of its register: waited for here before the
+    // read and, where a DPP move follows (LAST), after the write, as the compiler does not
+    // look into the assembly.
+    if constexpr (LAST)
+        asm("s_nop 1\n\t"
+            "v_fmac_f64_dpp %0, %1, %2 row_newbcast:%3 row_mask:%4 bank_mask:%5\n\t"
+            "s_nop 1"
+            : "+v"(acc)
+            : "v"(src), "v"(mul), "n"(LANE), "n"(ROWS), "n"(BANKS));
+    else
+        asm("s_nop 1\n\t"
+            "v_fmac_f64_dpp %0, %1, %2 row_newbcast:%3 row_mask:%4 bank_mask:%5"
+            : "+v"(acc)
+            : "v"(src), "v"(mul), "n"(LANE), "n"(ROWS), "n"(BANKS));
+    return acc;
+}
+
 // Wave-local inclusive forward scan of the lanes' local last values.
 template <int L, class T>
 __device__ __forceinline__ T fwd_scan(T c, const ScanMul<T>& sm) {
@@ -583,8 +603,14 @@ __device__ __forceinline__ T bwd_scan(T cb, const ScanMul<T>& sm, const Lanes& t
         cb = fma(sm.X16, readlane<16>(cb), cb);
     } else if constexpr (L == 32) {
         // two options per wave: each takes the first lane of its own second row
-        const T src = t.wrow < 2 ? readlane<16>(cb) : readlane<48>(cb);
-        cb = fma(sm.X16, src, cb);
+        if constexpr (sizeof(T) == 8) {
+            // one lane down, then across rows 0 and 2: the same FMA without the branch that
+            // a choice between two readlanes compiles to
+            cb = fmac_newbcast<15, 0x5, 0xF, true>(cb, dpp<kWaveShl1>(cb), sm.X16);
+        } else {
+            const T src = t.wrow < 2 ? readlane<16>(cb) : readlane<48>(cb);
+            cb = fma(sm.X16, src, cb);
+        }
     }
     return cb;
 }
@@ -597,25 +623,6 @@ __device__ __forceinline__ T bwd_scan(T cb, const ScanMul<T>& sm, const Lanes& t
 // one v_fmac_f64 for each source, the taking lanes selected by the instruction's bank and
 // row masks. 34 instructions for the two scans of 64 lanes instead of 43, 32 instead of 38
 // and two branches for 32, 26 instead of 32 for 16.
-template <int LANE, int ROWS, int BANKS, bool LAST = false>
-__device__ __forceinline__ double fmac_newbcast(double acc, double src, double mul) {
-    // acc += src[LANE of the row] * mul in the lanes of the given rows and quads. A DPP read
-    // wants two wait states after the VALU write of its register: waited for here before the
-    // read and, where a DPP move follows (LAST), after the write, as the compiler does not
-    // look into the assembly.
-    if constexpr (LAST)
-        asm("s_nop 1\n\t"
-            "v_fmac_f64_dpp %0, %1, %2 row_newbcast:%3 row_mask:%4 bank_mask:%5\n\t"
-            "s_nop 1"
-            : "+v"(acc)
-            : "v"(src), "v"(mul), "n"(LANE), "n"(ROWS), "n"(BANKS));
-    else
-        asm("s_nop 1\n\t"
-            "v_fmac_f64_dpp %0, %1, %2 row_newbcast:%3 row_mask:%4 bank_mask:%5"
-            : "+v"(acc)
-            : "v"(src), "v"(mul), "n"(LANE), "n"(ROWS), "n"(BANKS));
-    return acc;
-}
 template <int L>
 __device__ __forceinline__ double win_fwd_scan(double c, const ScanMul<double>& sm) {
     c = fma(sm.F1, dpp<kRowShr + 1>(c), c);
@@ -777,9 +784,11 @@ __device__ __forceinline__ void march_f64(double (&xv)[M], const double (&ap)[M]
     // LDS reads of the (Q, payoff) pairs in flight ahead of the row updates. Measured on
     // one box: the 1024-point one-wave kernel 9.81 ms at 3, 10.03 at 4, 10.06 at 1 (and
     // 10.3 at 0); the 2048-point two-wave kernel 13.2 ms at 0, 15.6 at 1, 22.3 at 3,
-    // where the extra registers turn into spill reloads inside the step loop; the
-    // 256- and 512-point kernels (4 and 2 options per wave) 2.69 and 5.34 ms at 0, 2.88
-    // and 6.33 at 3.
+    // where the extra registers turn into spill reloads inside the step loop. Several
+    // options per wave: with one wave on a SIMD, as in a small batch, each read at its point
+    // of use shows its whole latency, 16 times a step. Greeks of 20 options at 512 x 512
+    // (whole host call) 291 us at 0, 271 at 2, 238 at 4, 236 at 6; 300 at 256 x 512 325, 307,
+    // 275 and 387 us (spills); 32768 options at 512 x 60 494, 486, 474, 471 us.
     // Windowed marches hold fewer scan multipliers and no branch, and have the registers for
     // it at every width. 16384 options, 512 steps, on 256- and 512-point grids (16-lane
     // options mostly) and on 1024 points (32- and 64-lane ones): 741, 1088 and 1840 us with
