@@ -75,10 +75,13 @@ KWGPU_HD float critical_log_spot(float t, float z, float r, float q) {
 // error of e^-36 = 2e-16. Where the steps are few Crank-Nicolson's tails are heavier than
 // the Gaussian's: at 64 steps the exponent 36 loses 2 n (y^3/3 + ...), y = 36 / (2 n), 0.9.
 //
-// In the money the cut lies 0.04 in log S and 3 rows past the approximate critical spot:
-// about 10 rows of 1024 for a boundary that went past it in none of some 13000 random
-// windows (vol 1-200 %, T 0.005-30 years, rates -3-25 %) at 0.05 and 4, in 1 at 0.03 and 3
-// and in 19 at 0.02 and 2. It needs
+// In the money the cut lies min(0.075, 0.24 sigma sqrt(T)) in log S and 2 rows past the
+// approximate critical spot. Measured on 7400 marches (vol 1-200 %, T 0.005-30 years, rates
+// -3-25 %, 1024 and 2048 points) the boundary ended at most 0.070 past it, and 0.23 sigma
+// sqrt(T): where the rate is near 0 the approximation lies too near the strike (half of the
+// options: under 0.004). A cut that is too near costs a second march after the first, which
+// a whole launch may wait for (0.5 ms of 2.2 for one option of 16384); the margin costs about
+// 10 rows of 1024. The cut needs
 //   * kPinnedRows rows to forget the approximate value they are started from: with
 //     a = theta dt (sigma^2 / 2) / dx^2 at the cut, an error shrinks by about
 //     e^{-1/sqrt(a)} per row, and a <= 150 leaves 1e-9 of an error of O(dt^2);
@@ -115,10 +118,11 @@ KWGPU_HD Window window_of(const kwgpu_option& o, int N, int steps, double densit
     const double r = o.w < 0 ? o.r : o.q, q = o.w < 0 ? o.q : o.r;
     if (!o.e || !(r > 0.0)) return w;
     if (q > r && log(q / r) > 4.5 * s) return w;
-    const double xb = (double)critical_log_spot((float)o.t, (float)o.z, (float)r, (float)q) - 0.04;
+    const double xb = (double)critical_log_spot((float)o.t, (float)o.z, (float)r, (float)q) -
+                      fmin(0.075, 0.24 * s);
     if (!(xb > -6.9)) return w;  // nor when it is no number
     const double at = (asinh(xb / density) + Y) * per;
-    const int lo = (int)floor(at) - 3;
+    const int lo = (int)floor(at) - 2;
     if (lo < 16 || lo >= w.end - 8) return w;
     const double dx = sqrt(xb * xb + density * density) * h;
     const double a1 = 0.25 * s2 / steps;  // a at dx = 1

@@ -119,6 +119,18 @@ struct Geo {
     static constexpr int G = NT / LT;           // options per workgroup
 };
 
+// Orders an option's LDS accesses among its lanes: a wave's own are executed in order, so one
+// wave only has to keep the compiler from moving them; two waves meet at a barrier.
+template <int W>
+__device__ __forceinline__ void group_sync() {
+    if constexpr (W == 2) {
+        __syncthreads();
+    } else {
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+    }
+}
+
 struct Lanes {
     int gl, wv, lane, seg, ls, row16, wrow, pr;
 };
@@ -411,9 +423,9 @@ __device__ __forceinline__ void setup(const FdBatch& b, const Pde& d, const Lane
     }
     // the last row of a lane needs the next lane's first pivot (bu = 0 on the last real
     // row and on padding rows, so the segment end needs none)
-    __syncthreads();
+    group_sync<W>();
     qp[gl] = d0;
-    __syncthreads();
+    group_sync<W>();
     up[M - 1] = (TF)(buv[M - 1] * (t.ls + 1 < LT ? rcp(qp[gl + 1]) : 1.0));
     if constexpr (WIN) {
         // no carry enters a window: 0 from the pinned side (alpha is in k0), and x = 0
@@ -449,7 +461,7 @@ __device__ __forceinline__ void setup(const FdBatch& b, const Pde& d, const Lane
         const double w2 = Pl * dpp<kRowShr + 1>(Pl);  // Pl over lanes l-1 .. l
         const double w4 = w2 * dpp<kRowShr + 2>(w2);  // l-3 .. l
         const double w8 = w4 * dpp<kRowShr + 4>(w4);  // l-7 .. l
-        if constexpr (WIN) {
+        if constexpr (WIN && W == 1) {
             // quads first, then quads into rows: prefixes (Pl) and suffixes (Ql) within a quad
             const int qd = t.lane & 3;
             double a = Pl, z = Ql, x;
@@ -505,7 +517,7 @@ __device__ __forceinline__ void setup(const FdBatch& b, const Pde& d, const Lane
         sm.X16 = (TF)((w64 && wrow == 0) || (w32 && (wrow & 1) == 0) ? sq : 0.0);
         sm.X32 = (TF)(w64 && wrow == 1 ? sq : 0.0);
         sm.X48 = (TF)(w64 && wrow == 2 ? sq : 0.0);
-        if constexpr (WIN) {
+        if constexpr (WIN && W == 1) {
             sm.X16 = sq;  // rows 0 and 2 take the next row's first lane
             sm.X32 = wrow == 1 ? sq : wrow == 0 ? sq * rs1 : 0.0;  // rows 0, 1 take lane 32
         }
@@ -535,9 +547,9 @@ __device__ __forceinline__ int group_steps(const Pde& d, const Lanes& t, double*
         if (wmin) *wmin = d.steps;
         return d.steps;
     } else {
-        __syncthreads();
+        group_sync<W>();
         qp[t.gl] = (double)d.steps;
-        __syncthreads();
+        group_sync<W>();
         double mx = 0.0, mn = 1e300;
         for (int k = 0; k < Gm::NT; k += Gm::LT) {
             mx = fmax(mx, qp[k]);
@@ -794,7 +806,7 @@ __device__ __forceinline__ void march_f64(double (&xv)[M], const double (&ap)[M]
     // options mostly) and on 1024 points (32- and 64-lane ones): 741, 1088 and 1840 us with
     // the pairs read at the point of use, 566, 890 and 1525 us read 4 ahead; 2 to 8 ahead
     // differ by less than 3 %.
-    constexpr int PF0 = WIN ? (ONE ? 3 : 4) : W == 2 ? KWGPU_PF2 : ONE ? KWGPU_PF1 : KWGPU_PFG;
+    constexpr int PF0 = WIN ? (ONE && W == 1 ? 3 : 4) : W == 2 ? KWGPU_PF2 : ONE ? KWGPU_PF1 : KWGPU_PFG;
     constexpr int PF = PF0 < M ? PF0 : M - 1;  // 0: each pair read where it is used
     const int wv = __builtin_amdgcn_readfirstlane(t.wv);  // wave of a W = 2 group
     double g[M];
@@ -891,6 +903,29 @@ __device__ __forceinline__ void march_f64(double (&xv)[M], const double (&ap)[M]
     }
 }
 
+// Two-wave groups: the coefficients of the one value that the waves exchange per step (AW,
+// BW in `aw`, `bw`; TW0 in sm).
+__device__ __forceinline__ void two_wave_carries(double r0, const Lanes& t, ScanMul<double>& sm,
+                                                 double* xchg, double& aw, double& bw) {
+    // wave 1: c0 enters lane l's forward carry with FW of lane l-1 (1 in lane 0) and
+    // its backward carry through the backward scan of R_0 times that; wave 0: wave
+    // 1's first backward carry enters lane l's with ZW of lane l+1 (1 in lane 63)
+    // Every shift runs on the whole wave before any select: a DPP move inside a
+    // branch reads 0 from the lanes the branch turns off.
+    const double fw_prev = dpp<kWaveShr1>(sm.FW);
+    const double zw_next = dpp<kWaveShl1>(sm.ZW);
+    const double fws = t.wv == 1 ? (t.lane == 0 ? 1.0 : fw_prev) : 0.0;
+    const double tw = bwd_scan<64>(r0 * fws, sm, t);
+    const double tw_next = dpp<kWaveShl1>(tw);
+    const double zws = t.wv == 0 ? (t.lane == 63 ? 1.0 : zw_next) : 0.0;
+    aw = fws;
+    bw = t.wv == 0 ? zws : tw_next;
+    __syncthreads();
+    if (t.wv == 1 && t.lane == 0) xchg[0] = tw;
+    __syncthreads();
+    sm.TW0 = readlane<0>(xchg[0]);  // uniform: keep it in scalar registers
+}
+
 // GTH: general theta. The theta = 1/2 kernel holds only its own march, so set-up values
 // that only the general march needs are not kept (and spilled) on its path.
 template <int M, int L, int W, bool GTH>
@@ -912,25 +947,7 @@ __device__ __forceinline__ void solve_group_f64(const FdBatch& b, int group, dou
     wmin = __builtin_amdgcn_readfirstlane(wmin);
     double aw = 0.0, bw = 0.0;
     sm.TW0 = 0.0;
-    if constexpr (W == 2) {
-        // wave 1: c0 enters lane l's forward carry with FW of lane l-1 (1 in lane 0) and
-        // its backward carry through the backward scan of R_0 times that; wave 0: wave
-        // 1's first backward carry enters lane l's with ZW of lane l+1 (1 in lane 63)
-        // Every shift runs on the whole wave before any select: a DPP move inside a
-        // branch reads 0 from the lanes the branch turns off.
-        const double fw_prev = dpp<kWaveShr1>(sm.FW);
-        const double zw_next = dpp<kWaveShl1>(sm.ZW);
-        const double fws = t.wv == 1 ? (t.lane == 0 ? 1.0 : fw_prev) : 0.0;
-        const double tw = bwd_scan<L>(R[0] * fws, sm, t);
-        const double tw_next = dpp<kWaveShl1>(tw);
-        const double zws = t.wv == 0 ? (t.lane == 63 ? 1.0 : zw_next) : 0.0;
-        aw = fws;
-        bw = t.wv == 0 ? zws : tw_next;
-        __syncthreads();
-        if (t.wv == 1 && t.lane == 0) xchg[0] = tw;
-        __syncthreads();
-        sm.TW0 = readlane<0>(xchg[0]);  // uniform: keep it in scalar registers
-    }
+    if constexpr (W == 2) two_wave_carries(R[0], t, sm, xchg, aw, bw);
 
     // (Q_i, projection target_i) pairs of every thread at qpv[i * NT + gl]; two-wave
     // groups add (AW, BW) at qpv[M * NT + gl]
@@ -1166,22 +1183,29 @@ hipError_t launch_fd1d_lone(const FdBatch& b, hipStream_t s) {
     return hipGetLastError();
 }
 
-hipError_t launch_fd1d_windowed(const FdBatch& b, const WindowScratch& w, int n_big,
-                                hipStream_t s) {
+hipError_t launch_fd1d_windowed(const FdBatch& b, const WindowScratch& w, int n_big, hipStream_t s) {
     if (b.m <= 0) return hipSuccess;
+    if (b.m <= kLoneMax && n_big == 0) return launch_fd1d_lone(b, s);
     if (b.theta != 0.5 || !w.rec || !w.list || !w.counts) return hipErrorInvalidValue;
-    if (n_big == 0 && b.m <= kLoneMax) return launch_fd1d_lone(b, s);
-    int* cursor = w.counts + kWindowCounters / 2;
-    const unsigned nb = (unsigned)((b.m + 255) / 256);
+    uint32_t* later = w.list + b.m;
     if (hipError_t e = launch_zero_counters(w.counts, kWindowCounters, s)) return e;
-    hipLaunchKernelGGL(plan_windows, dim3(nb), dim3(256), 0, s, b, w.rec, w.counts);
-    hipLaunchKernelGGL(list_windows, dim3(nb), dim3(256), 0, s, b, (const int*)w.rec,
-                       (const int*)w.counts, cursor, w.list);
-    hipLaunchKernelGGL(fd1d_windowed, dim3(b.m), dim3(64), 0, s, b, (const int*)w.rec, w.counts,
-                       w.list);
+    if (b.m <= kLoneMax / 2) {
+        hipLaunchKernelGGL(fd1d_lone_big, dim3(b.m), dim3(128), 0, s, b, w.counts, later);
+    } else {
+        const unsigned nb = (unsigned)((b.m + 255) / 256);
+        hipLaunchKernelGGL(plan_windows, dim3(nb), dim3(256), 0, s, b, w.rec, w.counts);
+        hipLaunchKernelGGL(list_windows, dim3(nb), dim3(256), 0, s, b, (const int*)w.rec,
+                           (const int*)w.counts, w.counts + kWindowCounters / 2, w.list);
+        if (n_big > 0)
+            hipLaunchKernelGGL(fd1d_windowed_big, dim3(n_big + (b.m + 1) / 2), dim3(128), 0, s, b,
+                               (const int*)w.rec, w.counts, (const uint32_t*)w.list, later);
+        else
+            hipLaunchKernelGGL(fd1d_windowed, dim3(b.m), dim3(64), 0, s, b, (const int*)w.rec,
+                               w.counts, (const uint32_t*)w.list);
+    }
     if (n_big > 0)
-        hipLaunchKernelGGL(fd1d_window_big, dim3(n_big), dim3(128), 0, s, b, (const int*)w.counts,
-                           (const uint32_t*)w.list);
+        hipLaunchKernelGGL(fd1d_window_again, dim3(n_big), dim3(128), 0, s, b,
+                           (const int*)w.counts, (const uint32_t*)later);
     return hipGetLastError();
 }
 

@@ -6,33 +6,36 @@
 // the rows it carries: about 6 per row and step, plus two lane scans per wave and step.
 // A window holds 45 % of a grid's rows on average (1024 points, vol 10-60 %, T 1/12-3), so
 // most options of a 1024-point grid fit 512 rows, two to a wave. Measured against the
-// whole-grid march on one card: 32768 options at 1024 x 1024 9.73 -> 5.42 ms (VALU
+// whole-grid march on one card: 32768 options at 1024 x 1024 9.77 -> 5.44 ms (VALU
 // instructions 4.75e9 -> 2.49e9, their issue 90 % busy instead of 98 % at 1.9 GHz), 16384 on
-// per-option grids of 256 to 2048 points 3.53 -> 1.83 ms, 3001 at 777 x 301 267 -> 163 us.
+// per-option grids of 256 to 2048 points 3.58 -> 1.76 ms, 3001 at 777 x 301 267 -> 163 us.
 //
 // Rows run from the in-the-money side (positions in xi), so the rows in front of a window
 // are the ones pinned to the payoff: each step's forward elimination runs over constant
 // values there and leaves the same relation x_{lo-1} = alpha + beta x_lo at every step,
 // computed once. Nothing is approximated on that side. Beyond the window's end x is 0.
 
-// Row counts that a march is built for, the costliest first: class c holds up to M * L rows,
-// 64 / L options to a wave. The last class, kWindowBig, is for windows of over 1024 rows:
-// the whole 2048-point grid in two waves. VALU instructions per step and option, scans
-// included: 129, 105, 93, 64, 52, 30, 24, 18 (the whole-grid march: 137 for 1024 points, 69
-// for 512, 33 for 256).
+// Row counts that a march is built for: class c holds up to M * L * W rows. Class 0 is the
+// whole 2048-point grid in two waves and class 1 the two-wave march of 1280 rows (a sixth of
+// the windows of a 2048-point grid have 1025 to 1280 rows); of the one-wave classes the
+// costliest come first, 64 / L options to a wave. VALU instructions per step and option, scans
+// included, from class 2: 129, 105, 93, 64, 52, 30, 24, 18 (the whole-grid march: 137 for 1024
+// points, 69 for 512, 33 for 256); classes 0 and 1: 292 and 218.
 struct WindowClass {
-    int M, L;
+    int M, L, W;
 };
-constexpr WindowClass kWindowClasses[] = {{16, 64}, {12, 64}, {10, 64}, {16, 32},
-                                          {12, 32}, {16, 16}, {12, 16}, {8, 16}};
-constexpr int kWindowBig = sizeof(kWindowClasses) / sizeof(kWindowClasses[0]);
-static_assert(kWindowBig + 1 <= kWindowCounters / 2, "a count and a cursor per class");
+constexpr WindowClass kWindowClasses[] = {{16, 64, 2}, {10, 64, 2}, {16, 64, 1}, {12, 64, 1}, {10, 64, 1},
+                                          {16, 32, 1}, {12, 32, 1}, {16, 16, 1}, {12, 16, 1}, {8, 16, 1}};
+constexpr int kClasses = sizeof(kWindowClasses) / sizeof(kWindowClasses[0]);
+constexpr int kTwoWave = 2;         // classes below are two-wave
+constexpr int kAgain = kClasses;    // counter of the PDEs to be solved again in two waves
+static_assert(kClasses + 1 <= kWindowCounters / 2, "a count and a cursor per class");
 
 __device__ __forceinline__ int window_class(int rows) {
-    int c = kWindowBig;
+    int c = 0;
 #pragma unroll
-    for (int k = 0; k < kWindowBig; ++k)
-        if (rows <= kWindowClasses[k].M * kWindowClasses[k].L) c = k;
+    for (int k = 1; k < kClasses; ++k)
+        if (rows <= kWindowClasses[k].M * kWindowClasses[k].L * kWindowClasses[k].W) c = k;
     return c;
 }
 
@@ -72,12 +75,14 @@ __device__ __forceinline__ PinnedMap pinned_step(bool take, const PinnedMap& s) 
             take ? y.b : s.b, take ? y.c : s.c,   take ? y.d : s.d};
 }
 
-template <int L>
+// In a two-wave group both waves compute it.
+template <int L, int W>
 __device__ __forceinline__ void pinned_edge(const FdBatch& b, const PdeParams& P,
                                             const kwgpu_option& o, const Lanes& t, double* qp,
                                             Edge& e) {
     constexpr int K = kPinnedRows / L;
-    const int i0 = e.lo - kPinnedRows + t.ls * K;
+    const int l = W == 2 ? t.lane : t.ls;
+    const int i0 = e.lo - kPinnedRows + l * K;
     const double yj = (i0 - 1) * P.dy;
     double ey = exp(P.yMin * (1.0 - yj) + P.yMax * yj), ef = rcp(ey);
     const double grow = exp((P.yMax - P.yMin) * P.dy), shrink = rcp(grow);
@@ -118,31 +123,32 @@ __device__ __forceinline__ void pinned_edge(const FdBatch& b, const PdeParams& P
     s = pinned_step<kRowShr + 8>(t.pr >= 8, s);
     if constexpr (L >= 32) s = pinned_step<kRowBcast15, 0xA>(t.wrow & 1, s);
     if constexpr (L == 64) s = pinned_step<kRowBcast31, 0xC>(t.wrow >= 2, s);
-    __syncthreads();
-    if (t.ls == 0) qp[4 * t.seg] = start;
-    if (t.ls == L - 1) {
+    group_sync<W>();
+    if (l == 0) qp[4 * t.seg] = start;
+    if (l == L - 1) {
         qp[4 * t.seg + 1] = s.p;
         qp[4 * t.seg + 2] = s.q2;
         qp[4 * t.seg + 3] = s.b;
         qp[16 + t.seg] = s.d;
     }
-    __syncthreads();
+    group_sync<W>();
     const double inv = 1.0 / qp[16 + t.seg];
     const bool on = e.lo > 0;
     e.alpha = on ? (qp[4 * t.seg + 1] * (e.lo > kPinnedRows ? qp[4 * t.seg] : 0.0) + qp[4 * t.seg + 2]) * inv : 0.0;
     e.beta = on ? qp[4 * t.seg + 3] * inv : 0.0;
-    __syncthreads();
+    group_sync<W>();
 }
 
-// One wave's work: the options ids[slot] .. (or slot itself without ids), at most `slots`,
-// each on its window (rec[p], or its whole grid when rec is null). Bit k of the result:
-// segment k's option has to be solved again on its whole grid (nothing was written for it).
-template <int M, int L>
+// One wave's (W = 2: one workgroup's) work: the options ids[slot] .. (or slot itself without
+// ids), at most `slots`, each on its window (from rec[p], or lo_all when rec is null). Bit k
+// of the result: segment k's option has to be solved again on its whole grid (what was
+// written for it does not stand).
+template <int M, int L, int W = 1>
 __device__ __forceinline__ unsigned solve_window(const FdBatch& b, const uint32_t* ids,
                                                  const int* rec, int lo_all, int slot0, int slots,
-                                                 double* qp) {
-    using Gm = Geo<M, L, 1>;
-    constexpr int NT = Gm::NT;
+                                                 double* qp, double* xchg = nullptr) {
+    using Gm = Geo<M, L, W>;
+    constexpr int NT = Gm::NT, LT = Gm::LT;
     auto pde = [&](const Lanes& t, int s0, int& lo) {
         Pde d;
         const int slot = s0 + t.seg;
@@ -161,20 +167,37 @@ __device__ __forceinline__ unsigned solve_window(const FdBatch& b, const uint32_
         if (d.P.call) d.P.ax = -d.P.ax;
         return d;
     };
+    // one bit per segment in which any lane says so
+    auto segments = [&](bool v) {
+        unsigned r = 0;
+        if constexpr (W == 2) {
+            r = __syncthreads_or(v) ? 1u : 0u;
+        } else {
+            const uint64_t votes = __ballot(v);
+            constexpr uint64_t seg = L == 64 ? ~0ull : ((1ull << (L & 63)) - 1);
+#pragma unroll
+            for (int k = 0; k < Gm::G; ++k)
+                if (votes & (seg << (k * (L & 63)))) r |= 1u << k;
+        }
+        return r;
+    };
     unsigned again = 0;
     double xv[M];
     {
-        const Lanes t = lanes_of<M, L, 1>(threadIdx.x);
+        const Lanes t = lanes_of<M, L, W>(threadIdx.x & (NT - 1));
         Edge edge{};
         const Pde d = pde(t, slot0, edge.lo);
-        if (__ballot(edge.lo > 0)) pinned_edge<L>(b, d.P, d.opt, t, qp, edge);
+        if (__ballot(edge.lo > 0)) pinned_edge<L, W>(b, d.P, d.opt, t, qp, edge);
         double ap[M], lo[M], up[M], R[M], Q[M], blv[M], buv[M];
         ScanMul<double> sm;
-        setup<M, L, 1, true>(b, d, t, qp, xv, ap, lo, up, R, Q, blv, buv, sm, &edge);
+        setup<M, L, W, true>(b, d, t, qp, xv, ap, lo, up, R, Q, blv, buv, sm, &edge);
         int wmin = 0;
-        const int wsteps = __builtin_amdgcn_readfirstlane(group_steps<M, L, 1>(d, t, qp, &wmin));
+        const int wsteps = __builtin_amdgcn_readfirstlane(group_steps<M, L, W>(d, t, qp, &wmin));
         wmin = __builtin_amdgcn_readfirstlane(wmin);
-        __syncthreads();
+        double aw = 0.0, bw = 0.0;
+        sm.TW0 = 0.0;
+        if constexpr (W == 2) two_wave_carries(R[0], t, sm, xchg, aw, bw);
+        group_sync<W>();
         double2* qpv = reinterpret_cast<double2*>(qp);
 #pragma unroll
         for (int i = 0; i < M; ++i) {
@@ -184,40 +207,35 @@ __device__ __forceinline__ unsigned solve_window(const FdBatch& b, const uint32_
             const bool proj = d.P.american && at < d.N && at != (d.P.call ? 0 : d.N - 1);
             qpv[i * NT + t.gl] = make_double2(Q[i], proj ? xv[i] : -INFINITY);
         }
-        __syncthreads();
-        march_f64<M, L, 1, true, true>(xv, ap, lo, up, R, qpv, sm, t, t.ls == 0, t.ls == L - 1,
-                                       nullptr, wmin, wsteps, d.steps, 1.0, edge.k0);
+        if constexpr (W == 2) qpv[M * NT + t.gl] = make_double2(aw, bw);
+        group_sync<W>();
+        march_f64<M, L, W, true, true>(xv, ap, lo, up, R, qpv, sm, t, t.ls == 0, t.ls == LT - 1,
+                                       xchg, wmin, wsteps, d.steps, 1.0, edge.k0);
         // the cut holds if the window's first two rows are still pinned
-        const bool moved = t.ls == 0 && edge.lo > 0 &&
-                           !(xv[0] == qpv[t.gl].y && xv[1] == qpv[NT + t.gl].y);
-        const uint64_t votes = __ballot(moved);
-#pragma unroll
-        for (int k = 0; k < Gm::G; ++k)
-            if (votes >> (k * L) & 1) again |= 1u << k;
+        again = segments(t.ls == 0 && edge.lo > 0 &&
+                         !(xv[0] == qpv[t.gl].y && xv[1] == qpv[NT + t.gl].y));
     }
     // the option's record and lane indices are derived again rather than kept in registers
     // over the march (as in solve_group_f64)
-    int s2 = slot0, tid = threadIdx.x;
+    int s2 = slot0, tid = threadIdx.x & (NT - 1);
     asm volatile("" : "+v"(s2), "+v"(tid));
-    const Lanes t = lanes_of<M, L, 1>(tid);
+    const Lanes t = lanes_of<M, L, W>(tid);
     int lo = 0;
     const Pde d = pde(t, s2, lo);
     bool bad = false;
 #pragma unroll
     for (int i = 0; i < M; ++i) bad |= d.j0 + i < d.N && !isfinite(xv[i]);
-    const uint64_t votes = __ballot(bad);
-    const uint64_t mine = L == 64 ? ~0ull : (((1ull << (L & 63)) - 1) << (t.seg * L));
-    const bool seg_bad = (votes & mine) != 0;
-    __syncthreads();
+    const bool seg_bad = segments(bad) >> t.seg & 1;
+    group_sync<W>();
 #pragma unroll
-    for (int i = 0; i < M; ++i) qp[t.seg * L * M + t.ls * M + i] = xv[i];
-    __syncthreads();
+    for (int i = 0; i < M; ++i) qp[t.seg * LT * M + t.ls * M + i] = xv[i];
+    group_sync<W>();
     bool outside = false;
     if (d.live && !(again >> t.seg & 1)) {
-        const double* V = qp + t.seg * L * M;
+        const double* V = qp + t.seg * LT * M;
         const uint32_t beg = b.off ? b.off[d.p] : 0u;
         const uint32_t end = b.off ? b.off[d.p + 1] : 1u;
-        for (uint32_t k = beg + t.ls; k < end; k += L) {
+        for (uint32_t k = beg + t.ls; k < end; k += LT) {
             const uint32_t o2 = b.off ? b.list[k] : d.oi;
             const kwgpu_option q = b.off ? b.opts[o2] : d.opt;
             double price = NAN;
@@ -237,8 +255,8 @@ __device__ __forceinline__ unsigned solve_window(const FdBatch& b, const uint32_
                             outside |= d.P.call && at == 0;
                             return payoff(d.P, x);
                         }
-                        outside |= at >= lo + L * M;
-                        return V[min(at - lo, L * M - 1)];
+                        outside |= at >= lo + LT * M;
+                        return V[min(at - lo, LT * M - 1)];
                     };
                     const double v0 = value(j - 1, x0), v1 = value(j, x1);
                     if (seg_bad) {
@@ -253,12 +271,8 @@ __device__ __forceinline__ unsigned solve_window(const FdBatch& b, const uint32_
             if (b.status) b.status[o2] = st;
         }
     }
-    const uint64_t out = __ballot(outside);
-#pragma unroll
-    for (int k = 0; k < Gm::G; ++k) {
-        const uint64_t seg = L == 64 ? ~0ull : (((1ull << (L & 63)) - 1) << (k * L));
-        if (out & seg) again |= 1u << k;
-    }
+    again |= segments(outside);
+    if constexpr (W == 2) group_sync<W>();  // before LDS is used for the next option
     return again;
 }
 
@@ -282,8 +296,8 @@ __device__ __forceinline__ double far_xi(const FdBatch& b, int p, uint32_t oi, u
 constexpr uint32_t kFarOptions = 256;
 
 __global__ __launch_bounds__(256) void plan_windows(FdBatch b, int* rec, int* counts) {
-    __shared__ int n[kWindowBig + 1];
-    if (threadIdx.x <= kWindowBig) n[threadIdx.x] = 0;
+    __shared__ int n[kClasses];
+    if (threadIdx.x < kClasses) n[threadIdx.x] = 0;
     __syncthreads();
     const int slot = blockIdx.x * 256 + threadIdx.x;
     if (slot < b.m) {
@@ -294,20 +308,19 @@ __global__ __launch_bounds__(256) void plan_windows(FdBatch b, int* rec, int* co
         Window w{0, N};
         if (!b.off || b.off[p + 1] - b.off[p] <= kFarOptions)
             w = window_of(b.opts[oi], N, td - 1, b.density, b.scale, far_xi(b, p, oi, 0, 1));
-        int c = window_class(w.end - w.lo);
-        if (c == kWindowBig) w.lo = 0;
+        const int c = window_class(w.end - w.lo);
         rec[p] = w.lo | c << 16;
         atomicAdd(&n[c], 1);
     }
     __syncthreads();
-    if (threadIdx.x <= kWindowBig && n[threadIdx.x]) atomicAdd(&counts[threadIdx.x], n[threadIdx.x]);
+    if (threadIdx.x < kClasses && n[threadIdx.x]) atomicAdd(&counts[threadIdx.x], n[threadIdx.x]);
 }
 
 // ... and the PDEs listed class by class, in slot order within each block of 256 slots (so
 // PDEs sorted by march length stay so, and those that share a wave march about as long).
 __global__ __launch_bounds__(256) void list_windows(FdBatch b, const int* rec, const int* counts,
                                                     int* cursor, uint32_t* list) {
-    constexpr int C = kWindowBig + 1;
+    constexpr int C = kClasses;
     __shared__ int n[4][C], at[C];
     const int slot = blockIdx.x * 256 + threadIdx.x, w = threadIdx.x >> 6, lane = threadIdx.x & 63;
     int p = 0, c = -1;
@@ -336,70 +349,101 @@ __global__ __launch_bounds__(256) void list_windows(FdBatch b, const int* rec, c
     }
 }
 
+// An option whose boundary went past its window's cut, of a grid too large for one wave: to
+// be solved again by fd1d_window_again.
+__device__ __forceinline__ void solve_later(uint32_t p, int* counts, uint32_t* later) {
+    if ((threadIdx.x & 63) == 0) later[atomicAdd(&counts[kAgain], 1)] = p;
+}
+
 // Few options: one to a wave, spread over all 64 lanes with as few rows per lane as its window
-// needs, each finding its own window. Nothing is listed and no scratch is used. The step's
-// length is then its chain of dependent instructions -- the lane's two substitutions and the
-// lane scans -- rather than their number. Up to kLoneMax options, two waves to a SIMD, all
-// are resident at once. 512 x 512, by number of options: 128 in 142 us here (238 us on whole
-// grids, 16 rows a lane), 2048 in 199 us; listed by class 2048 take about 220 us and 3072
-// 230 us, here 287 us.
-__global__ __attribute__((amdgpu_flat_work_group_size(64, 64), amdgpu_waves_per_eu(2, 2)))
-void fd1d_lone(FdBatch b) {
-    __shared__ double qp[2 * 64 * 16];
-    const int slot = blockIdx.x;
+// needs, each finding its own window. Nothing is listed, and grids of up to 1024 points take
+// no scratch. The step's length is then its chain of dependent instructions -- the lane's two
+// substitutions and the lane scans -- rather than their number. Up to kLoneMax options, two
+// waves to a SIMD, all are resident at once. 512 x 512, by number of options: 128 in 142 us
+// here (238 us on whole grids, 16 rows a lane), 2048 in 199 us; listed by class 2048 take
+// about 220 us and 3072 230 us, here 287 us.
+struct LoneWindow {
+    int lo, rows, N;
+};
+__device__ __forceinline__ LoneWindow lone_window(const FdBatch& b, int slot) {
     const int p = b.order ? (int)b.order[slot] : slot;
     const uint32_t oi = b.rep ? b.rep[p] : (uint32_t)p;
     const int N = b.x_dims ? b.x_dims[oi] : b.x_dim;
     const int td = b.t_dims ? b.t_dims[oi] : b.t_dim;
-    double far = far_xi(b, p, oi, threadIdx.x, 64);
+    double far = far_xi(b, p, oi, threadIdx.x & 63, 64);
     for (int k = 32; k > 0; k >>= 1) far = fmax(far, __shfl_xor(far, k));
     const Window w = window_of(b.opts[oi], N, td - 1, b.density, b.scale, far);
-    int lo = __builtin_amdgcn_readfirstlane(w.lo);
-    int rows = __builtin_amdgcn_readfirstlane(w.end - w.lo);
+    return {__builtin_amdgcn_readfirstlane(w.lo), __builtin_amdgcn_readfirstlane(w.end - w.lo), N};
+}
+
+__device__ __forceinline__ void lone_wave(const FdBatch& b, int slot, LoneWindow w, double* qp,
+                                          int* counts, uint32_t* later) {
     for (;;) {
         unsigned again;
-        if (rows <= 256)
-            again = solve_window<4, 64>(b, b.order, nullptr, lo, slot, slot + 1, qp);
-        else if (rows <= 384)
-            again = solve_window<6, 64>(b, b.order, nullptr, lo, slot, slot + 1, qp);
-        else if (rows <= 512)
-            again = solve_window<8, 64>(b, b.order, nullptr, lo, slot, slot + 1, qp);
-        else if (rows <= 768)
-            again = solve_window<12, 64>(b, b.order, nullptr, lo, slot, slot + 1, qp);
+        if (w.rows <= 256)
+            again = solve_window<4, 64>(b, b.order, nullptr, w.lo, slot, slot + 1, qp);
+        else if (w.rows <= 384)
+            again = solve_window<6, 64>(b, b.order, nullptr, w.lo, slot, slot + 1, qp);
+        else if (w.rows <= 512)
+            again = solve_window<8, 64>(b, b.order, nullptr, w.lo, slot, slot + 1, qp);
+        else if (w.rows <= 768)
+            again = solve_window<12, 64>(b, b.order, nullptr, w.lo, slot, slot + 1, qp);
         else
-            again = solve_window<16, 64>(b, b.order, nullptr, lo, slot, slot + 1, qp);
+            again = solve_window<16, 64>(b, b.order, nullptr, w.lo, slot, slot + 1, qp);
         if (!again) return;
-        lo = 0;  // the whole grid: nothing is pinned, nothing lies outside
-        rows = N;
+        if (w.N > 1024) return solve_later(b.order ? b.order[slot] : (uint32_t)slot, counts, later);
+        w.lo = 0;  // the whole grid: nothing is pinned, nothing lies outside
+        w.rows = w.N;
     }
 }
 
-// Runs class c's march over the wave starting at slot.
+__global__ __attribute__((amdgpu_flat_work_group_size(64, 64), amdgpu_waves_per_eu(2, 2)))
+void fd1d_lone(FdBatch b) {
+    __shared__ double qp[2 * 64 * 16];
+    lone_wave(b, blockIdx.x, lone_window(b, blockIdx.x), qp, nullptr, nullptr);
+}
+
+// ... and with grids of over 1024 points: a workgroup of two waves an option, for windows of
+// over 1024 rows, which march on their whole grids; otherwise the second wave ends at once.
+// (The two kinds of march in launches of their own, side by side, kept each other from the
+// SIMDs: 1024 options at 2048 x 512 took 705 us.) Up to kLoneMax / 2 options are resident.
+__global__ __attribute__((amdgpu_flat_work_group_size(128, 128), amdgpu_waves_per_eu(2, 2)))
+void fd1d_lone_big(FdBatch b, int* counts, uint32_t* later) {
+    __shared__ double qp[2 * 128 * 17];
+    __shared__ double xchg[4];
+    const LoneWindow w = lone_window(b, blockIdx.x);
+    if (w.rows > 1024)
+        solve_group_f64<16, 64, 2, false>(b, blockIdx.x, qp, xchg);
+    else if (threadIdx.x < 64)
+        lone_wave(b, blockIdx.x, w, qp, counts, later);
+}
+
+// Runs one-wave class c's march over the wave starting at slot.
 __device__ __forceinline__ unsigned run_class(int c, const FdBatch& b, const uint32_t* ids,
                                               const int* rec, int lo, int slot, int slots,
                                               double* qp) {
     switch (c) {
-        case 0: return solve_window<16, 64>(b, ids, rec, lo, slot, slots, qp);
-        case 1: return solve_window<12, 64>(b, ids, rec, lo, slot, slots, qp);
-        case 2: return solve_window<10, 64>(b, ids, rec, lo, slot, slots, qp);
-        case 3: return solve_window<16, 32>(b, ids, rec, lo, slot, slots, qp);
-        case 4: return solve_window<12, 32>(b, ids, rec, lo, slot, slots, qp);
-        case 5: return solve_window<16, 16>(b, ids, rec, lo, slot, slots, qp);
-        case 6: return solve_window<12, 16>(b, ids, rec, lo, slot, slots, qp);
+        case 2: return solve_window<16, 64>(b, ids, rec, lo, slot, slots, qp);
+        case 3: return solve_window<12, 64>(b, ids, rec, lo, slot, slots, qp);
+        case 4: return solve_window<10, 64>(b, ids, rec, lo, slot, slots, qp);
+        case 5: return solve_window<16, 32>(b, ids, rec, lo, slot, slots, qp);
+        case 6: return solve_window<12, 32>(b, ids, rec, lo, slot, slots, qp);
+        case 7: return solve_window<16, 16>(b, ids, rec, lo, slot, slots, qp);
+        case 8: return solve_window<12, 16>(b, ids, rec, lo, slot, slots, qp);
         default: return solve_window<8, 16>(b, ids, rec, lo, slot, slots, qp);
     }
 }
 
-// All classes but kWindowBig in one launch (one kernel: no tail of idle SIMDs between
-// classes): workgroup i takes the i-th wave of work, classes in order; those past the last
-// wave leave at once. An option whose boundary passed its cut is solved again on its whole
-// grid by the same wave, or, above 1024 points, joins the two-wave launch's list.
-__global__ __attribute__((amdgpu_flat_work_group_size(64, 64), amdgpu_waves_per_eu(2, 2)))
-void fd1d_windowed(FdBatch b, const int* rec, int* counts, uint32_t* list) {
-    __shared__ double qp[2 * 64 * 16];
-    int c = 0, begin = 0, g = blockIdx.x, slots = 0;
+// Wave g's share of the one-wave classes, in order; nothing past the last one. An option whose
+// boundary passed its cut is solved again on its whole grid by the same wave, or, above 1024
+// points, later.
+__device__ __forceinline__ void run_wave(const FdBatch& b, int g, const int* rec, int* counts,
+                                         const uint32_t* list, uint32_t* later, double* qp) {
+    int c = kTwoWave, begin = 0, slots = 0;
+#pragma unroll
+    for (int k = 0; k < kTwoWave; ++k) begin += counts[k];
     for (;; ++c) {
-        if (c == kWindowBig) return;
+        if (c == kClasses) return;
         slots = counts[c];
         const int G = 64 / kWindowClasses[c].L, groups = (slots + G - 1) / G;
         if (g < groups) break;
@@ -417,29 +461,54 @@ void fd1d_windowed(FdBatch b, const int* rec, int* counts, uint32_t* list) {
             slot = first + __ffs(pending) - 1;
             const uint32_t p = ids[slot], oi = b.rep ? b.rep[p] : p;
             if ((b.x_dims ? b.x_dims[oi] : b.x_dim) <= 1024) break;
-            if (threadIdx.x == 0) {
-                int base = 0;
-                for (int i = 0; i < kWindowBig; ++i) base += counts[i];
-                list[base + atomicAdd(&counts[kWindowBig], 1)] = p;
-            }
+            solve_later(p, counts, later);
         }
         if (!pending) return;
         pending &= pending - 1;
-        c = 0;
+        c = kTwoWave;
         slots = slot + 1;
     }
 }
 
-// The whole-grid two-wave march over the list's last class. `counts` is final by now: the
-// launch above has ended.
+// All classes in one launch. 16384 options on per-option grids, one call at a time: 2.56 ms
+// with the two-wave groups, on whole grids, in a launch after the others (each launch ends
+// with idle SIMDs), 2.12 ms with three launches on streams of their own (which keep each other
+// from the SIMDs when several contexts are at work), 2.20 ms as one; 65536 8.28, 7.83 and 7.30
+// ms. Grids of up to 1024 points: a wave a workgroup.
+__global__ __attribute__((amdgpu_flat_work_group_size(64, 64), amdgpu_waves_per_eu(2, 2)))
+void fd1d_windowed(FdBatch b, const int* rec, int* counts, const uint32_t* list) {
+    __shared__ double qp[2 * 64 * 16];
+    run_wave(b, blockIdx.x, rec, counts, list, nullptr, qp);
+}
+
+// ... and larger ones: workgroups of two waves, first (they march longest) one option each of
+// class 0, on its whole 2048-point grid, and of class 1, then two independent waves of work.
+// The whole-grid march has registers that a windowed one of 16 rows a lane does not: there
+// every LDS read of the step loop went through one buffer (0.81 instead of 0.58 us a step).
 __global__ __attribute__((amdgpu_flat_work_group_size(128, 128), amdgpu_waves_per_eu(2, 2)))
-void fd1d_window_big(FdBatch b, const int* counts, const uint32_t* list) {
+void fd1d_windowed_big(FdBatch b, const int* rec, int* counts, const uint32_t* list, uint32_t* later) {
     __shared__ double qp[2 * 128 * 17];
     __shared__ double xchg[4];
-    int base = 0;
-    for (int i = 0; i < kWindowBig; ++i) base += counts[i];
-    b.m = counts[kWindowBig];
+    const int slot = blockIdx.x, whole = counts[0], both = whole + counts[1];
+    if (slot >= both) {
+        const int w = threadIdx.x >> 6;
+        run_wave(b, 2 * (slot - both) + w, rec, counts, list, later, qp + w * (2 * 64 * 16));
+        return;
+    }
+    if (slot >= whole && !solve_window<10, 64, 2>(b, list, rec, 0, slot, both, qp, xchg)) return;
+    b.m = both;
+    b.order = list;
+    solve_group_f64<16, 64, 2, false>(b, slot, qp, xchg);
+}
+
+// The PDEs left for later, on their whole grids. Their count is final by now: the launch that
+// adds to it has ended.
+__global__ __attribute__((amdgpu_flat_work_group_size(128, 128), amdgpu_waves_per_eu(2, 2)))
+void fd1d_window_again(FdBatch b, const int* counts, const uint32_t* later) {
+    __shared__ double qp[2 * 128 * 17];
+    __shared__ double xchg[4];
+    b.m = counts[kAgain];
     if ((int)blockIdx.x >= b.m) return;
-    b.order = list + base;
+    b.order = later;
     solve_group_f64<16, 64, 2, false>(b, blockIdx.x, qp, xchg);
 }

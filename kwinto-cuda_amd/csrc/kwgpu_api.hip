@@ -190,6 +190,13 @@ bool windowed_fits(int cap, int precision, double theta) {
     return cap >= 256 && cap <= 2048 && precision == KWGPU_FP64 && theta == 0.5;
 }
 
+// ... but not for a uniform batch of short marches, whose windows are their whole grids, nor
+// for few PDEs of over 1024 points: some window then needs the two-wave march anyway, and the
+// batch takes its time (600 at 2048 x 512: 393 us windowed, 387 us not; 1500: 426 and 747).
+bool uniform_windowed(size_t m, int x_dim, int t_dim) {
+    return t_dim - 1 >= kwgpu::kWindowMinSteps && (x_dim <= 1024 || m > kwgpu::kLoneMax / 2);
+}
+
 Choice choice_for(const kwgpu_ctx* c, int cap, int precision, int layout, double theta) {
     Choice ch;
     if (cap == kLaneCap) return ch;  // lane layout
@@ -414,15 +421,11 @@ int run_fd_on(kwgpu_ctx* c, FdBatch b, const int32_t* pde_x, const int32_t* pde_
         const int cap = bucket_of(b.x_dim, precision, layout);
         Choice ch = choice_for(c, cap, precision, layout, theta);
         if (ch.variant == kWindowed) {
-            const bool lone = b.m <= kwgpu::kLoneMax && b.x_dim <= 1024;
-            if (b.t_dim - 1 >= kwgpu::kWindowMinSteps && lone) {
-                if (hipError_t e = kwgpu::launch_fd1d_lone(b, s); e != hipSuccess)
-                    return hip_fail(c, e, "kwgpu: windowed kernel launch");
-                return KWGPU_OK;
-            }
-            if (b.t_dim - 1 >= kwgpu::kWindowMinSteps && !capturing(s)) {
+            const bool scratch = b.m > kwgpu::kLoneMax || b.x_dim > 1024;
+            if (uniform_windowed(b.m, b.x_dim, b.t_dim) && !(scratch && capturing(s))) {
                 const int big = b.x_dim > 1024 ? b.m : 0;
-                if (int rc = ensure_window(c, b.m, b.m, big)) return rc;
+                if (scratch)
+                    if (int rc = ensure_window(c, b.m, b.m, big)) return rc;
                 if (hipError_t e = kwgpu::launch_fd1d_windowed(b, window_scratch(c), big, s))
                     return hip_fail(c, e, "kwgpu: windowed kernel launch");
                 return KWGPU_OK;
@@ -1145,7 +1148,7 @@ int kwgpu_fd1d_price_device_noalloc(kwgpu_ctx* c, const kwgpu_option* d_opts, si
     if (!hx && !ht) {
         const int cap = bucket_of(p->x_dim, p->precision, p->layout);
         Choice ch = choice_for(c, cap, p->precision, p->layout, p->theta);
-        if (ch.variant == kWindowed && p->t_dim - 1 < kwgpu::kWindowMinSteps)
+        if (ch.variant == kWindowed && !uniform_windowed(n, p->x_dim, p->t_dim))
             ch = Choice{kwgpu::default_wave_variant(cap), true};
         plan.push_back(Bucket{cap, ch, 0, n, p->x_dim, p->precision, p->x_dim > 1024 ? (int)n : 0});
     } else {

@@ -202,7 +202,8 @@ hipError_t launch_fd1d_wave_variant(const FdBatch& b, int variant, int precision
 bool wave_layout_fits(int x_dim, int precision);
 // FP64 at theta 1/2 on each PDE's window of rows (fd1d_window.h), x_dim <= 2048. Device
 // scratch of the caller: a record per PDE number (all that b.order may name), a list of
-// b.m + n_big entries and kWindowCounters counters. n_big: how many of the b.m PDEs have over
+// b.m + n_big entries and kWindowCounters counters (none with at most kLoneMax PDEs and n_big
+// = 0). n_big: how many of the b.m PDEs have over
 // 1024 x-points.
 constexpr int kWindowCounters = 32;
 struct WindowScratch {
@@ -210,8 +211,7 @@ struct WindowScratch {
     uint32_t* list;
     int* counts;
 };
-hipError_t launch_fd1d_windowed(const FdBatch& b, const WindowScratch& w, int n_big,
-                                hipStream_t s);
+hipError_t launch_fd1d_windowed(const FdBatch& b, const WindowScratch& w, int n_big, hipStream_t s);
 // The same for at most kLoneMax PDEs, x_dim <= 1024, without scratch: one PDE a wave.
 constexpr int kLoneMax = 2048;
 hipError_t launch_fd1d_lone(const FdBatch& b, hipStream_t s);
