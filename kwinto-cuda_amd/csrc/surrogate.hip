@@ -27,6 +27,7 @@
 #include <random>
 #include <string>
 #include <thread>
+#include <type_traits>
 #include <vector>
 
 #include "kwgpu_internal.h"
@@ -45,13 +46,8 @@ constexpr int kW1 = 0, kB1 = kW1 + H * F, kW2 = kB1 + H, kB2 = kW2 + H * H, kW3 
               kB3 = kW3 + H * H, kW4 = kB3 + H, kB4 = kW4 + H * H, kW5 = kB4 + H, kB5 = kW5 + H,
               kP = kB5 + 1;
 static_assert(kP == KWGPU_SURROGATE_PARAMS, "parameter layout");
-// partial-sum slots of the column reductions: at most kPartRows row blocks, each
-// at most kPartWidth sums (the layer-1 block W1 | b1), per member
-constexpr int kPartRows = 128, kPartWidth = H * F + H;
-// ... and of the weight-gradient GEMMs' K splits (at most kMaxSplits slots of H x H)
-constexpr int kMaxSplits = 32;
-constexpr size_t kPartFloats = std::max<size_t>((size_t)kPartRows * kPartWidth,
-                                                (size_t)kMaxSplits * H * H);
+// row blocks of the column sums, and splits of the weight gradients' rows, at most
+constexpr int kPartRows = 128, kMaxSplits = 32;
 // Target: y = (premium - base) / (base + kEps K), the part of the FD pricer's premium
 // that the control variate (base, the premium from the exercise boundary below) misses,
 // relative to it (floored at kEps K). A network error dy then costs (base + kEps K) dy in
@@ -579,13 +575,6 @@ __device__ inline double euro_bs(kwgpu_option o) {
     return bs_one(o);
 }
 
-__device__ __forceinline__ float sigm(float z) { return 1.0f / (1.0f + __expf(-z)); }
-__device__ __forceinline__ float silu(float z) { return z * sigm(z); }
-__device__ __forceinline__ float dsilu(float z) {
-    const float s = sigm(z);
-    return s * (1.0f + z * (1.0f - s));
-}
-
 // ---- data ------------------------------------------------------------------------
 // Grid of row i: per-row sizes when given, else the uniform ones.
 struct GridArg {
@@ -610,20 +599,6 @@ __global__ void features_kernel(const kwgpu_option* opts, size_t n, GridArg g, c
         target[i] = (float)((premium[i] - base) / (base + kEps * o.k));
     }
     if (in_box) in_box[i] = in ? 1 : 0;
-}
-
-// Member-batched kernels: the pointer arguments are the first member's; member k's
-// data follows at the given element strides, k = blockIdx.y (blockIdx.z for 2-D grids).
-
-// batch rows of member k: its permutation idx + k * sidx picks the samples
-__global__ void gather_kernel(const float* feat, const float* target, const uint32_t* idx,
-                              long sidx, int n, float* bfeat, float* btarget, long srow) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const int k = blockIdx.y;
-    const uint32_t s = idx[k * sidx + i];
-    for (int f = 0; f < F; ++f) bfeat[k * srow * F + i * F + f] = feat[(size_t)s * F + f];
-    btarget[k * srow + i] = target[s];
 }
 
 // Labels at nodes: option i gives node options a_i (row i) and b_i (row n + i) with the
@@ -733,496 +708,145 @@ __global__ void baseline_kernel(const kwgpu_option* opts, size_t n, double* out)
     if (i < n) out[i] = baseline_premium(opts[i]);
 }
 
-// ---- layers ----------------------------------------------------------------------
-// input layer in FP32: Z1 = x W1^T + b1, H1 = silu(Z1) in BF16
-__global__ void l1_fwd(const float* x, long sx, const float* p, int n, float* Z, bf16* Hb,
-                       long sz) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n * H) return;
-    const int k = blockIdx.y;
-    x += k * sx;
-    p += (long)k * kP;
-    Hb += k * sz;
-    const int m = i / H, j = i - m * H;
-    float z = p[kB1 + j];
-#pragma unroll
-    for (int f = 0; f < F; ++f) z = fmaf(p[kW1 + j * F + f], x[m * F + f], z);
-    if (Z) Z[k * sz + i] = z;  // prediction keeps no pre-activations
-    Hb[i] = (bf16)silu(z);
-}
-
-enum { EPI_FWD = 0, EPI_BWD = 1, EPI_WGRAD = 2 };
-
-struct GemmArgs {
-    const bf16* A;  // A(m, k) = A[m * sam + k * sak]
-    long sam, sak;
-    const bf16* B;  // B(k, n) = B[k * sbk + n * sbn]
-    long sbk, sbn;
-    int M, N, K;
-    const float* bias;  // EPI_FWD: bias[n]
-    float* Z;           // EPI_FWD: writes pre-activations (unless null); EPI_BWD: reads them
-    bf16* Hout;         // EPI_FWD: silu(Z); EPI_BWD: dZ = C * silu'(Z)
-    float* C;           // EPI_WGRAD: C[z][m * N + n] = sum over this block's K range, one
-                        // M x N slot per blockIdx.z (member, split), summed afterwards
-    int k_split;        // EPI_WGRAD: K range per split
-    int splits;         // EPI_WGRAD: K splits; blockIdx.z = member * splits + split
-    long mA, mB, mBias, mZ, mH;  // member strides (elements)
-};
-
-// C(M x N) = A(M x K) B(K x N), 64 x 64 tile per 256-thread workgroup, each wave a
-// 32 x 32 quarter as 2 x 2 MFMA 16x16x32 tiles; K in steps of BK through LDS.
-template <int EPI, int BK>
-__global__ __launch_bounds__(256) void gemm_bf16(GemmArgs g) {
-    constexpr int BM = 64, BN = 64, LD = BK + 8;
-    static_assert(BK % 32 == 0 && (EPI != EPI_WGRAD || BK == 32),
-                  "k staged in 32-wide chunks; the transposing loader stages 32");
-    __shared__ __attribute__((aligned(16))) bf16 As[BM * LD];
-    __shared__ __attribute__((aligned(16))) bf16 Bs[BN * LD];
-    const int t = threadIdx.x, w = t >> 6, l = t & 63;
-    const int m0 = blockIdx.y * BM, n0 = blockIdx.x * BN;
-    int kb = 0, ke = g.K;
-    const int mem = EPI == EPI_WGRAD ? blockIdx.z / g.splits : blockIdx.z;
-    if constexpr (EPI == EPI_WGRAD) {
-        kb = (blockIdx.z - mem * g.splits) * g.k_split;
-        ke = min(g.K, kb + g.k_split);
-    }
-    g.A += mem * g.mA;
-    g.B += mem * g.mB;
-    if constexpr (EPI == EPI_FWD) g.bias += mem * g.mBias;
-    if constexpr (EPI != EPI_WGRAD) {
-        if (g.Z) g.Z += mem * g.mZ;
-        g.Hout += mem * g.mH;
-    } else {
-        g.C += (long)blockIdx.z * g.M * g.N;
-    }
-    const int wm = (w >> 1) * 32, wn = (w & 1) * 32;
-    floatx4 acc[2][2];
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-        for (int j = 0; j < 2; ++j) acc[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
-    const int lr = t >> 2, lc = (t & 3) * 8;  // tile row 0..63, k offset 0/8/16/24
-    for (int k0 = kb; k0 < ke; k0 += BK) {
-        if constexpr (EPI == EPI_WGRAD) {
-            // both operands have K (the batch) across rows and M / N along them: load 16
-            // bytes along the row and transpose into the K-contiguous LDS tiles
-            const int kk = t >> 3, c8 = (t & 7) * 8;  // k row 0..31, column group 0..56
-            const int k = k0 + kk;
-            bf16x8 va, vb;
-            if (g.sam == 1 && g.sbn == 1 && k < ke && m0 + c8 + 8 <= g.M && n0 + c8 + 8 <= g.N) {
-                va = *reinterpret_cast<const bf16x8*>(g.A + (long)k * g.sak + m0 + c8);
-                vb = *reinterpret_cast<const bf16x8*>(g.B + (long)k * g.sbk + n0 + c8);
-            } else {
-#pragma unroll
-                for (int i = 0; i < 8; ++i) {
-                    const int m = m0 + c8 + i, n = n0 + c8 + i;
-                    va[i] = (k < ke && m < g.M) ? g.A[(long)m * g.sam + (long)k * g.sak] : (bf16)0.0f;
-                    vb[i] = (k < ke && n < g.N) ? g.B[(long)k * g.sbk + (long)n * g.sbn] : (bf16)0.0f;
-                }
-            }
-#pragma unroll
-            for (int i = 0; i < 8; ++i) {
-                As[(c8 + i) * LD + kk] = va[i];
-                Bs[(c8 + i) * LD + kk] = vb[i];
-            }
-        } else {
-            // BK / 32 chunks of 16 bytes per thread and operand, all loads issued before
-            // the first LDS store
-            constexpr int KC = BK / 32;
-            bf16x8 va[KC], vb[KC];
-#pragma unroll
-            for (int c = 0; c < KC; ++c) {
-                const int m = m0 + lr, n = n0 + lr, k = k0 + 32 * c + lc;
-                if (g.sak == 1 && m < g.M && k + 8 <= ke) {
-                    va[c] = *reinterpret_cast<const bf16x8*>(g.A + (long)m * g.sam + k);
-                } else {
-#pragma unroll
-                    for (int i = 0; i < 8; ++i)
-                        va[c][i] = (m < g.M && k + i < ke)
-                                       ? g.A[(long)m * g.sam + (long)(k + i) * g.sak]
-                                       : (bf16)0.0f;
-                }
-                if (g.sbk == 1 && n < g.N && k + 8 <= ke) {
-                    vb[c] = *reinterpret_cast<const bf16x8*>(g.B + (long)n * g.sbn + k);
-                } else {
-#pragma unroll
-                    for (int i = 0; i < 8; ++i)
-                        vb[c][i] = (n < g.N && k + i < ke)
-                                       ? g.B[(long)(k + i) * g.sbk + (long)n * g.sbn]
-                                       : (bf16)0.0f;
-                }
-            }
-#pragma unroll
-            for (int c = 0; c < KC; ++c) {
-                *reinterpret_cast<bf16x8*>(&As[lr * LD + 32 * c + lc]) = va[c];
-                *reinterpret_cast<bf16x8*>(&Bs[lr * LD + 32 * c + lc]) = vb[c];
-            }
-        }
-        __syncthreads();
-#pragma unroll
-        for (int kk = 0; kk < BK; kk += 32)
-#pragma unroll
-            for (int i = 0; i < 2; ++i) {
-                const bf16x8 a = *reinterpret_cast<const bf16x8*>(
-                    &As[(wm + 16 * i + (l & 15)) * LD + kk + 8 * (l >> 4)]);
-#pragma unroll
-                for (int j = 0; j < 2; ++j) {
-                    const bf16x8 b = *reinterpret_cast<const bf16x8*>(
-                        &Bs[(wn + 16 * j + (l & 15)) * LD + kk + 8 * (l >> 4)]);
-                    acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, acc[i][j], 0, 0, 0);
-                }
-            }
-        __syncthreads();
-    }
-    // D layout of v_mfma_f32_16x16x32: lane l, element e -> row 4 (l / 16) + e, col l % 16
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-        for (int j = 0; j < 2; ++j)
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                const int m = m0 + wm + 16 * i + 4 * (l >> 4) + e;
-                const int n = n0 + wn + 16 * j + (l & 15);
-                if (m >= g.M || n >= g.N) continue;
-                const float v = acc[i][j][e];
-                const long o = (long)m * g.N + n;
-                if constexpr (EPI == EPI_FWD) {
-                    const float z = v + g.bias[n];
-                    if (g.Z) g.Z[o] = z;
-                    g.Hout[o] = (bf16)silu(z);
-                } else if constexpr (EPI == EPI_BWD) {
-                    g.Hout[o] = (bf16)(v * dsilu(g.Z[o]));
-                } else {
-                    g.C[o] = v;
-                }
-            }
-}
-
-// output layer: y = silu(Z4) W5 + b5; with targets also dy = 2 (y - t) / n and the loss
-// sum. kOutSPW samples per wave; the loss is reduced in the block before one atomic.
-constexpr int kOutSPW = 8;
-__global__ __launch_bounds__(256) void out_fwd(const float* Z4, long sz, const float* p, int n,
-                                               const float* target, float* y, long sy, float* dy,
-                                               long srow, float* loss_sum) {
-    __shared__ float part[4];
-    const int wave = threadIdx.x >> 6, l = threadIdx.x & 63;
-    {
-        const int k = blockIdx.y;
-        Z4 += k * sz;
-        p += (long)k * kP;
-        y += k * sy;
-        if (target) {
-            target += k * srow;
-            dy += k * srow;
-            loss_sum += k;
-        }
-    }
-    const int m0 = (blockIdx.x * 4 + wave) * kOutSPW;
-    float loss = 0.0f;
-    for (int k = 0; k < kOutSPW; ++k) {
-        const int m = m0 + k;
-        if (m >= n) break;  // uniform per wave
-        float s = 0.0f;
-#pragma unroll
-        for (int c = l; c < H; c += 64) s = fmaf(p[kW5 + c], silu(Z4[(long)m * H + c]), s);
-        for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o);
-        if (l == 0) {
-            const float v = s + p[kB5];
-            y[m] = v;
-            if (target) {
-                const float d = v - target[m];
-                dy[m] = 2.0f * d / (float)n;
-                loss += d * d;
-            }
-        }
-    }
-    if (l == 0) part[wave] = loss;
-    __syncthreads();
-    if (target && threadIdx.x == 0) atomicAdd(loss_sum, part[0] + part[1] + part[2] + part[3]);
-}
+// ---- training step ----------------------------------------------------------------
+#include "surrogate_step.h"
 
 // ---- prediction: the whole member MLP in one kernel ----------------------------------
-// kPredRows node rows of one member (blockIdx.y) per 256-thread workgroup. The input
+// kPredRows node rows of one member (blockIdx.x) per workgroup of eight waves. The input
 // layer (FP32) writes silu(Z1) in BF16 to LDS; each 256 x 256 layer then runs on MFMA
-// 16x16x32, wave w computing output columns 64w .. 64w + 63 of every row of the tile
-// with its weights W[n][k] read from L2; once every wave has read the layer's input,
-// bias and SiLU are applied to the accumulators and overwrite it in LDS. The output
-// layer is reduced from the last layer's accumulators. The arithmetic is forward()'s --
-// the same FP32 input layer, BF16 activations and weights, the same MFMA sequence over
-// k with FP32 accumulation, FP32 pre-activations of the last layer -- up to the order
-// of the output layer's FP32 sum, but no activation goes to HBM: prediction moved
-// 0.15 GB per 25k node rows of a 4-member ensemble through the separate kernels.
+// 16x16x32, wave w computing columns 32 w .. 32 w + 31 of every row of the tile with its
+// weights from L2; once every wave has read the layer's input, bias and SiLU are applied
+// to the accumulators and overwrite it in LDS. The output layer is reduced from the last
+// layer's accumulators. The arithmetic is the training step's -- the same FP32 input
+// layer, BF16 activations and weights, the same MFMA sequence over k with FP32
+// accumulation, FP32 pre-activations of the last layer -- up to the order of the output
+// layer's FP32 sum. One buffer of 128 rows (66 KB) and 128 registers: two workgroups per
+// CU, so that one's SiLU runs beside the other's MFMA. 23000 rows of four networks: 113 ->
+// 70 us with the weights in the fragments' order and the one-step division; bound by the
+// SiLU's VALU and transcendental instructions.
 constexpr int kPredRows = 128;
-constexpr int kPredLd = H + 8;  // LDS row pitch in BF16 elements: rows 16 bytes apart mod 128
 
-__global__ __attribute__((amdgpu_flat_work_group_size(256, 256), amdgpu_waves_per_eu(2, 2)))
+__global__ __attribute__((amdgpu_flat_work_group_size(512, 512), amdgpu_waves_per_eu(4, 4)))
 void mlp_predict(const float* __restrict__ x, const float* __restrict__ pall,
                  const bf16* __restrict__ wball, int n, float* __restrict__ yall, long sy) {
-    static_assert(H == 256 && kPredRows % 16 == 0, "four waves of 64 output columns");
     constexpr int RT = kPredRows / 16;  // 16-row MFMA tiles
-    __shared__ __attribute__((aligned(16))) bf16 act[kPredRows * kPredLd];
-    __shared__ float xs[kPredRows * F];
-    __shared__ float red[4][kPredRows];
+    static_assert(H == 256 && kPredRows * F == 2 * 512, "eight waves of 32 columns");
+    __shared__ __attribute__((aligned(16))) bf16 act[kPredRows * kStepLd];
+    __shared__ __attribute__((aligned(16))) float xs[kPredRows * F];
+    __shared__ float red[8][kPredRows];
     const int t = threadIdx.x, w = t >> 6, l = t & 63;
-    const int mem = blockIdx.y;
+    const int mem = blockIdx.x;
     const float* p = pall + (long)mem * kP;
-    const bf16* wb = wball + (long)mem * 3 * H * H;
-    const int r0 = blockIdx.x * kPredRows;
-    for (int i = t; i < kPredRows * F; i += 256)  // rows past n read as 0
+    constexpr int LW = H * H / 8;  // a layer's fragments
+    const bf16x8* W = reinterpret_cast<const bf16x8*>(wball) + (long)mem * 3 * LW +
+                      2 * w * (H / 32) * 64 + l;
+    const int c0 = 32 * w + 4 * (l >> 4), row = l & 15;  // columns c0 + 16 j + 0 .. 3, rows + 16 i
+    const int r0 = blockIdx.y * kPredRows;
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {  // rows past n read as 0
+        const int i = t + 512 * k;
         xs[i] = r0 + i / F < n ? x[(long)r0 * F + i] : 0.0f;
+    }
     __syncthreads();
-    {  // input layer, as l1_fwd: thread t computes hidden unit t of every row
-        float w1[F];
+    const auto put = [&](const float (&z)[4], int i, int j) {
+        float s[4];
+        sigm4(z, s);
+        bf16x4 h;
 #pragma unroll
-        for (int f = 0; f < F; ++f) w1[f] = p[kW1 + t * F + f];
-        const float b1 = p[kB1 + t];
-        for (int r = 0; r < kPredRows; ++r) {
-            float z = b1;
+        for (int e = 0; e < 4; ++e) h[e] = (bf16)(z[e] * s[e]);
+        *reinterpret_cast<bf16x4*>(act + (16 * i + row) * kStepLd + c0 + 16 * j) = h;
+    };
 #pragma unroll
-            for (int f = 0; f < F; ++f) z = fmaf(w1[f], xs[r * F + f], z);
-            act[r * kPredLd + t] = (bf16)silu(z);
+    for (int j = 0; j < 2; ++j) {  // input layer
+        float w1[4][F], b1[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const int c = c0 + 16 * j + e;
+            b1[e] = p[kB1 + c];
+#pragma unroll
+            for (int f = 0; f < F; ++f) w1[e][f] = p[kW1 + c * F + f];
+        }
+#pragma unroll
+        for (int i = 0; i < RT; ++i) {
+            const float* xr = xs + (16 * i + row) * F;
+            const floatx4 xa = *reinterpret_cast<const floatx4*>(xr);
+            const floatx4 xb = *reinterpret_cast<const floatx4*>(xr + 4);
+            float z[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                z[e] = b1[e];
+#pragma unroll
+                for (int f = 0; f < 4; ++f) z[e] = fmaf(w1[e][f], xa[f], z[e]);
+#pragma unroll
+                for (int f = 0; f < 4; ++f) z[e] = fmaf(w1[e][4 + f], xb[f], z[e]);
+            }
+            put(z, i, j);
         }
     }
     __syncthreads();
-    const int col = 64 * w + (l & 15);  // + 16 j: this lane's output columns
+#pragma unroll 1
     for (int layer = 0; layer < 3; ++layer) {
-        const bf16* W = wb + (long)layer * H * H;
-        floatx4 acc[RT][4];
+        floatx4 acc[RT][2];
+        floatx4u bias[2], w5[2];
+        wave_mma<RT>(acc, W + layer * LW, act, l);
 #pragma unroll
-        for (int i = 0; i < RT; ++i)
-#pragma unroll
-            for (int j = 0; j < 4; ++j) acc[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
-        // k in the 32-wide steps of gemm_bf16, so each accumulator sees the same MFMAs
-#pragma unroll 2
-        for (int k0 = 0; k0 < H; k0 += 32) {
-            bf16x8 b[4];
-#pragma unroll
-            for (int j = 0; j < 4; ++j)
-                b[j] = *reinterpret_cast<const bf16x8*>(W + (long)(col + 16 * j) * H + k0 +
-                                                        8 * (l >> 4));
-#pragma unroll
-            for (int i = 0; i < RT; ++i) {
-                const bf16x8 a = *reinterpret_cast<const bf16x8*>(
-                    &act[(16 * i + (l & 15)) * kPredLd + k0 + 8 * (l >> 4)]);
-#pragma unroll
-                for (int j = 0; j < 4; ++j)
-                    acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b[j], acc[i][j], 0, 0, 0);
-            }
-        }
-        __syncthreads();  // every wave has read this layer's input
-        const float* bias = p + kB2 + layer * (H * H + H);
-        // D layout of v_mfma_f32_16x16x32: lane l, element e -> row 4 (l / 16) + e, col l % 16
+        for (int j = 0; j < 2; ++j)
+            bias[j] = *reinterpret_cast<const floatx4u*>(p + kB2 + layer * (H * H + H) + c0 + 16 * j);
         if (layer < 2) {
+            __syncthreads();  // every wave has read this layer's input
 #pragma unroll
             for (int i = 0; i < RT; ++i)
 #pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    const float bj = bias[col + 16 * j];
+                for (int j = 0; j < 2; ++j) {
+                    float z[4];
 #pragma unroll
-                    for (int e = 0; e < 4; ++e)
-                        act[(16 * i + 4 * (l >> 4) + e) * kPredLd + col + 16 * j] =
-                            (bf16)silu(acc[i][j][e] + bj);
+                    for (int e = 0; e < 4; ++e) z[e] = acc[i][j][e] + bias[j][e];
+                    put(z, i, j);
                 }
             __syncthreads();
         } else {
-            // output layer: y = b5 + sum_c W5[c] silu(Z4[c]); this lane's four columns,
-            // then the 16 lanes of a row group, then the four waves
-            float w5[4], bj[4];
+            // output layer: y = b5 + sum_c W5[c] silu(Z4[c]); this lane's eight columns,
+            // then the wave's 32, then the eight waves
 #pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                w5[j] = p[kW5 + col + 16 * j];
-                bj[j] = bias[col + 16 * j];
-            }
+            for (int j = 0; j < 2; ++j)
+                w5[j] = *reinterpret_cast<const floatx4u*>(p + kW5 + c0 + 16 * j);
 #pragma unroll
-            for (int i = 0; i < RT; ++i)
+            for (int i = 0; i < RT; ++i) {
+                float y = 0.0f;
 #pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    float s = 0.0f;
+                for (int j = 0; j < 2; ++j) {
+                    float z[4], s[4];
 #pragma unroll
-                    for (int j = 0; j < 4; ++j) s = fmaf(w5[j], silu(acc[i][j][e] + bj[j]), s);
+                    for (int e = 0; e < 4; ++e) z[e] = acc[i][j][e] + bias[j][e];
+                    sigm4(z, s);
 #pragma unroll
-                    for (int o = 1; o < 16; o <<= 1) s += __shfl_xor(s, o);
-                    if ((l & 15) == 0) red[w][16 * i + 4 * (l >> 4) + e] = s;
+                    for (int e = 0; e < 4; ++e) y = fmaf(w5[j][e], z[e] * s[e], y);
                 }
+                y += __shfl_xor(y, 16);
+                y += __shfl_xor(y, 32);
+                if (l < 16) red[w][16 * i + l] = y;
+            }
             __syncthreads();
             if (t < kPredRows && r0 + t < n)
-                yall[mem * sy + r0 + t] = p[kB5] + ((red[0][t] + red[1][t]) + (red[2][t] + red[3][t]));
+                yall[mem * sy + r0 + t] =
+                    p[kB5] + (((red[0][t] + red[1][t]) + (red[2][t] + red[3][t])) +
+                              ((red[4][t] + red[5][t]) + (red[6][t] + red[7][t])));
         }
     }
 }
 
-// dZ4 = dy W5 silu'(Z4) (BF16 for the next GEMMs)
-__global__ void out_bwd(const float* Z4, long sz, const float* p, const float* dy, long srow, int n,
-                        bf16* dZ, long sdz) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n * H) return;
-    const int mem = blockIdx.y;
-    Z4 += mem * sz;
-    p += (long)mem * kP;
-    dy += mem * srow;
-    dZ += mem * sdz;
-    const int m = i / H, c = i - m * H;
-    dZ[i] = (bf16)(dy[m] * p[kW5 + c] * dsilu(Z4[i]));
-}
-
-// grad[kB? + n] += sum_m dZ[m][n]   and, for the output layer,
-// grad[kW5 + n] += sum_m dy[m] silu(Z4[m][n]), grad[kB5] += sum_m dy[m]
-// The column reductions below: 256 threads = 64 columns x 4 row phases; the four
-// phases are summed in LDS, and each block stores one partial sum per column into its
-// own slot of `part` (added up by sum_parts).
-__device__ __forceinline__ float phase_sum(float v, float* lds) {
-    lds[threadIdx.x] = v;
-    __syncthreads();
-    const int c = threadIdx.x & 63;
-    return lds[c] + lds[64 + c] + lds[128 + c] + lds[192 + c];
-}
-__global__ __launch_bounds__(256) void colsum_bf16(const bf16* dZ, long sdz, int n, float* part) {
-    __shared__ float lds[256];
-    dZ += blockIdx.z * sdz;
-    part += ((long)blockIdx.z * gridDim.y + blockIdx.y) * H;  // this block's column sums
-    const int col = blockIdx.x * 64 + (threadIdx.x & 63);
-    const int r0 = blockIdx.y * 4 + (threadIdx.x >> 6);
-    float s = 0.0f;
-#pragma unroll 4
-    for (int m = r0; m < n; m += 4 * gridDim.y) s += (float)dZ[(long)m * H + col];
-    s = phase_sum(s, lds);
-    if (threadIdx.x < 64) part[col] = s;
-}
-__global__ __launch_bounds__(256) void out_grad(const float* Z4, long sz, const float* dy,
-                                                long srow, int n, float* part) {
-    __shared__ float lds[256];
-    Z4 += blockIdx.z * sz;
-    dy += blockIdx.z * srow;
-    part += ((long)blockIdx.z * gridDim.y + blockIdx.y) * (H + 1);  // this block's W5 | b5 sums
-    const int col = blockIdx.x * 64 + (threadIdx.x & 63);
-    const int r0 = blockIdx.y * 4 + (threadIdx.x >> 6);
-    float s = 0.0f, sb = 0.0f;
-    for (int m = r0; m < n; m += 4 * gridDim.y) {
-        s = fmaf(dy[m], silu(Z4[(long)m * H + col]), s);
-        if (col == 0) sb += dy[m];
-    }
-    s = phase_sum(s, lds);
-    __syncthreads();
-    sb = phase_sum(sb, lds);
-    if (threadIdx.x < 64) {
-        part[col] = s;
-        if (col == 0) part[H] = sb;
-    }
-}
-// input layer gradients: grad W1[j][f] += sum_m dZ1[m][j] x[m][f], b1[j] += sum_m dZ1[m][j]
-// Layer-1 gradient: seven sums per hidden column (six W1 weights and the bias). Each
-// lane owns four adjacent columns, so a wave reads one whole 512-byte dZ1 row per
-// iteration and the row's six inputs once (wave-uniform); the four waves' partial sums
-// meet in LDS and each block stores its 1792 sums into its own slot of `part`.
-typedef bf16 bf16x4 __attribute__((ext_vector_type(4)));
-__global__ __launch_bounds__(256) void l1_grad(const bf16* dZ1, long sdz, const float* x, long sx,
-                                               int n, float* part) {
-    static_assert(H == 256, "one wave covers a row as 64 lanes x 4 columns");
-    constexpr int V = 4 * (F + 1);
-    __shared__ float lds[V * 256];
-    dZ1 += blockIdx.y * sdz;
-    x += blockIdx.y * sx;
-    part += ((long)blockIdx.y * gridDim.x + blockIdx.x) * (H * F + H);  // W1 | b1 order
-    const int lane = threadIdx.x & 63;
-    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    float s[V] = {};
-    // U rows per wave per pass, all loads issued before any use (one wave per SIMD
-    // here, so the loads' latency is hidden only by having several in flight)
-    constexpr int U = 8;
-    const int stride = 4 * gridDim.x;
-    for (int m0 = blockIdx.x * 4 + w; m0 < n; m0 += U * stride) {
-        bf16x4 d4[U];
-        float xf[U][F];
-#pragma unroll
-        for (int u = 0; u < U; ++u) {
-            // rows past the end load the last row (no branch around the loads) and
-            // contribute d = 0
-            const int m = m0 + u * stride;
-            const int mc = min(m, n - 1);
-            const bf16x4 v = *(const bf16x4*)(dZ1 + (long)mc * H + 4 * lane);
-            d4[u] = m < n ? v : bf16x4{};
-#pragma unroll
-            for (int f = 0; f < F; ++f) xf[u][f] = x[mc * F + f];
-        }
-#pragma unroll
-        for (int u = 0; u < U; ++u)
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                const float d = (float)d4[u][j];
-#pragma unroll
-                for (int f = 0; f < F; ++f) s[j * (F + 1) + f] = fmaf(d, xf[u][f], s[j * (F + 1) + f]);
-                s[j * (F + 1) + F] += d;
-            }
-    }
-#pragma unroll
-    for (int v = 0; v < V; ++v) lds[v * 256 + threadIdx.x] = s[v];
-    __syncthreads();
-    for (int o = threadIdx.x; o < V * 64; o += 256) {
-        const int v = o >> 6, l = o & 63;
-        const float t = lds[v * 256 + l] + lds[v * 256 + 64 + l] + lds[v * 256 + 128 + l] +
-                        lds[v * 256 + 192 + l];
-        const int col = 4 * l + v / (F + 1), f = v % (F + 1);
-        part[f < F ? col * F + f : H * F + col] = t;
-    }
-}
-
-// grad[member][offset + o] += sum over the nb blocks' partial sums part[member][b][o]: the
-// second stage of the column reductions above. Many blocks adding into the same few
-// hundred addresses with device-scope atomics serialise on them; this reads each
-// partial once, coalesced.
-// 64 outputs per 256-thread block: the four waves take every fourth partial, 4 loads in
-// flight each, and meet in LDS.
-__global__ __launch_bounds__(256) void sum_parts(const float* part, int nb, int width,
-                                                 float* grad, int offset) {
-    __shared__ float lds[256];
-    const int o = blockIdx.x * 64 + (threadIdx.x & 63), ph = threadIdx.x >> 6;
-    const int oc = min(o, width - 1);  // lanes past the end load a valid slot, write nothing
-    part += (long)blockIdx.y * nb * width + oc;
-    float s0 = 0.0f, s1 = 0.0f, s2 = 0.0f, s3 = 0.0f;
-    int b = ph;
-    for (; b + 12 < nb; b += 16) {
-        s0 += part[(long)b * width];
-        s1 += part[(long)(b + 4) * width];
-        s2 += part[(long)(b + 8) * width];
-        s3 += part[(long)(b + 12) * width];
-    }
-    for (; b < nb; b += 4) s0 += part[(long)b * width];
-    const float t = phase_sum((s0 + s1) + (s2 + s3), lds);
-    if (threadIdx.x < 64 && o < width) grad[(long)blockIdx.y * kP + offset + o] += t;
-}
-
-__global__ void adam_kernel(float* p, const float* g, float* m1, float* m2, int np, float lr,
-                            float b1, float b2, float eps, float c1, float c2) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= np) return;
-    const long o = (long)blockIdx.y * kP;  // member
-    p += o;
-    g += o;
-    m1 += o;
-    m2 += o;
-    const float gi = g[i];
-    const float a = b1 * m1[i] + (1.0f - b1) * gi;
-    const float v = b2 * m2[i] + (1.0f - b2) * gi * gi;
-    m1[i] = a;
-    m2[i] = v;
-    p[i] -= lr * (a / c1) / (sqrtf(v / c2) + eps);
-}
-
-// BF16 copies of W2..W4 and of their transposes: blockIdx.y = 3 * member + layer
-// (one 16 x 16 tile per 256-thread block; the transpose goes through LDS so that both
-// copies are written in 32-byte row segments)
+// BF16 copies of W2..W4 and of their transposes in the fragments' order: blockIdx.y = 3 *
+// member + layer, one 16 x 16 tile per 256-thread block (a training step makes them in
+// step_update)
 __global__ __launch_bounds__(256) void to_bf16(const float* p, bf16* w, bf16* wT) {
     static_assert(H % 16 == 0, "16 x 16 tiles");
-    __shared__ bf16 tile[16][17];
     const int t = threadIdx.x, tr = blockIdx.x / (H / 16), tc = blockIdx.x % (H / 16);
     const int k = blockIdx.y / 3, l = blockIdx.y - 3 * k;
     const long o = (long)k * 3 * H * H + (long)l * H * H;
     const int r = tr * 16 + (t >> 4), c = tc * 16 + (t & 15);
     const bf16 v = (bf16)p[(long)k * kP + kW2 + l * (H * H + H) + r * H + c];
-    w[o + r * H + c] = v;
-    tile[t >> 4][t & 15] = v;
-    __syncthreads();
-    wT[o + (long)(tc * 16 + (t >> 4)) * H + tr * 16 + (t & 15)] = tile[t & 15][t >> 4];  // WT[c][r]
+    w[o + frag_at(r, c)] = v;
+    wT[o + frag_at(c, r)] = v;
 }
 
 __global__ void zero_f(float* p, size_t n) {
@@ -1463,15 +1087,14 @@ struct kwgpu_surrogate {
     float *grad = nullptr, *m1 = nullptr, *m2 = nullptr, *loss = nullptr;  // per member
     // per-member scratch slots of `cap` rows each (grown on demand)
     size_t cap = 0;
-    float *x = nullptr, *tg = nullptr, *y = nullptr, *dy = nullptr, *Z = nullptr;
-    bf16 *Hb = nullptr, *dZa = nullptr, *dZb = nullptr;
-    uint32_t* idx = nullptr;
+    float *x = nullptr, *tg = nullptr;
+    bf16* act = nullptr;  // kPlanes planes per member
+    // a step's partial sums: weight gradients per split, the column sums per row block
+    float *part_w = nullptr, *part_b = nullptr, *part_o = nullptr, *part_1 = nullptr;
     float* yall = nullptr;  // prediction: the members' outputs, 2 rows per option
     size_t yall_cap = 0;
     float* xp = nullptr;    // prediction: node features, 2 rows per option
     size_t xp_cap = 0;
-    float* part = nullptr;  // per-block partial sums of the column reductions (kPartRows
-                            // blocks x kPartWidth per member)
     void* serve = nullptr;  // kwgpu_surrogate_price's per-option buffers (grown on demand)
     size_t serve_cap = 0;   // options they hold
     // the FD configuration the network emulates (set by kwgpu_surrogate_fit; by default
@@ -1520,147 +1143,102 @@ GridArg grid_arg(const kwgpu_surrogate* s, const kwgpu_fd1d_params* fd) {
 }
 
 void free_scratch(kwgpu_surrogate* s) {
-    for (void* q : {(void*)s->x, (void*)s->tg, (void*)s->y, (void*)s->dy, (void*)s->Z,
-                    (void*)s->Hb, (void*)s->dZa, (void*)s->dZb, (void*)s->idx})
+    for (void* q : {(void*)s->x, (void*)s->tg, (void*)s->act, (void*)s->part_w, (void*)s->part_b,
+                    (void*)s->part_o, (void*)s->part_1})
         if (q) (void)hipFree(q);
-    s->x = s->tg = s->y = s->dy = s->Z = nullptr;
-    s->Hb = s->dZa = s->dZb = nullptr;
-    s->idx = nullptr;
+    s->x = s->tg = s->part_w = s->part_b = s->part_o = s->part_1 = nullptr;
+    s->act = nullptr;
     s->cap = 0;
 }
 
-// batch scratch, one slot of `rows` samples per member: x, targets, y, dy, Z and H for 4
-// layers, two dZ buffers
+// batch scratch, one slot of `rows` samples per member: x, targets, the BF16 planes, and
+// the partial sums of a step of so many rows (their block counts do not fall with the rows)
 hipError_t ensure_scratch(kwgpu_surrogate* s, size_t rows) {
     if (s->cap >= rows) return hipSuccess;
     free_scratch(s);
     const size_t M = (size_t)s->members;
+    const int n = (int)rows;
     hipError_t e;
     if ((e = hipMalloc(&s->x, M * rows * F * sizeof(float))) ||
         (e = hipMalloc(&s->tg, M * rows * sizeof(float))) ||
-        (e = hipMalloc(&s->y, M * rows * sizeof(float))) ||
-        (e = hipMalloc(&s->dy, M * rows * sizeof(float))) ||
-        (e = hipMalloc(&s->Z, M * 4 * rows * H * sizeof(float))) ||
-        (e = hipMalloc(&s->Hb, M * 4 * rows * H * sizeof(bf16))) ||
-        (e = hipMalloc(&s->dZa, M * rows * H * sizeof(bf16))) ||
-        (e = hipMalloc(&s->dZb, M * rows * H * sizeof(bf16))) ||
-        (e = hipMalloc(&s->idx, rows * sizeof(uint32_t))))
+        (e = hipMalloc(&s->act, M * kPlanes * rows * H * sizeof(bf16))) ||
+        (e = hipMalloc(&s->part_w, M * 3 * wgrad_splits(n) * H * H * sizeof(float))) ||
+        (e = hipMalloc(&s->part_b, M * 3 * sum_blocks(n) * H * sizeof(float))) ||
+        (e = hipMalloc(&s->part_o, M * sum_blocks(n) * (H + 1) * sizeof(float))) ||
+        (e = hipMalloc(&s->part_1, M * l1_blocks(n) * (H * F + H) * sizeof(float)))) {
+        free_scratch(s);
         return e;
+    }
     s->cap = rows;
     return hipSuccess;
 }
 
-GemmArgs gemm_fwd(const bf16* Hin, const bf16* W, int n, const float* bias, float* Z, bf16* Hout) {
-    GemmArgs g{};
-    g.A = Hin; g.sam = H; g.sak = 1;        // H_{l-1}[m][k]
-    g.B = W; g.sbk = 1; g.sbn = H;          // W_l[n][k]
-    g.M = n; g.N = H; g.K = H;
-    g.bias = bias; g.Z = Z; g.Hout = Hout;
-    return g;
-}
-
-hipError_t launch_gemm(int epi, const GemmArgs& g, hipStream_t st, int z) {
-    dim3 grid(nblk(g.N, 64), nblk(g.M, 64), z);
-    // k in 32-wide stages: 64- and 128-wide stages (more loads in flight and MFMAs per
-    // barrier) raise the register count to 108 / 184 and measured slower (the layer
-    // GEMMs are bound by their FP32 pre-activation traffic, not by the operand loads)
-    if (epi == EPI_FWD)
-        hipLaunchKernelGGL((gemm_bf16<EPI_FWD, 32>), grid, dim3(256), 0, st, g);
-    else if (epi == EPI_BWD)
-        hipLaunchKernelGGL((gemm_bf16<EPI_BWD, 32>), grid, dim3(256), 0, st, g);
+// Partial gradients and losses (added to s->loss) of members m0 .. m0 + cnt - 1 over n rows:
+// row m is sample idx[k sidx + m] of feat and target (k: slot of the member), or sample m
+// itself, with feat = s->x, where idx is null.
+hipError_t gradients(kwgpu_surrogate* s, int m0, int cnt, int n, const float* feat,
+                     const float* target, const uint32_t* idx, long sidx, hipStream_t st) {
+    StepArgs a{};
+    a.feat = feat;
+    a.target = target;
+    a.idx = idx;
+    a.sidx = sidx;
+    a.n = n;
+    a.rs = sum_blocks(n);
+    a.p = s->p[m0];
+    a.wb = s->wb[m0];
+    a.wbT = s->wbT[m0];
+    a.x = idx ? s->x : nullptr;
+    a.srow = (long)s->cap;
+    a.act = s->act;
+    a.plane = (long)s->cap * H;
+    a.part_b = s->part_b;
+    a.part_o = s->part_o;
+    a.loss = s->loss;
+    // 16-row tiles of a block's rows, four or five a pass: five where that saves a pass
+    const int tiles = (n + 16 * a.rs - 1) / (16 * a.rs);
+    if ((tiles + 4) / 5 < (tiles + 3) / 4)
+        hipLaunchKernelGGL(step_rows<5>, dim3(cnt, a.rs), dim3(512), 0, st, a);
     else
-        hipLaunchKernelGGL((gemm_bf16<EPI_WGRAD, 32>), grid, dim3(256), 0, st, g);
+        hipLaunchKernelGGL(step_rows<4>, dim3(cnt, a.rs), dim3(512), 0, st, a);
+    if (hipError_t e = hipGetLastError()) return e;
+    WgradArgs w{};
+    w.act = s->act;
+    w.plane = a.plane;
+    w.n = n;
+    w.members = cnt;
+    w.splits = wgrad_splits(n);
+    w.k_split = ((n + w.splits - 1) / w.splits + 31) / 32 * 32;
+    w.l1 = l1_blocks(n);
+    w.x = s->x;
+    w.sx = (long)s->cap * F;
+    w.part_w = s->part_w;
+    w.part_1 = s->part_1;
+    hipLaunchKernelGGL(step_wgrad, dim3(cnt * (w.l1 + 4 * 3 * w.splits)), dim3(256), 0, st, w);
     return hipGetLastError();
 }
 
-// Forward of members m0 .. m0+cnt-1 (parameters), scratch slots 0 .. cnt-1, n rows each:
-// features from s->x (slot k, or slot 0 for every member when shared_x); y into
-// yout + k sy; with targets (s->tg) also dy and the loss sums s->loss[k].
-hipError_t forward(kwgpu_surrogate* s, int m0, int cnt, int n, bool shared_x, float* yout,
-                   long sy, bool with_targets, hipStream_t st) {
-    const float* p = s->p[m0];
-    const bf16* wb = s->wb[m0];
-    const long cap = (long)s->cap, sz = 4 * cap * H, sx = shared_x ? 0 : cap * F;
-    float* Z = s->Z;
-    bf16* Hb = s->Hb;
-    const size_t L = (size_t)n * H;
-    // without targets (prediction) no backward follows: only the last layer's FP32
-    // pre-activations, which the output layer reads, are stored
-    const bool keep = with_targets;
-    hipLaunchKernelGGL(l1_fwd, dim3(nblk(L, 256), cnt), dim3(256), 0, st, s->x, sx, p, n,
-                       keep ? Z : nullptr, Hb, sz);
-    for (int l = 0; l < 3; ++l) {
-        GemmArgs g = gemm_fwd(Hb + l * L, wb + l * H * H, n, p + kB2 + l * (H * H + H),
-                              keep || l == 2 ? Z + (l + 1) * L : nullptr, Hb + (l + 1) * L);
-        g.mA = sz;
-        g.mB = 3 * H * H;
-        g.mBias = kP;
-        g.mZ = sz;
-        g.mH = sz;
-        if (hipError_t e = launch_gemm(EPI_FWD, g, st, cnt)) return e;
-    }
-    hipLaunchKernelGGL(out_fwd, dim3(nblk(n, 4 * kOutSPW), cnt), dim3(256), 0, st, Z + 3 * L, sz, p,
-                       n, with_targets ? (const float*)s->tg : nullptr, yout, sy, s->dy, cap,
-                       s->loss);
-    return hipGetLastError();
-}
-
-// Backward after forward() for the same members; gradients into s->grad slots 0 .. cnt-1
-// (zeroed here).
-hipError_t backward(kwgpu_surrogate* s, int m0, int cnt, int n, hipStream_t st) {
-    const float* p = s->p[m0];
-    const bf16* wbT = s->wbT[m0];
-    const long cap = (long)s->cap, sz = 4 * cap * H, sx = cap * F, sdz = cap * H, srow = cap;
-    const size_t L = (size_t)n * H;
-    float* g = s->grad;
-    hipLaunchKernelGGL(zero_f, dim3(nblk((size_t)cnt * kP, 256)), dim3(256), 0, st, g,
-                       (size_t)cnt * kP);
-    // row splits of the column reductions: 16 rows per thread at the default batch
-    const int rs = std::max(1, std::min(kPartRows, n / 64));
-    hipLaunchKernelGGL(out_grad, dim3(H / 64, rs, cnt), dim3(256), 0, st, s->Z + 3 * L, sz, s->dy,
-                       srow, n, s->part);
-    hipLaunchKernelGGL(sum_parts, dim3(nblk(H + 1, 64), cnt), dim3(256), 0, st, s->part, rs, H + 1,
-                       g, kW5);
-    hipLaunchKernelGGL(out_bwd, dim3(nblk(L, 256), cnt), dim3(256), 0, st, s->Z + 3 * L, sz, p,
-                       s->dy, srow, n, s->dZa, sdz);
-    bf16* dz = s->dZa;
-    bf16* dzn = s->dZb;
-    for (int l = 2; l >= 0; --l) {  // hidden layer l+2: weights W_{l+2}, input H_{l+1}
-        const int splits = std::max(1, std::min(kMaxSplits, n / 512));
-        GemmArgs gw{};
-        gw.A = dz; gw.sam = 1; gw.sak = H;               // A(o, m) = dZ[m][o]
-        gw.B = s->Hb + l * L; gw.sbk = H; gw.sbn = 1;    // B(m, i) = H_{l+1}[m][i]
-        gw.M = H; gw.N = H; gw.K = n;
-        gw.C = s->part;  // one H x H slot per (member, split)
-        gw.k_split = ((n + splits - 1) / splits + 31) / 32 * 32;
-        gw.splits = splits;
-        gw.mA = sdz;
-        gw.mB = sz;
-        if (hipError_t e = launch_gemm(EPI_WGRAD, gw, st, cnt * splits)) return e;
-        hipLaunchKernelGGL(sum_parts, dim3(nblk(H * H, 64), cnt), dim3(256), 0, st, s->part,
-                           splits, H * H, g, kW2 + l * (H * H + H));
-        hipLaunchKernelGGL(colsum_bf16, dim3(H / 64, rs, cnt), dim3(256), 0, st, dz, sdz, n,
-                           s->part);
-        hipLaunchKernelGGL(sum_parts, dim3(nblk(H, 64), cnt), dim3(256), 0, st, s->part, rs, H, g,
-                           kB2 + l * (H * H + H));
-        GemmArgs gb{};
-        gb.A = dz; gb.sam = H; gb.sak = 1;                     // A(m, o) = dZ[m][o]
-        gb.B = wbT + l * H * H; gb.sbk = 1; gb.sbn = H;       // B(o, i) = W[o][i] = WT[i][o]
-        gb.M = n; gb.N = H; gb.K = H;
-        gb.Z = s->Z + l * L;                                   // pre-activations of H_{l+1}
-        gb.Hout = dzn;
-        gb.mA = sdz;
-        gb.mB = 3 * H * H;
-        gb.mZ = sz;
-        gb.mH = sdz;
-        if (hipError_t e = launch_gemm(EPI_BWD, gb, st, cnt)) return e;
-        std::swap(dz, dzn);
-    }
-    const int rs1 = std::max(1, std::min(64, n / 128));
-    static_assert(64 <= kPartRows, "partial slots");
-    hipLaunchKernelGGL(l1_grad, dim3(rs1, cnt), dim3(256), 0, st, dz, sdz, s->x, sx, n, s->part);
-    hipLaunchKernelGGL(sum_parts, dim3(nblk(kPartWidth, 64), cnt), dim3(256), 0, st, s->part, rs1,
-                       kPartWidth, g, kW1);
+// The gradients' sums after gradients() over n rows: Adam on the members' parameters, or
+// (adam null) to s->grad.
+hipError_t update(kwgpu_surrogate* s, int cnt, int n, const UpdateArgs* adam, hipStream_t st) {
+    UpdateArgs u = adam ? *adam : UpdateArgs{};
+    u.part_w = s->part_w;
+    u.part_b = s->part_b;
+    u.part_o = s->part_o;
+    u.part_1 = s->part_1;
+    u.splits = wgrad_splits(n);
+    u.rs = sum_blocks(n);
+    u.l1 = l1_blocks(n);
+    u.p = s->pall;
+    u.m1 = s->m1;
+    u.m2 = s->m2;
+    u.grad = s->grad;
+    u.wb = s->wball;
+    u.wbT = s->wballT;
+    if (adam)
+        hipLaunchKernelGGL(step_update<true>, dim3(kUpdateBlks, cnt), dim3(256), 0, st, u);
+    else
+        hipLaunchKernelGGL(step_update<false>, dim3(kUpdateBlks, cnt), dim3(256), 0, st, u);
     return hipGetLastError();
 }
 
@@ -1721,7 +1299,6 @@ int kwgpu_surrogate_create(kwgpu_ctx* ctx, int32_t members, uint64_t seed, kwgpu
     if (hipMalloc(&s->pall, M * kP * sizeof(float)) ||
         hipMalloc(&s->wball, M * 3 * H * H * sizeof(bf16)) ||
         hipMalloc(&s->wballT, M * 3 * H * H * sizeof(bf16)) ||
-        hipMalloc(&s->part, M * kPartFloats * sizeof(float)) ||
         hipMalloc(&s->grad, M * kP * sizeof(float)) || hipMalloc(&s->m1, M * kP * sizeof(float)) ||
         hipMalloc(&s->m2, M * kP * sizeof(float)) || hipMalloc(&s->loss, M * sizeof(float))) {
         kwgpu_surrogate_destroy(s);
@@ -1752,7 +1329,7 @@ void kwgpu_surrogate_destroy(kwgpu_surrogate* s) {
     free_scratch(s);
     for (void* q : {(void*)s->pall, (void*)s->wball, (void*)s->wballT, (void*)s->grad,
                     (void*)s->m1, (void*)s->m2,
-                    (void*)s->loss, (void*)s->yall, (void*)s->xp, (void*)s->part, s->serve})
+                    (void*)s->loss, (void*)s->yall, (void*)s->xp, s->serve})
         if (q) (void)hipFree(q);
     if (s->ev_done) (void)hipEventDestroy(s->ev_done);
     delete s;
@@ -1822,8 +1399,8 @@ int kwgpu_surrogate_loss_grad(kwgpu_ctx* ctx, kwgpu_surrogate* s, int32_t member
     HIPCHK(hipMemcpy(s->x, host_x, n * F * sizeof(float), hipMemcpyHostToDevice));
     HIPCHK(hipMemcpy(s->tg, host_t, n * sizeof(float), hipMemcpyHostToDevice));
     hipLaunchKernelGGL(zero_f, dim3(1), dim3(64), 0, st, s->loss, (size_t)1);
-    HIPCHK(forward(s, member, 1, (int)n, false, s->y, (long)s->cap, true, st));
-    HIPCHK(backward(s, member, 1, (int)n, st));
+    HIPCHK(gradients(s, member, 1, (int)n, s->x, s->tg, nullptr, 0, st));
+    HIPCHK(update(s, 1, (int)n, nullptr, st));
     HIPCHK(hipStreamSynchronize(st));
     float l = 0;
     HIPCHK(hipMemcpy(&l, s->loss, sizeof(float), hipMemcpyDeviceToHost));
@@ -1892,7 +1469,6 @@ int train_rows(kwgpu_ctx* ctx, kwgpu_surrogate* s, const kwgpu_option* d_opts,
     };
     const size_t steps_per_epoch = nr / B;  // drop the ragged tail
     const double total = (double)steps_per_epoch * tp->epochs;
-    const long cap = (long)s->cap;
     hipLaunchKernelGGL(zero_f, dim3(nblk((size_t)M * kP, 256)), dim3(256), 0, st, s->m1,
                        (size_t)M * kP);
     hipLaunchKernelGGL(zero_f, dim3(nblk((size_t)M * kP, 256)), dim3(256), 0, st, s->m2,
@@ -1912,19 +1488,20 @@ int train_rows(kwgpu_ctx* ctx, kwgpu_surrogate* s, const kwgpu_option* d_opts,
         if (ep + 1 < tp->epochs) next = std::thread(draw, hperm[(ep + 1) & 1]);
         hipLaunchKernelGGL(zero_f, dim3(1), dim3(64), 0, st, s->loss, (size_t)M);
         for (size_t b = 0; b < steps_per_epoch; ++b, ++step) {
-            hipLaunchKernelGGL(gather_kernel, dim3(nblk(B, 256), M), dim3(256), 0, st, feat, tgt,
-                               didx + b * B, (long)nr, B, s->x, s->tg, cap);
-            hipError_t e = forward(s, 0, M, B, false, s->y, cap, true, st);
-            if (!e) e = backward(s, 0, M, B, st);
+            hipError_t e = gradients(s, 0, M, B, feat, tgt, didx + b * B, (long)nr, st);
             const double frac = step / total;
             const float lr = (float)(tp->lr_final + 0.5 * (tp->lr - tp->lr_final) *
                                                          (1.0 + std::cos(M_PI * frac)));
             const float c1 = 1.0f - std::pow(tp->beta1, (float)(step + 1));
             const float c2 = 1.0f - std::pow(tp->beta2, (float)(step + 1));
-            hipLaunchKernelGGL(adam_kernel, dim3(nblk(kP, 256), M), dim3(256), 0, st, s->pall,
-                               s->grad, s->m1, s->m2, kP, lr, tp->beta1, tp->beta2, tp->eps, c1,
-                               c2);
-            if (!e) e = refresh_bf16(s, 0, M, st);
+            UpdateArgs u{};
+            u.lr = lr;
+            u.b1 = tp->beta1;
+            u.b2 = tp->beta2;
+            u.eps = tp->eps;
+            u.c1 = c1;
+            u.c2 = c2;
+            if (!e) e = update(s, M, B, &u, st);
             if (e) {
                 rc = kwgpu::ctx_fail(ctx, KWGPU_ERR_HIP,
                                      std::string("train step: ") + hipGetErrorString(e));
@@ -2133,7 +1710,7 @@ int kwgpu_surrogate_predict(kwgpu_ctx* ctx, kwgpu_surrogate* s, const kwgpu_opti
                            d_opts + c0, cn, g, s->xp, d_in_box ? d_in_box + c0 : nullptr);
         // the whole ensemble at once on the shared features, one fused kernel per
         // 128-row tile and member
-        hipLaunchKernelGGL(mlp_predict, dim3(nblk(2 * cn, kPredRows), s->members), dim3(256), 0,
+        hipLaunchKernelGGL(mlp_predict, dim3(s->members, nblk(2 * cn, kPredRows)), dim3(512), 0,
                            st, s->xp, s->p[0], s->wb[0], (int)(2 * cn), s->yall, (long)(2 * cn));
         // kGroup lanes per candidate, which together solve its exercise boundary
         hipLaunchKernelGGL(node_combine_kernel, dim3(nblk(kGroup * cn, 64)), dim3(64), 0, st,
