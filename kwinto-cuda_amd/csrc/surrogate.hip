@@ -27,7 +27,6 @@
 #include <random>
 #include <string>
 #include <thread>
-#include <type_traits>
 #include <vector>
 
 #include "kwgpu_internal.h"
@@ -298,16 +297,15 @@ __host__ __device__ inline void boundary_fit(Boundary& bd, const double (&b)[kBn
     boundary_fit_log(bd, lb);
 }
 
-// Parameters, node times tau_i and the starting boundary b_i.
-__host__ __device__ inline void boundary_start(const kwgpu_option& o, Boundary& bd,
-                                               double (&b)[kBn + 1], double (&tau)[kBn + 1]) {
+// Parameters, and b_T / X for the starting boundary.
+__host__ __device__ inline double boundary_params(const kwgpu_option& o, Boundary& bd) {
     bd.call = !(o.w < 0);
     bd.r = bd.call ? o.q : o.r;
     bd.q = bd.call ? o.r : o.q;
     bd.z = o.z;
     bd.t = o.t;
     bd.none = !(o.k > 0 && o.t > 0 && o.z > 0) || !(bd.r > 0);
-    if (bd.none) return;
+    if (bd.none) return 0.0;
     bd.st = sqrt(o.t);
     bd.x0 = bd.q > 0 ? fmin(1.0, bd.r / bd.q) : 1.0;
     kwgpu_option u{};  // the unit-strike put, for b_T
@@ -319,13 +317,19 @@ __host__ __device__ inline void boundary_start(const kwgpu_option& o, Boundary& 
     u.s = 1.0;
     u.e = 1;
     u.w = -1;
-    const double bT = fmin(baseline_setup(u).ss, bd.x0);
-    for (int i = 0; i <= kBn; ++i) {
-        const double f = 0.5 * (1.0 - cos6(i));  // xi_i / sqrt T
-        tau[i] = o.t * f * f;
-        b[i] = bd.x0 * pow(bT / bd.x0, f);
-    }
-    b[0] = bd.x0;
+    return fmin(baseline_setup(u).ss, bd.x0) / bd.x0;
+}
+// Node i's time tau_i and starting boundary b_i.
+__host__ __device__ inline double boundary_node(const Boundary& bd, double ratio, int i, double& tau) {
+    const double f = 0.5 * (1.0 - cos6(i));  // xi_i / sqrt T
+    tau = bd.t * f * f;
+    return i == 0 ? bd.x0 : bd.x0 * pow(ratio, f);
+}
+__host__ __device__ inline void boundary_start(const kwgpu_option& o, Boundary& bd,
+                                               double (&b)[kBn + 1], double (&tau)[kBn + 1]) {
+    const double ratio = boundary_params(o, bd);
+    if (bd.none) return;
+    for (int i = 0; i <= kBn; ++i) b[i] = boundary_node(bd, ratio, i, tau[i]);
 }
 
 // One fixed-point step at node tau_i (b_i its current value), with bd fitted to the
@@ -467,16 +471,17 @@ __host__ __device__ inline double boundary_exercised(const Boundary& bd, double 
     const double eu = exp(-r * T) * phi_cdf(-dm) - x * exp(-q * T) * phi_cdf(-dm - sd);
     return kk * ((1.0 - x) - eu);
 }
-__host__ __device__ inline double boundary_integral(const Boundary& bd, double x, int k0, int kstep) {
+__host__ __device__ inline double boundary_term(const Boundary& bd, double x, int k) {
     const double r = bd.r, q = bd.q, sg = bd.z, T = bd.t;
     const double lx = log(x / bd.x0), c = r - q - 0.5 * sg * sg;
+    const double dt = T * ts_a(kTs - 1 - k);            // T - u
+    const double sd = sg * bd.st * ts_sa(kTs - 1 - k);  // sigma sqrt(T - u)
+    const double dm = (lx - boundary_lnb(bd, 1.0 - 2.0 * ts_sa(k)) + c * dt) / sd;
+    return r * exp(-r * dt) * phi_cdf(-dm) - q * x * exp(-q * dt) * phi_cdf(-dm - sd);
+}
+__host__ __device__ inline double boundary_integral(const Boundary& bd, double x, int k0, int kstep) {
     double p = 0.0;
-    for (int k = k0; k < kTs; k += kstep) {
-        const double dt = T * ts_a(kTs - 1 - k);            // T - u
-        const double sd = sg * bd.st * ts_sa(kTs - 1 - k);  // sigma sqrt(T - u)
-        const double dm = (lx - boundary_lnb(bd, 1.0 - 2.0 * ts_sa(k)) + c * dt) / sd;
-        p += ts_w(k) * (r * exp(-r * dt) * phi_cdf(-dm) - q * x * exp(-q * dt) * phi_cdf(-dm - sd));
-    }
+    for (int k = k0; k < kTs; k += kstep) p += ts_w(k) * boundary_term(bd, x, k);
     return p;
 }
 __host__ __device__ inline double boundary_at(const kwgpu_option& o, const Boundary& bd, double s) {
@@ -586,19 +591,83 @@ struct GridArg {
     __device__ int t(size_t i) const { return t_dims ? t_dims[i] : t_dim; }
 };
 
-__global__ void features_kernel(const kwgpu_option* opts, size_t n, GridArg g, const double* premium,
-                                float* feat, float* target, uint8_t* in_box) {
-    const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const kwgpu_option o = opts[i];
-    float f[F];
-    const bool in = option_features(o, g.x(i), g.t(i), f);
-    for (int k = 0; k < F; ++k) feat[i * F + k] = f[k];
-    if (target) {
-        const double base = boundary_premium(o);
+// Features and targets of training rows, six lanes to rows i and i + h, h = ceil(n / 2), and
+// ten such pairs a wave: lane j steps node 1 + j of the boundary's fixed point. A fit's rows
+// are the two nodes of each option, i and i + h, which differ in spot only and so share the
+// boundary; where the parameters differ, the second is solved on its own. Every sum is
+// boundary_setup's and boundary_at's, term by term (a target's last bit reaches the trained
+// weights), so the points of the last integral, shared out over the lanes, are added in order
+// by each. Bound by the FP64 issue of erfc: 32768 rows in 673 us with a lane a row (one wave
+// for every other SIMD), 380 us with six lanes a row, 219 us so.
+constexpr int kRowLanes = kBn, kPairsPerWave = 64 / kRowLanes;
+__global__ __launch_bounds__(64) void features_kernel(const kwgpu_option* opts, size_t n, GridArg g,
+                                                      const double* premium, float* feat,
+                                                      float* target) {
+    __shared__ double er[kTs][64], eq[kTs][64];  // e^{r u}, e^{q u} at this lane's points
+    const int l = threadIdx.x, j = l % kRowLanes, l0 = l - j;
+    const size_t h = (n + 1) / 2, i0 = (size_t)blockIdx.x * kPairsPerWave + l / kRowLanes;
+    if (l >= kPairsPerWave * kRowLanes || i0 >= h) return;  // a row's lanes go together from here
+    Boundary bd{};
+    kwgpu_option first{};
+#pragma unroll 1
+    for (size_t i = i0; i < n; i += h) {
+        const kwgpu_option o = opts[i];
+        const bool same = i != i0 && o.t == first.t && o.z == first.z && o.r == first.r &&
+                          o.q == first.q && (o.w < 0) == (first.w < 0) && o.k > 0 && first.k > 0;
+        if (!same) {
+            first = o;
+            const double ratio = boundary_params(o, bd);
+            if (!bd.none) {
+                double lb[kBn + 1] = {}, ti;
+                double bi = boundary_node(bd, ratio, j + 1, ti);
+#pragma unroll 1
+                for (int k = 0; k < kTs; ++k) {
+                    const double u1 = ti * ts_a(k);
+                    er[k][l] = exp(bd.r * u1);
+                    eq[k][l] = exp(bd.q * u1);
+                }
+#pragma unroll 1
+                for (int it = 0; it <= kBit; ++it) {
+                    const double lbi = log(bi / bd.x0);
+#pragma unroll
+                    for (int k = 1; k <= kBn; ++k) lb[k] = __shfl(lbi, l0 + k - 1);
+                    boundary_fit_log(bd, lb);
+                    if (it == kBit) break;
+                    const NodeStep nd = node_step(bd, ti, lbi);
+                    double ni = 0.0, di = 0.0;
+#pragma unroll 1
+                    for (int k = 0; k < kTs; ++k)
+                        boundary_point(bd, nd, k, er[k][l], eq[k][l], ni, di);
+                    bi = boundary_next(bd, ti, bi, ni, di);
+                }
+            }
+        }
+        double base = 0.0;
+        if (!bd.none && o.s > 0) {
+            double kk, x;
+            boundary_spot(o, bd, o.s, kk, x);
+            if (x <= boundary_bT(bd)) {
+                base = boundary_exercised(bd, kk, x);
+            } else {
+                double p = 0.0;
+#pragma unroll 1
+                for (int k0 = 0; k0 < kTs; k0 += kRowLanes) {
+                    const double v = boundary_term(bd, x, min(k0 + j, kTs - 1));
+#pragma unroll
+                    for (int m = 0; m < kRowLanes; ++m) {
+                        const double vm = __shfl(v, l0 + m);
+                        if (k0 + m < kTs) p += ts_w(k0 + m) * vm;
+                    }
+                }
+                base = kk * bd.t * p;
+            }
+        }
+        if (j != 0) continue;
+        float f[F];
+        option_features(o, g.x(i), g.t(i), f);
+        for (int k = 0; k < F; ++k) feat[i * F + k] = f[k];
         target[i] = (float)((premium[i] - base) / (base + kEps * o.k));
     }
-    if (in_box) in_box[i] = in ? 1 : 0;
 }
 
 // Labels at nodes: option i gives node options a_i (row i) and b_i (row n + i) with the
@@ -1089,7 +1158,7 @@ struct kwgpu_surrogate {
     size_t cap = 0;
     float *x = nullptr, *tg = nullptr;
     bf16* act = nullptr;  // kPlanes planes per member
-    // a step's partial sums: weight gradients per split, the column sums per row block
+    // a step's partial sums: weight gradients in four phases, the column sums per row block
     float *part_w = nullptr, *part_b = nullptr, *part_o = nullptr, *part_1 = nullptr;
     float* yall = nullptr;  // prediction: the members' outputs, 2 rows per option
     size_t yall_cap = 0;
@@ -1162,7 +1231,7 @@ hipError_t ensure_scratch(kwgpu_surrogate* s, size_t rows) {
     if ((e = hipMalloc(&s->x, M * rows * F * sizeof(float))) ||
         (e = hipMalloc(&s->tg, M * rows * sizeof(float))) ||
         (e = hipMalloc(&s->act, M * kPlanes * rows * H * sizeof(bf16))) ||
-        (e = hipMalloc(&s->part_w, M * 3 * wgrad_splits(n) * H * H * sizeof(float))) ||
+        (e = hipMalloc(&s->part_w, M * 3 * 4 * H * H * sizeof(float))) ||
         (e = hipMalloc(&s->part_b, M * 3 * sum_blocks(n) * H * sizeof(float))) ||
         (e = hipMalloc(&s->part_o, M * sum_blocks(n) * (H + 1) * sizeof(float))) ||
         (e = hipMalloc(&s->part_1, M * l1_blocks(n) * (H * F + H) * sizeof(float)))) {
@@ -1214,7 +1283,7 @@ hipError_t gradients(kwgpu_surrogate* s, int m0, int cnt, int n, const float* fe
     w.sx = (long)s->cap * F;
     w.part_w = s->part_w;
     w.part_1 = s->part_1;
-    hipLaunchKernelGGL(step_wgrad, dim3(cnt * (w.l1 + 4 * 3 * w.splits)), dim3(256), 0, st, w);
+    hipLaunchKernelGGL(step_wgrad, dim3(cnt * (w.l1 + kWgradTiles * 3 * std::min(4, w.splits))), dim3(256), 0, st, w);
     return hipGetLastError();
 }
 
@@ -1451,8 +1520,8 @@ int train_rows(kwgpu_ctx* ctx, kwgpu_surrogate* s, const kwgpu_option* d_opts,
         cleanup();
         return kwgpu::ctx_fail(ctx, KWGPU_ERR_NOMEM, "kwgpu_surrogate_train: allocation");
     }
-    hipLaunchKernelGGL(features_kernel, dim3(nblk(n, 256)), dim3(256), 0, st, d_opts, n, g,
-                       d_premium, feat, tgt, (uint8_t*)nullptr);
+    hipLaunchKernelGGL(features_kernel, dim3(nblk((n + 1) / 2, kPairsPerWave)), dim3(64), 0, st, d_opts, n, g,
+                       d_premium, feat, tgt);
     // every member steps at once (one launch per layer for the whole ensemble), each on
     // its own shuffle of the rows
     std::vector<std::mt19937_64> rng;

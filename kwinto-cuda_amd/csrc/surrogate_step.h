@@ -12,10 +12,11 @@
 //
 // Four networks, 8192 rows each, one step: 444 us as 25 launches (the FP32 pre-activations of
 // four layers written and read twice, an FP32 exponential and division per activation and
-// direction), 134 us as these three (72, 43 and 19 us); a training step's products take 16 us
+// direction), 113 us as these three (61, 38 and 14 us); a training step's products take 16 us
 // at the dense BF16 rate.
 
 typedef bf16 bf16x4 __attribute__((ext_vector_type(4)));
+typedef bf16 bf16x2 __attribute__((ext_vector_type(2)));
 typedef short shortx4 __attribute__((ext_vector_type(4)));
 // four floats at any float's address (a member's parameters start at a multiple of kP floats,
 // which is odd)
@@ -38,6 +39,13 @@ __device__ __forceinline__ void sigm4(const float (&z)[4], float (&s)[4]) {
 #pragma unroll
         for (int e = 0; e < 4; ++e) s[e] = 1.0f / x[e];
     }
+}
+
+// v of the lane N below in its row of 16, around the row.
+template <int N>
+__device__ __forceinline__ float row_ror(float v) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v),
+                                                                 0x120 + N, 0xf, 0xf, true));
 }
 
 // The BF16 weights are held in the order in which MFMA 16x16x32 takes them, so that a wave's
@@ -148,16 +156,20 @@ __device__ __forceinline__ void wave_mma(floatx4 (&acc)[RT][2], const bf16x8* W,
 // every row, with the weights as the A operand: a lane then holds four adjacent columns of a
 // row. The derivative of SiLU is kept in registers (3 x 8 RT) from the forward pass, so each
 // activation costs one exponential. To memory go the rows' H1..H3 and dZ1..dZ4 in BF16 (the
-// weight gradients read them), 117 MB for four networks of 8192 rows, instead of 0.6 GB.
+// weight gradients read them), 117 MB for four networks of 8192 rows, instead of 0.6 GB. The
+// 512 workgroups of that batch run in two rounds of 65000 cycles: SiLU's VALU and the MFMA of
+// the two waves of a SIMD take 40000 of them, the rows' gather and the barriers the rest.
 template <int RT>
 __global__ __attribute__((amdgpu_flat_work_group_size(512, 512), amdgpu_waves_per_eu(2, 2)))
 void step_rows(StepArgs g) {
     constexpr int R = 16 * RT;
-    static_assert(H == 256 && R / 8 <= 16, "eight waves of 32 columns and R / 8 rows");
+    static_assert(H == 256 && R <= 32 * 16, "eight waves of 32 columns; 16 passes of 32 rows");
     static_assert(kZ4Ld * sizeof(float) >= kStepLd * sizeof(bf16), "the buffers' union");
     __shared__ __attribute__((aligned(16))) bf16 act0[R * kStepLd];
     __shared__ __attribute__((aligned(16))) float z4[R * kZ4Ld];
     __shared__ __attribute__((aligned(16))) float xs[R * F];
+    __shared__ __attribute__((aligned(16))) float ws[H * F + H];  // W1 | b1
+    __shared__ __attribute__((aligned(16))) float bs[4][H];  // b2, b3, b4 and W5
     __shared__ float tg[R], sdy[R], lred[8];
     bf16* const act1 = reinterpret_cast<bf16*>(z4);
     const int t = threadIdx.x, w = t >> 6, l = t & 63;
@@ -172,15 +184,16 @@ void step_rows(StepArgs g) {
     const auto batch_row = [&](int r, int j0) { return 4 * by + (r & 3) + stride * (j0 + (r >> 2)); };
     // rows of the tile in buffer b to plane q of act, 16 bytes a lane
     const auto copy_out = [&](const bf16* b, int q, int j0) {
-        bf16* out = g.act + ((long)mem * kPlanes + q) * g.plane;
         const int m = batch_row(t >> 5, j0);
-        out += (long)m * H + 8 * (t & 31);
+        bf16* out = g.act + ((long)mem * kPlanes + q) * g.plane + (long)m * H + 8 * (t & 31);
         b += (t >> 5) * kStepLd + 8 * (t & 31);
+        bf16x8 v[RT];
+#pragma unroll
+        for (int i = 0; i < RT; ++i) v[i] = *reinterpret_cast<const bf16x8*>(b + 16 * i * kStepLd);
 #pragma unroll
         for (int i = 0; i < RT; ++i)
             if (m + 4 * i * stride < g.n)
-                *reinterpret_cast<bf16x8*>(out + (long)(4 * i * stride) * H) =
-                    *reinterpret_cast<const bf16x8*>(b + 16 * i * kStepLd);
+                *reinterpret_cast<bf16x8*>(out + (long)(4 * i * stride) * H) = v[i];
     };
     for (int j0 = 0; batch_row(0, j0) < g.n; j0 += 4 * RT) {
         // the parameters' addresses, made new in each pass: kept over the loop, what is loaded
@@ -194,6 +207,7 @@ void step_rows(StepArgs g) {
         // rows of this phase in the tile
         const int m0 = batch_row(ph, j0);
         const int nq = m0 < g.n ? min(4 * RT, (g.n - m0 + stride - 1) / stride) : 0;
+        // the rows first: their indices and then their features take a memory latency each
         if (t < R) {
             const int m = batch_row(t, j0);
             floatx4 xa = {0.f, 0.f, 0.f, 0.f}, xb = xa;
@@ -212,9 +226,17 @@ void step_rows(StepArgs g) {
             *reinterpret_cast<floatx4*>(xs + t * F) = xa;
             *reinterpret_cast<floatx4*>(xs + t * F + 4) = xb;
             tg[t] = y;
+        } else {
+            // W1 | b1, then b2, b3, b4 and W5
+            for (int c = t - R; c < kB1 + H; c += 512 - R) ws[c] = p[c];
+            for (int c = t - R; c < 4 * H; c += 512 - R) {
+                const int k = c / H;
+                bs[k][c % H] = p[(k < 3 ? kB2 + k * (H * H + H) : kW5) + c % H];
+            }
         }
         WeightFrags wf;
         load_frags(wf, W);
+        const float b5 = p[kB5];
         __syncthreads();
         floatx4 acc[RT][2];
         float d1[RT][2][4], d2[RT][2][4], d3[RT][2][4];  // SiLU' of layers 1 .. 3
@@ -233,19 +255,12 @@ void step_rows(StepArgs g) {
         };
 #pragma unroll
         for (int j = 0; j < 2; ++j) {  // input layer, FP32
-            float w1[4][F], b1[4];
+            floatx4 w1[4][2], b1 = *reinterpret_cast<const floatx4*>(ws + kB1 + c0 + 16 * j);
 #pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                const int c = c0 + 16 * j + e;
-                const floatx4u wa = *reinterpret_cast<const floatx4u*>(p + kW1 + c * F);
-                const floatx4u wc = *reinterpret_cast<const floatx4u*>(p + kW1 + c * F + 4);
-                b1[e] = p[kB1 + c];
+            for (int e = 0; e < 4; ++e)
 #pragma unroll
-                for (int f = 0; f < 4; ++f) {
-                    w1[e][f] = wa[f];
-                    w1[e][4 + f] = wc[f];
-                }
-            }
+                for (int f = 0; f < 2; ++f)
+                    w1[e][f] = *reinterpret_cast<const floatx4*>(ws + (c0 + 16 * j + e) * F + 4 * f);
 #pragma unroll
             for (int i = 0; i < RT; ++i) {
                 const float* xr = xs + (16 * i + row) * F;
@@ -256,23 +271,23 @@ void step_rows(StepArgs g) {
                 for (int e = 0; e < 4; ++e) {
                     z[e] = b1[e];
 #pragma unroll
-                    for (int f = 0; f < 4; ++f) z[e] = fmaf(w1[e][f], xa[f], z[e]);
+                    for (int f = 0; f < 4; ++f) z[e] = fmaf(w1[e][0][f], xa[f], z[e]);
 #pragma unroll
-                    for (int f = 0; f < 4; ++f) z[e] = fmaf(w1[e][4 + f], xb[f], z[e]);
+                    for (int f = 0; f < 4; ++f) z[e] = fmaf(w1[e][1][f], xb[f], z[e]);
                 }
                 activate(z, d1[i][j], act0, i, j);
             }
         }
         __syncthreads();
         // hidden layer `layer` (0 .. 2) from buffer in: its sums in acc, biases in bias
-        floatx4u bias[2];
+        floatx4 bias[2];
         const auto product = [&](int layer, const bf16* in) {
+            step_mma<RT>(acc, wf, W + layer * LW, in, l);
+            load_frags(wf, layer < 2 ? W + (layer + 1) * LW : WT + 2 * LW);
+            copy_out(in, layer, j0);
 #pragma unroll
             for (int j = 0; j < 2; ++j)
-                bias[j] = *reinterpret_cast<const floatx4u*>(p + kB2 + layer * (H * H + H) + c0 + 16 * j);
-            step_mma<RT>(acc, wf, W + layer * LW, in, l);
-            copy_out(in, layer, j0);
-            load_frags(wf, layer < 2 ? W + (layer + 1) * LW : WT + 2 * LW);
+                bias[j] = *reinterpret_cast<const floatx4*>(&bs[layer][c0 + 16 * j]);
         };
         const auto hidden = [&](int layer, const bf16* in, bf16* out, float (&d)[RT][2][4]) {
             product(layer, in);
@@ -309,25 +324,33 @@ void step_rows(StepArgs g) {
                 *reinterpret_cast<floatx4*>(z4 + (16 * i + row) * kZ4Ld + c0 + 16 * j) = h;
             }
         __syncthreads();
-        {  // output layer and its error, a row at a time per wave
-            float w5[H / 64];
+        {  // output layer and its error: 16 lanes a row, four rows a wave at a time
+            const int c = l & 15;
+            float w5[H / 16];
 #pragma unroll
-            for (int q = 0; q < H / 64; ++q) w5[q] = p[kW5 + l + 64 * q];
-            const float b5 = p[kB5];
-            // rows w + 8 k, of which lane k keeps the k-th
-            float y = 0.0f;
+            for (int q = 0; q < H / 16; ++q) w5[q] = bs[3][c + 16 * q];
+            float y = 0.0f;  // lane c keeps row 32 c + 4 w + l / 16
 #pragma unroll
-            for (int k = 0; k < R / 8; ++k) {
-                const float* z = z4 + (w + 8 * k) * kZ4Ld + l;
-                float s = 0.0f;
+            for (int k = 0; k < RT / 2 + RT % 2; ++k) {
+                const int r = 32 * k + 4 * w + (l >> 4);
+                const float* z = z4 + min(r, R - 1) * kZ4Ld + c;
+                float s[4];  // columns c + 16 a, + 64, + 128, + 192
 #pragma unroll
-                for (int q = 0; q < H / 64; ++q) s = fmaf(w5[q], z[64 * q], s);
+                for (int a = 0; a < 4; ++a) {
+                    s[a] = 0.0f;
 #pragma unroll
-                for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o);
-                y = l == k ? s : y;
+                    for (int q = 0; q < H / 64; ++q)
+                        s[a] = fmaf(w5[a + 4 * q], z[16 * a + 64 * q], s[a]);
+                }
+                float v = (s[0] + s[2]) + (s[1] + s[3]);
+                v += row_ror<8>(v);
+                v += row_ror<4>(v);
+                v += row_ror<2>(v);
+                v += row_ror<1>(v);
+                y = c == k ? v : y;
             }
-            const int r = w + 8 * l;
-            if (l < R / 8) {
+            const int r = 32 * c + 4 * w + (l >> 4);
+            if (r < R) {
                 const float d = y + b5 - tg[r];
                 const bool in = batch_row(r, j0) < g.n;
                 sdy[r] = in ? 2.0f * d / (float)g.n : 0.0f;
@@ -335,20 +358,25 @@ void step_rows(StepArgs g) {
             }
         }
         __syncthreads();
-#pragma unroll 4
-        for (int q = 0; q < nq; ++q) {  // gradient of W5 and b5
+        const auto out_grad = [&](int q) {  // gradient of W5 and b5
             const int r = 4 * q + ph;
             const float dy = sdy[r];
             const float2 h = *reinterpret_cast<const float2*>(z4 + r * kZ4Ld + 2 * cp);
             so[0] = fmaf(dy, h.x, so[0]);
             so[1] = fmaf(dy, h.y, so[1]);
             sb5 += dy;
+        };
+        if (nq >= 16) {
+#pragma unroll
+            for (int q = 0; q < 16; ++q) out_grad(q);
+            for (int q = 16; q < nq; ++q) out_grad(q);
+        } else {
+            for (int q = 0; q < nq; ++q) out_grad(q);
         }
         {
-            floatx4u w5[2];
+            floatx4 w5[2];
 #pragma unroll
-            for (int j = 0; j < 2; ++j)
-                w5[j] = *reinterpret_cast<const floatx4u*>(p + kW5 + c0 + 16 * j);
+            for (int j = 0; j < 2; ++j) w5[j] = *reinterpret_cast<const floatx4*>(&bs[3][c0 + 16 * j]);
 #pragma unroll
             for (int i = 0; i < RT; ++i) {
                 const float dy = sdy[16 * i + row];
@@ -366,13 +394,25 @@ void step_rows(StepArgs g) {
         // layer below to buffer out
         const auto back = [&](int layer, const bf16* in, bf16* out, const float (&d)[RT][2][4]) {
             step_mma<RT>(acc, wf, WT + layer * LW, in, l);
-            copy_out(in, kPlaneDZ + 1 + layer, j0);
             if (layer > 0) load_frags(wf, WT + (layer - 1) * LW);
-#pragma unroll 4
-            for (int q = 0; q < nq; ++q) {
-                const bf16* v = in + (4 * q + ph) * kStepLd + 2 * cp;
-                sb[layer][0] += (float)v[0];
-                sb[layer][1] += (float)v[1];
+            const bf16* v = in + ph * kStepLd + 2 * cp;
+            const auto at = [&](int q) {
+                return *reinterpret_cast<const bf16x2*>(v + 4 * q * kStepLd);
+            };
+            const auto add = [&](bf16x2 x) {
+                sb[layer][0] += (float)x[0];
+                sb[layer][1] += (float)x[1];
+            };
+            copy_out(in, kPlaneDZ + 1 + layer, j0);
+            if (nq >= 16) {
+                bf16x2 x[16];
+#pragma unroll
+                for (int q = 0; q < 16; ++q) x[q] = at(q);
+#pragma unroll
+                for (int q = 0; q < 16; ++q) add(x[q]);
+                for (int q = 16; q < nq; ++q) add(at(q));
+            } else {
+                for (int q = 0; q < nq; ++q) add(at(q));
             }
 #pragma unroll
             for (int i = 0; i < RT; ++i)
@@ -399,7 +439,7 @@ void step_rows(StepArgs g) {
         z4[(12 + ph) * H + 2 * cp + e] = so[e];
     }
     if (cp == 0) sdy[ph] = sb5;
-    for (int o = 8; o > 0; o >>= 1) loss += __shfl_xor(loss, o);  // lanes 0 .. R / 8 - 1
+    for (int o = 32; o > 0; o >>= 1) loss += __shfl_xor(loss, o);
     if (l == 0) lred[w] = loss;
     __syncthreads();
     for (int o = t; o < 4 * H; o += 512) {
@@ -425,7 +465,7 @@ struct WgradArgs {
     int n, members, splits, k_split, l1;  // l1: blocks of the input layer's gradient per member
     const float* x;
     long sx;
-    float *part_w, *part_1;  // [member][layer][split][H H], [member][block][H F + H]
+    float *part_w, *part_1;  // [member][layer][phase][H H], [member][block][H F + H]
 };
 
 // Input layer gradients of one block: part W1[j][f] = sum_m dZ1[m][j] x[m][f], b1[j] = sum_m
@@ -482,102 +522,159 @@ __device__ __forceinline__ void l1_grad(const WgradArgs& g, int mem, int blk, fl
     }
 }
 
-// Weight gradients dW[o][i] = sum_m dZ[m][o] H[m][i] of a split's rows, a 128 x 128 tile per
-// workgroup and 64 x 64 per wave, all layers and members in one launch; the first l1 x
-// members workgroups take the input layer's. Both operands have the sum's index m across
-// rows: 32 rows x 128 columns of each are staged in LDS as they lie and read transposed
+// The splits of phase ph in the order of their sum (phase_chain below): chain 0 takes splits
+// ph, ph + 16 .. and the tail, chain c of 1 .. 3 takes ph + 4 c, ph + 4 c + 16 ..; within a
+// split, rows in steps of 32.
+struct SplitRows {
+    int ph, nb, m, n0, k_split, n;  // m splits a chain, n0 in chain 0
+    int q, chain, k0, ke;           // split number q of the phase: its chain, rows k0 .. ke
+    bool end;
+    __device__ SplitRows(int ph, int nb, int k_split, int n) : ph(ph), nb(nb), k_split(k_split), n(n) {
+        m = nb > ph + 12 ? (nb - ph - 12 + 15) / 16 : 0;
+        n0 = m + (nb - ph - 16 * m > 0 ? (nb - ph - 16 * m + 3) / 4 : 0);
+        q = -1;
+        split();
+    }
+    __device__ void split() {  // the next one that has rows
+        do {
+            ++q;
+            end = q >= n0 + 3 * m;
+            const int r = q - n0;
+            chain = r < 0 ? 0 : r < m ? 1 : r < 2 * m ? 2 : 3;
+            const int b = r >= 0 ? ph + 4 * chain + 16 * (r - (chain - 1) * m)
+                                 : q < m ? ph + 16 * q : ph + 16 * m + 4 * (q - m);
+            k0 = b * k_split;
+            ke = min(n, k0 + k_split);
+        } while (!end && k0 >= ke);
+    }
+    __device__ void next() {
+        k0 += 32;
+        if (k0 >= ke) split();
+    }
+};
+
+// Weight gradients dW[o][i] = sum_m dZ[m][o] H[m][i], summed over splits of consecutive rows
+// and those over phases: a workgroup takes the splits of one phase (split % 4) one after
+// another for a tile of 64 o x 128 i, 32 x 64 per wave, so that four partial sums go to memory
+// instead of one per split. All layers and members in one launch; the last l1 x members
+// workgroups take the input layer's gradient. Both operands have the sum's index m across
+// rows: 32 rows of each are staged in LDS as they lie and read transposed
 // (ds_read_b64_tr_b16: 16 lanes read 4 rows x 16 columns, lane c gets column c). Rows 8 g + r
 // and 8 g + 4 + r, r < 4, lie at LDS rows 4 g + r and 16 + 4 g + r, 32 bytes apart mod 256,
-// so that the 16 rows of one read spread over all banks.
-__global__ __launch_bounds__(256) void step_wgrad(WgradArgs g) {
-    constexpr int BK = 32, BT = 128, LD = BT + 16;
-    constexpr int kStage = 2 * BK * LD;  // BF16 values of one stage: dZ, then H
-    static_assert(2 * kStage * sizeof(bf16) >= kL1V * 256 * sizeof(float), "l1_grad's LDS");
-    __shared__ __attribute__((aligned(16))) bf16 lds[2 * kStage];
-    if ((int)blockIdx.x < g.l1 * g.members) {
-        l1_grad(g, blockIdx.x % g.members, blockIdx.x / g.members, reinterpret_cast<float*>(lds));
+// so that the 16 rows of one read spread over all banks. Bound by reading the activations
+// (117 MB at four networks of 8192 rows): 43 us
+// with a partial sum and a 128 x 128 tile per split, 38 us so, and step_update 19 -> 14 us.
+constexpr int kTileO = 64, kTileI = 128, kWgradTiles = (H / kTileO) * (H / kTileI);
+__global__ __attribute__((amdgpu_flat_work_group_size(256, 256), amdgpu_waves_per_eu(2, 2)))
+void step_wgrad(WgradArgs g) {
+    constexpr int BK = 32, LA = kTileO + 16, LB = kTileI + 16;  // LDS row pitches
+    constexpr int kStage = BK * (LA + LB);  // BF16 values of one stage: dZ, then H
+    constexpr int kLds = std::max<int>(2 * kStage * sizeof(bf16), kL1V * 256 * sizeof(float));
+    __shared__ __attribute__((aligned(16))) char raw[kLds];
+    const int phases = min(4, g.splits), units = 3 * g.members * phases;
+    const int id = blockIdx.x;
+    if (id >= kWgradTiles * units) {
+        const int b = id - kWgradTiles * units;
+        l1_grad(g, b % g.members, b / g.members, reinterpret_cast<float*>(raw));
         return;
     }
-    const int units = 3 * g.members * g.splits;
-    const int id = blockIdx.x - g.l1 * g.members;
-    // the four tiles of a unit, which share their rows, are `units` workgroups apart: on the
-    // same L2 where 8 divides that
+    bf16* const lds = reinterpret_cast<bf16*>(raw);
+    // the tiles of a unit, which share their rows, are `units` workgroups apart: on the same
+    // L2 where 8 divides that
     const int unit = id % units, tile = id / units;
-    const int mem = unit % g.members, layer = unit / g.members % 3, split = unit / g.members / 3;
-    const int o0 = (tile >> 1) * BT, i0 = (tile & 1) * BT;
-    const int kb = split * g.k_split, ke = min(g.n, kb + g.k_split);
-    const bf16* A = g.act + ((long)mem * kPlanes + kPlaneDZ + 1 + layer) * g.plane + o0;
-    const bf16* B = g.act + ((long)mem * kPlanes + layer) * g.plane + i0;
+    const int mem = unit % g.members, layer = unit / g.members % 3, ph = unit / g.members / 3;
+    const int o0 = tile / (H / kTileI) * kTileO, i0 = tile % (H / kTileI) * kTileI;
     const int t = threadIdx.x, w = t >> 6, l = t & 63;
-    floatx4 acc[4][4];
+    // staging: 16 bytes of a row of dZ (8 lanes a row) and of two rows of H (16 lanes a row)
+    const int ra = t >> 3, ca = 8 * (t & 7), rb = t >> 4, cb = 8 * (t & 15);
+    const bf16* A = g.act + ((long)mem * kPlanes + kPlaneDZ + 1 + layer) * g.plane + o0 + ca;
+    const bf16* B = g.act + ((long)mem * kPlanes + layer) * g.plane + i0 + cb;
+    struct Stage {
+        bf16x8 a, b[2];
+    };
+    const auto load = [&](Stage& v, const SplitRows& s) {
+        v.a = v.b[0] = v.b[1] = bf16x8{};
+        if (s.end) return;
+        if (s.k0 + ra < s.ke) v.a = *reinterpret_cast<const bf16x8*>(A + (long)(s.k0 + ra) * H);
 #pragma unroll
-    for (int a = 0; a < 4; ++a)
-#pragma unroll
-        for (int b = 0; b < 4; ++b) acc[a][b] = floatx4{0.f, 0.f, 0.f, 0.f};
-    // staging: 16 bytes of rows t / 16 and 16 + t / 16 of both operands
-    bf16x8 va[2], vb[2];
-    const auto load = [&](int k0) {
-#pragma unroll
-        for (int q = 0; q < 2; ++q) {
-            const int m = k0 + 16 * q + (t >> 4);
-            va[q] = vb[q] = bf16x8{};
-            if (m < ke) {
-                va[q] = *reinterpret_cast<const bf16x8*>(A + (long)m * H + 8 * (t & 15));
-                vb[q] = *reinterpret_cast<const bf16x8*>(B + (long)m * H + 8 * (t & 15));
-            }
-        }
+        for (int q = 0; q < 2; ++q)
+            if (s.k0 + 16 * q + rb < s.ke)
+                v.b[q] = *reinterpret_cast<const bf16x8*>(B + (long)(s.k0 + 16 * q + rb) * H);
     };
     const auto lds_row = [](int m) { return ((m >> 2) & 1) * 16 + (m >> 3) * 4 + (m & 3); };
-    const auto store = [&](bf16* s) {
+    const auto store = [&](const Stage& v, bf16* s) {
+        *reinterpret_cast<bf16x8*>(s + lds_row(ra) * LA + ca) = v.a;
 #pragma unroll
-        for (int q = 0; q < 2; ++q) {
-            const int r = lds_row(16 * q + (t >> 4));
-            *reinterpret_cast<bf16x8*>(s + r * LD + 8 * (t & 15)) = va[q];
-            *reinterpret_cast<bf16x8*>(s + BK * LD + r * LD + 8 * (t & 15)) = vb[q];
-        }
+        for (int q = 0; q < 2; ++q)
+            *reinterpret_cast<bf16x8*>(s + BK * LA + lds_row(16 * q + rb) * LB + cb) = v.b[q];
     };
     // a fragment: column c0 + l % 16, rows 8 (l / 16) .. + 7 of a stage
-    const auto frag = [&](const bf16* s, int c0) {
+    const auto frag = [&](const bf16* s, int ld, int c0) {
         typedef __attribute__((address_space(3))) shortx4 lds_s4;
-        const bf16* q = s + (l >> 2) * LD + c0 + 4 * (l & 3);
+        const bf16* q = s + (l >> 2) * ld + c0 + 4 * (l & 3);
         const shortx4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s4*)q);
-        const shortx4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s4*)(q + 16 * LD));
+        const shortx4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s4*)(q + 16 * ld));
         return __builtin_bit_cast(bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
     };
-    if (kb < ke) {
-        load(kb);
-        store(lds);
-        __syncthreads();
-        const int co = 64 * (w >> 1), ci = 64 * (w & 1);
-        int cur = 0;
-        for (int k0 = kb; k0 < ke; k0 += BK, cur ^= 1) {
-            const bool more = k0 + BK < ke;
-            if (more) load(k0 + BK);
-            const bf16* s = lds + cur * kStage;
-            bf16x8 fa[4], fb[4];
+    const int co = 32 * (w >> 1), ci = 64 * (w & 1);
+    floatx4 acc[2][4], sum[2][4], s01[2][4], s23[2][4];  // split, chain, chains 0 + 1, 2 + 3
+    const auto each = [&](auto f) {
 #pragma unroll
-            for (int a = 0; a < 4; ++a) fa[a] = frag(s, co + 16 * a);
+        for (int a = 0; a < 2; ++a)
 #pragma unroll
-            for (int b = 0; b < 4; ++b) fb[b] = frag(s + BK * LD, ci + 16 * b);
+            for (int b = 0; b < 4; ++b) f(a, b);
+    };
+    const floatx4 zero = {0.f, 0.f, 0.f, 0.f};
+    each([&](int a, int b) { acc[a][b] = sum[a][b] = s01[a][b] = s23[a][b] = zero; });
+    const auto product = [&](const bf16* s) {
+        bf16x8 fa[2], fb[4];
 #pragma unroll
-            for (int a = 0; a < 4; ++a)
+        for (int a = 0; a < 2; ++a) fa[a] = frag(s, LA, co + 16 * a);
 #pragma unroll
-                for (int b = 0; b < 4; ++b)
-                    acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fb[b], fa[a], acc[a][b], 0, 0, 0);
-            if (more) store(lds + (cur ^ 1) * kStage);
+        for (int b = 0; b < 4; ++b) fb[b] = frag(s + BK * LA, LB, ci + 16 * b);
+        each([&](int a, int b) {
+            acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fb[b], fa[a], acc[a][b], 0, 0, 0);
+        });
+    };
+    // four stages on the way to registers, two in LDS in turn
+    SplitRows from(ph, g.splits, g.k_split, g.n), at = from;
+    constexpr int NS = 4;
+    Stage st[NS];
+#pragma unroll
+    for (int u = 0; u < NS; ++u) {
+        load(st[u], from);
+        if (!from.end) from.next();
+    }
+    if (!at.end) store(st[0], lds);
+    while (!at.end) {
+#pragma unroll
+        for (int u = 0; u < NS; ++u) {
+            load(st[u], from);
+            if (!from.end) from.next();
             __syncthreads();
+            product(lds + u % 2 * kStage);
+            const int q = at.q, chain = at.chain;
+            at.next();
+            if (at.q != q) {  // a split is complete
+                each([&](int a, int b) {
+                    sum[a][b] += acc[a][b];
+                    acc[a][b] = zero;
+                });
+                if (at.end || at.chain != chain) each([&](int a, int b) {
+                    (chain < 2 ? s01 : s23)[a][b] += sum[a][b];
+                    sum[a][b] = zero;
+                });
+            }
+            if (at.end) break;
+            store(st[(u + 1) % NS], lds + (u + 1) % 2 * kStage);
         }
     }
     // lane: column o = l % 16, rows i = 4 (l / 16) + e of each tile
-    float* C = g.part_w + (((long)mem * 3 + layer) * g.splits + split) * (H * H);
-#pragma unroll
-    for (int a = 0; a < 4; ++a)
-#pragma unroll
-        for (int b = 0; b < 4; ++b) {
-            const int o = o0 + 64 * (w >> 1) + 16 * a + (l & 15);
-            const int i = i0 + 64 * (w & 1) + 16 * b + 4 * (l >> 4);
-            *reinterpret_cast<floatx4*>(C + o * H + i) = acc[a][b];
-        }
+    float* C = g.part_w + (((long)mem * 3 + layer) * 4 + ph) * (H * H);
+    each([&](int a, int b) {
+        const int o = o0 + co + 16 * a + (l & 15), i = i0 + ci + 16 * b + 4 * (l >> 4);
+        *reinterpret_cast<floatx4*>(C + o * H + i) = s01[a][b] + s23[a][b];
+    });
 }
 
 struct UpdateArgs {
@@ -588,21 +685,18 @@ struct UpdateArgs {
     float lr, b1, b2, eps, c1, c2;
 };
 
-// The sum of nb partial sums v[b * width] (T: one or four adjacent ones) as four phases b % 4
-// of four chains each, the chains' and phases' order fixed.
-template <class T>
-__device__ __forceinline__ T phase_chain(const float* v, long width, int nb, int ph) {
-    typedef std::conditional_t<sizeof(T) == 16, floatx4, float> V;
-    V s0 = {}, s1 = {}, s2 = {}, s3 = {};
-    const auto at = [&](int b) { return (V) * reinterpret_cast<const T*>(v + b * width); };
+// Phase ph of the sum of nb partial sums v[b * width]: those with b % 4 = ph, in four chains
+// whose order is fixed (the weight gradients' splits are summed likewise in step_wgrad).
+__device__ __forceinline__ float phase_chain(const float* v, long width, int nb, int ph) {
+    float s0 = 0.0f, s1 = 0.0f, s2 = 0.0f, s3 = 0.0f;
     int b = ph;
     for (; b + 12 < nb; b += 16) {
-        s0 += at(b);
-        s1 += at(b + 4);
-        s2 += at(b + 8);
-        s3 += at(b + 12);
+        s0 += v[b * width];
+        s1 += v[(b + 4) * width];
+        s2 += v[(b + 8) * width];
+        s3 += v[(b + 12) * width];
     }
-    for (; b < nb; b += 4) s0 += at(b);
+    for (; b < nb; b += 4) s0 += v[b * width];
     return (s0 + s1) + (s2 + s3);
 }
 
@@ -618,8 +712,7 @@ __device__ __forceinline__ float adam_one(const UpdateArgs& u, long o, float gi)
 // Gradients from the partial sums, and Adam on them (or, ADAM false, the gradients alone to
 // `grad`). blockIdx.x: 64 tiles of 32 x 32 weights of each hidden layer, then the other
 // parameters by 64, four lanes' phases each. A tile's new weights also go out in BF16, as
-// they are and transposed through LDS, in the fragments' order. Bound by reading the splits'
-// partial sums (50 MB at four networks and 16 splits).
+// they are and transposed through LDS, in the fragments' order.
 constexpr int kWTiles = (H / 32) * (H / 32);
 constexpr int kL1Blks = (H * F + H) / 64, kBiasBlks = H / 64, kOutBlks = (H + 1 + 63) / 64;
 constexpr int kUpdateBlks = 3 * kWTiles + kL1Blks + 3 * kBiasBlks + kOutBlks;
@@ -632,9 +725,13 @@ __global__ __launch_bounds__(256) void step_update(UpdateArgs u) {
         __shared__ bf16 tile[32][36];
         const int layer = b / kWTiles, n0 = b % kWTiles / (H / 32) * 32, k0 = b % (H / 32) * 32;
         const int n = n0 + (t >> 3), k = k0 + 4 * (t & 7);
-        const float* v = u.part_w + ((long)mem * 3 + layer) * u.splits * (H * H) + n * H + k;
-        floatx4 s = phase_chain<floatx4>(v, H * H, u.splits, 0);
-        for (int ph = 1; ph < 4; ++ph) s += phase_chain<floatx4>(v, H * H, u.splits, ph);
+        const float* v = u.part_w + ((long)mem * 3 + layer) * 4 * (H * H) + n * H + k;
+        floatx4 c[4];
+#pragma unroll
+        for (int ph = 0; ph < 4; ++ph)
+            c[ph] = ph < u.splits ? *reinterpret_cast<const floatx4*>(v + ph * (H * H))
+                                  : floatx4{0.f, 0.f, 0.f, 0.f};
+        const floatx4 s = c[0] + c[1] + c[2] + c[3];
         const long o = pofs + kW2 + layer * (H * H + H) + n * H + k;
         if constexpr (ADAM) {
             bf16x4 h;
@@ -680,7 +777,7 @@ __global__ __launch_bounds__(256) void step_update(UpdateArgs u) {
         ofs = kW5;
     }
     const int o = b * 64 + (t & 63);
-    lds[t] = phase_chain<float>(part + min(o, width - 1), width, nb, t >> 6);
+    lds[t] = phase_chain(part + min(o, width - 1), width, nb, t >> 6);
     __syncthreads();
     if (t >= 64 || o >= width) return;
     const float gi = lds[t] + lds[64 + t] + lds[128 + t] + lds[192 + t];
