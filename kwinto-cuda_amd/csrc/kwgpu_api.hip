@@ -79,7 +79,9 @@ struct kwgpu_ctx {
     int device = 0;
     hipStream_t stream = nullptr;
     std::string err;
-    DevBuf opts, prices, status, rep, off, list, order, xd, td, ws, counters;
+    DevBuf opts, prices, in, out, order, ws, counters;
+    char* stage = nullptr;  // pinned host copy of `in` and `out` (up to kStageMax)
+    size_t stage_cap = 0;
     DevBuf window;     // the windowed march's counters, records (of wrecs PDEs) and list
     size_t wrecs = 0;
     // autotuned choices per (bucket, precision), and per precision whether an uneven
@@ -646,10 +648,37 @@ void group_pdes(const kwgpu_option* opts, size_t n, const int32_t* xd, const int
     for (size_t i = 0; i < n; ++i) list[fill[pde[i]]++] = (uint32_t)i;  // ascending per PDE
 }
 
-// Host-pointer FD price with the reference's PDE compression; results are left in
-// the device buffers `d_prices` / `d_status` (sized n). Returns KWGPU_OK or an error.
+// Host memory for a call's inputs and results, laid out as the device buffers c->in and
+// c->out, so that each goes over in one copy: twelve options took four uploads from pageable memory, a wait
+// and two downloads: 192 us a call, 162 us so. Pinned and kept with the context up to
+// kStageMax bytes (freed with it), pageable and the call's own beyond.
+constexpr size_t kStageMax = size_t(16) << 20;
+struct HostIo {
+    std::vector<char> large;
+    const double* prices = nullptr;    // results, per option
+    const int32_t* status = nullptr;
+};
+
+char* stage(kwgpu_ctx* c, HostIo& io, size_t bytes) {
+    if (bytes > kStageMax) {
+        io.large.resize(bytes);
+        return io.large.data();
+    }
+    if (c->stage_cap < bytes) {
+        if (c->stage) (void)hipHostFree(c->stage);
+        c->stage = nullptr;
+        c->stage_cap = 0;
+        const size_t want = std::max<size_t>(bytes + bytes / 4, size_t(64) << 10);
+        if (hipHostMalloc((void**)&c->stage, want, hipHostMallocDefault) != hipSuccess) return nullptr;
+        c->stage_cap = want;
+    }
+    return c->stage;
+}
+
+// Host-pointer FD price with the reference's PDE compression; results in io. combine: n is
+// both legs of the control variate, whose prices are combined into the first n / 2.
 int fd_price_host(kwgpu_ctx* c, const kwgpu_option* opts, size_t n, const kwgpu_fd1d_params* p,
-                  DevBuf& d_opts, DevBuf& d_prices, DevBuf& d_status, bool whole = false) {
+                  HostIo& io, bool whole = false, bool combine = false) {
     hipStream_t s = c->stream;
     // PDE compression, src/Pricer/kwFd1d.cpp:28-65: options equal in (t, r, q, z, e, w)
     // -- and, for uneven batches, in grid size -- share one solve.
@@ -675,66 +704,82 @@ int fd_price_host(kwgpu_ctx* c, const kwgpu_option* opts, size_t n, const kwgpu_
         if (!any) pprec.clear();
     }
 
+    const bool uneven = p->x_dims || p->t_dims;
+    size_t bytes = 0;
+    const auto carve = [&](size_t len) {
+        const size_t at = bytes;
+        bytes += (len + 255) / 256 * 256;
+        return at;
+    };
+    const size_t at_opts = carve(n * sizeof(kwgpu_option)), at_rep = carve(m * sizeof(uint32_t)),
+                 at_off = carve((m + 1) * sizeof(uint32_t)), at_list = carve(n * sizeof(uint32_t)),
+                 at_x = uneven ? carve(n * sizeof(int32_t)) : 0,
+                 at_t = uneven ? carve(n * sizeof(int32_t)) : 0, in_bytes = bytes,
+                 at_prices = carve(n * sizeof(double)), at_status = carve(n * sizeof(int32_t));
     hipError_t e;
-    if ((e = ensure(d_opts, n * sizeof(kwgpu_option))) != hipSuccess ||
-        (e = ensure(d_prices, n * sizeof(double))) != hipSuccess ||
-        (e = ensure(d_status, n * sizeof(int32_t))) != hipSuccess ||
-        (e = ensure(c->rep, m * sizeof(uint32_t))) != hipSuccess ||
-        (e = ensure(c->off, (m + 1) * sizeof(uint32_t))) != hipSuccess ||
-        (e = ensure(c->list, n * sizeof(uint32_t))) != hipSuccess)
+    if ((e = ensure(c->in, in_bytes)) != hipSuccess ||
+        (e = ensure(c->out, bytes - in_bytes)) != hipSuccess)
         return fail(c, KWGPU_ERR_NOMEM, "kwgpu: device allocation failed");
-    if ((e = hipMemcpyAsync(d_opts.p, opts, n * sizeof(kwgpu_option), hipMemcpyHostToDevice, s)) ||
-        (e = hipMemcpyAsync(c->rep.p, rep.data(), m * sizeof(uint32_t), hipMemcpyHostToDevice, s)) ||
-        (e = hipMemcpyAsync(c->off.p, off.data(), (m + 1) * sizeof(uint32_t), hipMemcpyHostToDevice,
-                            s)) ||
-        (e = hipMemcpyAsync(c->list.p, list.data(), n * sizeof(uint32_t), hipMemcpyHostToDevice, s)))
-        return hip_fail(c, e, "kwgpu: upload");
-
-    FdBatch b{};
-    b.opts = (const kwgpu_option*)d_opts.p;
-    b.rep = (const uint32_t*)c->rep.p;
-    b.off = (const uint32_t*)c->off.p;
-    b.list = (const uint32_t*)c->list.p;
-    b.m = (int)m;
-    b.x_dim = p->x_dim;
-    b.t_dim = p->t_dim;
-    b.density = p->density;
-    b.scale = p->scale;
-    b.theta = p->theta;
-    b.prices = (double*)d_prices.p;
-    b.status = (int32_t*)d_status.p;
+    char* const h = stage(c, io, bytes);
+    if (!h) return fail(c, KWGPU_ERR_NOMEM, "kwgpu: pinned staging allocation failed");
+    char *const d = (char*)c->in.p, *const d_out = (char*)c->out.p;
+    std::memcpy(h + at_opts, opts, n * sizeof(kwgpu_option));
+    std::memcpy(h + at_rep, rep.data(), m * sizeof(uint32_t));
+    std::memcpy(h + at_off, off.data(), (m + 1) * sizeof(uint32_t));
+    std::memcpy(h + at_list, list.data(), n * sizeof(uint32_t));
     std::vector<int32_t> pde_x, pde_t;
-    if (p->x_dims || p->t_dims) {
+    if (uneven) {
         // per-option sizes travel with the options (indexed by option)
-        if ((e = ensure(c->xd, n * sizeof(int32_t))) != hipSuccess ||
-            (e = ensure(c->td, n * sizeof(int32_t))) != hipSuccess)
-            return fail(c, KWGPU_ERR_NOMEM, "kwgpu: device allocation failed");
-        std::vector<int32_t> hx(n), ht(n);
+        int32_t *hx = (int32_t*)(h + at_x), *ht = (int32_t*)(h + at_t);
         for (size_t i = 0; i < n; ++i) {
             hx[i] = gx(i);
             ht[i] = gt(i);
         }
-        if ((e = hipMemcpyAsync(c->xd.p, hx.data(), n * sizeof(int32_t), hipMemcpyHostToDevice, s)) ||
-            (e = hipMemcpyAsync(c->td.p, ht.data(), n * sizeof(int32_t), hipMemcpyHostToDevice, s)))
-            return hip_fail(c, e, "kwgpu: upload");
-        b.x_dims = (const int32_t*)c->xd.p;
-        b.t_dims = (const int32_t*)c->td.p;
         pde_x.resize(m);
         pde_t.resize(m);
         for (size_t k = 0; k < m; ++k) {
             pde_x[k] = hx[rep[k]];
             pde_t[k] = ht[rep[k]];
         }
-        // the host vectors must outlive the async copies
-        if ((e = hipStreamSynchronize(s)) != hipSuccess) return hip_fail(c, e, "kwgpu: sync");
+    }
+    if ((e = hipMemcpyAsync(d, h, in_bytes, hipMemcpyHostToDevice, s))) {
+        (void)hipStreamSynchronize(s);
+        return hip_fail(c, e, "kwgpu: upload");
+    }
+
+    FdBatch b{};
+    b.opts = (const kwgpu_option*)(d + at_opts);
+    b.rep = (const uint32_t*)(d + at_rep);
+    b.off = (const uint32_t*)(d + at_off);
+    b.list = (const uint32_t*)(d + at_list);
+    b.m = (int)m;
+    b.x_dim = p->x_dim;
+    b.t_dim = p->t_dim;
+    b.density = p->density;
+    b.scale = p->scale;
+    b.theta = p->theta;
+    b.prices = (double*)d_out;
+    b.status = (int32_t*)(d_out + (at_status - at_prices));
+    if (uneven) {
+        b.x_dims = (const int32_t*)(d + at_x);
+        b.t_dims = (const int32_t*)(d + at_t);
     }
     const int rc = run_fd(c, b, pde_x.empty() ? nullptr : pde_x.data(),
                           pde_t.empty() ? nullptr : pde_t.data(), p->precision, p->layout, s,
                           pprec.empty() ? nullptr : pprec.data(), whole);
-    // the host vectors above must outlive every copy queued from them
-    e = hipStreamSynchronize(s);
+    // leg 3 of the control variate: price += BS(euro) - FD(euro)
+    // (src/Pricer/kwFd1d_BlackScholes.cpp:30-40)
+    e = hipSuccess;
+    if (!rc && combine)
+        e = kwgpu::launch_fd1d_bs_combine(b.opts, n / 2, b.prices, b.prices + n / 2, s);
+    if (!rc && !e)
+        e = hipMemcpyAsync(h + at_prices, d_out, bytes - at_prices, hipMemcpyDeviceToHost, s);
+    // the host memory must outlive every copy queued on it
+    const hipError_t es = hipStreamSynchronize(s);
     if (rc) return rc;
-    if (e != hipSuccess) return hip_fail(c, e, "kwgpu: FD solve");
+    if (e || es) return hip_fail(c, e ? e : es, "kwgpu: FD solve");
+    io.prices = (const double*)(h + at_prices);
+    io.status = (const int32_t*)(h + at_status);
     return KWGPU_OK;
 }
 
@@ -754,7 +799,7 @@ std::string range_error(const kwgpu_option& a, double density, double scale, int
 }
 
 int collect(kwgpu_ctx* c, const kwgpu_option* opts, size_t n, const kwgpu_fd1d_params* p,
-            const std::vector<int32_t>& st, const char* prefix) {
+            const int32_t* st, const char* prefix) {
     for (size_t i = 0; i < n; ++i) {
         if (st[i] == KWGPU_STATUS_OK) continue;
         const int xd = p->x_dims ? p->x_dims[i] : p->x_dim;
@@ -891,8 +936,8 @@ void kwgpu_destroy(kwgpu_ctx* c) {
     (void)hipEventDestroy(c->ev_graph);
     (void)hipEventDestroy(c->ev_done);
     if (c->hsizes) (void)hipHostFree(c->hsizes);
-    for (DevBuf* b : {&c->opts, &c->prices, &c->status, &c->rep, &c->off, &c->list, &c->order,
-                      &c->xd, &c->td, &c->ws, &c->counters, &c->window})
+    if (c->stage) (void)hipHostFree(c->stage);
+    for (DevBuf* b : {&c->opts, &c->prices, &c->in, &c->out, &c->order, &c->ws, &c->counters, &c->window})
         free_buf(*b);
     (void)hipStreamDestroy(c->stream);
     delete c;
@@ -919,14 +964,11 @@ int kwgpu_fd1d_price(kwgpu_ctx* c, const kwgpu_option* opts, size_t n,
     if (n > 0x7fffffffu) return fail(c, KWGPU_ERR_INVALID, "kwgpu: too many options");
     if (int rc = check_dims(c, p->x_dims, p->t_dims, n)) return rc;
     if (hipError_t e = hipSetDevice(c->device); e != hipSuccess) return hip_fail(c, e, "hipSetDevice");
-    if (int rc = fd_price_host(c, opts, n, p, c->opts, c->prices, c->status)) return rc;
-    std::vector<int32_t> st(n);
-    hipError_t e;
-    if ((e = hipMemcpy(prices, c->prices.p, n * sizeof(double), hipMemcpyDeviceToHost)) ||
-        (e = hipMemcpy(st.data(), c->status.p, n * sizeof(int32_t), hipMemcpyDeviceToHost)))
-        return hip_fail(c, e, "kwgpu: download");
-    if (status) std::memcpy(status, st.data(), n * sizeof(int32_t));
-    return collect(c, opts, n, p, st, "");
+    HostIo io;
+    if (int rc = fd_price_host(c, opts, n, p, io)) return rc;
+    std::memcpy(prices, io.prices, n * sizeof(double));
+    if (status) std::memcpy(status, io.status, n * sizeof(int32_t));
+    return collect(c, opts, n, p, io.status, "");
 }
 
 int kwgpu_fd1d_price_device(kwgpu_ctx* c, const kwgpu_option* d_opts, size_t n,
@@ -998,24 +1040,15 @@ int kwgpu_fd1d_bs_price(kwgpu_ctx* c, const kwgpu_option* opts, size_t n,
         td2.insert(td2.end(), p->t_dims, p->t_dims + n);
         p2.t_dims = td2.data();
     }
-    if (int rc = fd_price_host(c, both.data(), 2 * n, &p2, c->opts, c->prices, c->status)) return rc;
-    hipError_t e;
-    // leg 3 and combine: price += BS(euro) - FD(euro) (:30-40)
-    if ((e = kwgpu::launch_fd1d_bs_combine((const kwgpu_option*)c->opts.p, n, (double*)c->prices.p,
-                                           (const double*)c->prices.p + n, c->stream)))
-        return hip_fail(c, e, "kwgpu: combine kernel launch");
-    std::vector<int32_t> st(2 * n);
-    if ((e = hipMemcpyAsync(prices, c->prices.p, n * sizeof(double), hipMemcpyDeviceToHost,
-                            c->stream)) ||
-        (e = hipMemcpyAsync(st.data(), c->status.p, 2 * n * sizeof(int32_t), hipMemcpyDeviceToHost,
-                            c->stream)) ||
-        (e = hipStreamSynchronize(c->stream)))
-        return hip_fail(c, e, "kwgpu: download");
+    HostIo io;
+    if (int rc = fd_price_host(c, both.data(), 2 * n, &p2, io, false, true)) return rc;
+    std::memcpy(prices, io.prices, n * sizeof(double));
+    std::vector<int32_t> st(io.status, io.status + 2 * n);
     for (size_t i = 0; i < n; ++i)
         if (st[i] == KWGPU_STATUS_OK && st[n + i] != KWGPU_STATUS_OK) st[i] = st[n + i];
     st.resize(n);
     if (status) std::memcpy(status, st.data(), n * sizeof(int32_t));
-    return collect(c, opts, n, p, st, prefix);
+    return collect(c, opts, n, p, st.data(), prefix);
 }
 
 int kwgpu_fd1d_greeks(kwgpu_ctx* c, const kwgpu_option* opts, size_t n,
@@ -1062,14 +1095,10 @@ int kwgpu_fd1d_greeks(kwgpu_ctx* c, const kwgpu_option* opts, size_t n,
     // turns any other rounding of the march into leading digits (300 options with rates down
     // to 3e-4: 7e-10 of rho between the two marches), and windows save nothing here that a
     // book of this size is bound by
-    if (int rc = fd_price_host(c, all.data(), n9, &p9, c->opts, c->prices, c->status, true))
-        return rc;
-    std::vector<double> v(n9);
-    std::vector<int32_t> st(n9);
-    hipError_t e;
-    if ((e = hipMemcpy(v.data(), c->prices.p, n9 * sizeof(double), hipMemcpyDeviceToHost)) ||
-        (e = hipMemcpy(st.data(), c->status.p, n9 * sizeof(int32_t), hipMemcpyDeviceToHost)))
-        return hip_fail(c, e, "kwgpu: download");
+    HostIo io;
+    if (int rc = fd_price_host(c, all.data(), n9, &p9, io, true)) return rc;
+    const double* v = io.prices;
+    const int32_t* st = io.status;
     for (size_t i = 0; i < n; ++i) {
         const double* w = &v[kSets * i];
         const kwgpu_option& a = opts[i];

@@ -1164,6 +1164,12 @@ struct kwgpu_surrogate {
     size_t yall_cap = 0;
     float* xp = nullptr;    // prediction: node features, 2 rows per option
     size_t xp_cap = 0;
+    // a training call's samples, row orders (two, in pinned memory and on the device; the
+    // event marks an order's copy) and losses: kept up to kTrainKeep bytes
+    float *feat = nullptr, *tgt = nullptr, *eloss = nullptr;
+    uint32_t *dperm[2] = {}, *hperm[2] = {};
+    hipEvent_t ev_perm[2] = {};
+    size_t feat_cap = 0, perm_cap = 0, eloss_cap = 0;  // samples, members' rows, losses
     void* serve = nullptr;  // kwgpu_surrogate_price's per-option buffers (grown on demand)
     size_t serve_cap = 0;   // options they hold
     // the FD configuration the network emulates (set by kwgpu_surrogate_fit; by default
@@ -1220,6 +1226,40 @@ void free_scratch(kwgpu_surrogate* s) {
     s->cap = 0;
 }
 
+// Allocating and freeing a training call's buffers took 0.2 ms of a 1.6 ms call.
+constexpr size_t kTrainKeep = size_t(64) << 20;
+
+void free_train(kwgpu_surrogate* s) {
+    for (void* q : {(void*)s->feat, (void*)s->tgt, (void*)s->eloss, (void*)s->dperm[0],
+                    (void*)s->dperm[1]})
+        if (q) (void)hipFree(q);
+    for (uint32_t* q : s->hperm)
+        if (q) (void)hipHostFree(q);
+    s->feat = s->tgt = s->eloss = nullptr;
+    s->dperm[0] = s->dperm[1] = s->hperm[0] = s->hperm[1] = nullptr;
+    s->feat_cap = s->perm_cap = s->eloss_cap = 0;
+}
+
+// Buffers for n samples, `rows` rows to shuffle per member and `losses` losses.
+bool ensure_train(kwgpu_surrogate* s, size_t n, size_t rows, size_t losses) {
+    const size_t M = (size_t)s->members;
+    if (s->feat_cap >= n && s->perm_cap >= M * rows && s->eloss_cap >= losses) return true;
+    free_train(s);
+    const size_t pb = M * rows * sizeof(uint32_t);
+    if (hipMalloc(&s->feat, n * F * sizeof(float)) || hipMalloc(&s->tgt, n * sizeof(float)) ||
+        hipMalloc(&s->eloss, losses * sizeof(float)) || hipMalloc(&s->dperm[0], pb) ||
+        hipMalloc(&s->dperm[1], pb) ||
+        hipHostMalloc((void**)&s->hperm[0], pb, hipHostMallocDefault) ||
+        hipHostMalloc((void**)&s->hperm[1], pb, hipHostMallocDefault)) {
+        free_train(s);
+        return false;
+    }
+    s->feat_cap = n;
+    s->perm_cap = M * rows;
+    s->eloss_cap = losses;
+    return true;
+}
+
 // batch scratch, one slot of `rows` samples per member: x, targets, the BF16 planes, and
 // the partial sums of a step of so many rows (their block counts do not fall with the rows)
 hipError_t ensure_scratch(kwgpu_surrogate* s, size_t rows) {
@@ -1242,11 +1282,12 @@ hipError_t ensure_scratch(kwgpu_surrogate* s, size_t rows) {
     return hipSuccess;
 }
 
-// Partial gradients and losses (added to s->loss) of members m0 .. m0 + cnt - 1 over n rows:
+// Partial gradients and losses (added to `loss`) of members m0 .. m0 + cnt - 1 over n rows:
 // row m is sample idx[k sidx + m] of feat and target (k: slot of the member), or sample m
 // itself, with feat = s->x, where idx is null.
 hipError_t gradients(kwgpu_surrogate* s, int m0, int cnt, int n, const float* feat,
-                     const float* target, const uint32_t* idx, long sidx, hipStream_t st) {
+                     const float* target, const uint32_t* idx, long sidx, float* loss,
+                     hipStream_t st) {
     StepArgs a{};
     a.feat = feat;
     a.target = target;
@@ -1263,7 +1304,7 @@ hipError_t gradients(kwgpu_surrogate* s, int m0, int cnt, int n, const float* fe
     a.plane = (long)s->cap * H;
     a.part_b = s->part_b;
     a.part_o = s->part_o;
-    a.loss = s->loss;
+    a.loss = loss;
     // 16-row tiles of a block's rows, four or five a pass: five where that saves a pass
     const int tiles = (n + 16 * a.rs - 1) / (16 * a.rs);
     if ((tiles + 4) / 5 < (tiles + 3) / 4)
@@ -1358,7 +1399,11 @@ int kwgpu_surrogate_create(kwgpu_ctx* ctx, int32_t members, uint64_t seed, kwgpu
     auto* s = new kwgpu_surrogate();
     s->members = members;
     s->device = kwgpu::ctx_device(ctx);
-    if (hipEventCreateWithFlags(&s->ev_done, hipEventDisableTiming)) {
+    if (hipEventCreateWithFlags(&s->ev_done, hipEventDisableTiming) ||
+        hipEventCreateWithFlags(&s->ev_perm[0], hipEventDisableTiming) ||
+        hipEventCreateWithFlags(&s->ev_perm[1], hipEventDisableTiming)) {
+        for (hipEvent_t e : {s->ev_done, s->ev_perm[0], s->ev_perm[1]})
+            if (e) (void)hipEventDestroy(e);
         delete s;
         return kwgpu::ctx_fail(ctx, KWGPU_ERR_HIP, "kwgpu_surrogate_create: event");
     }
@@ -1396,6 +1441,9 @@ void kwgpu_surrogate_destroy(kwgpu_surrogate* s) {
     (void)hipSetDevice(s->device);
     (void)hipDeviceSynchronize();
     free_scratch(s);
+    free_train(s);
+    for (hipEvent_t e : s->ev_perm)
+        if (e) (void)hipEventDestroy(e);
     for (void* q : {(void*)s->pall, (void*)s->wball, (void*)s->wballT, (void*)s->grad,
                     (void*)s->m1, (void*)s->m2,
                     (void*)s->loss, (void*)s->yall, (void*)s->xp, s->serve})
@@ -1468,7 +1516,7 @@ int kwgpu_surrogate_loss_grad(kwgpu_ctx* ctx, kwgpu_surrogate* s, int32_t member
     HIPCHK(hipMemcpy(s->x, host_x, n * F * sizeof(float), hipMemcpyHostToDevice));
     HIPCHK(hipMemcpy(s->tg, host_t, n * sizeof(float), hipMemcpyHostToDevice));
     hipLaunchKernelGGL(zero_f, dim3(1), dim3(64), 0, st, s->loss, (size_t)1);
-    HIPCHK(gradients(s, member, 1, (int)n, s->x, s->tg, nullptr, 0, st));
+    HIPCHK(gradients(s, member, 1, (int)n, s->x, s->tg, nullptr, 0, s->loss, st));
     HIPCHK(update(s, 1, (int)n, nullptr, st));
     HIPCHK(hipStreamSynchronize(st));
     float l = 0;
@@ -1486,7 +1534,8 @@ namespace {
 // taken on grid g; `rows` (host, optional) lists the rows to use, all n otherwise. Member
 // m shuffles with its own stream seeded from tp->seed; the next epoch's permutation is
 // drawn on a host thread while the current epoch runs, into the other of two pinned /
-// device buffer pairs.
+// device buffer pairs. The epochs are queued without a wait between them, but for the order
+// buffers' reuse; the losses come down at the end.
 int train_rows(kwgpu_ctx* ctx, kwgpu_surrogate* s, const kwgpu_option* d_opts,
                const double* d_premium, size_t n, const GridArg& g,
                const std::vector<uint32_t>* rows, const kwgpu_surrogate_train_params* tp,
@@ -1499,29 +1548,22 @@ int train_rows(kwgpu_ctx* ctx, kwgpu_surrogate* s, const kwgpu_option* d_opts,
         return kwgpu::ctx_fail(ctx, KWGPU_ERR_INVALID,
                                "kwgpu_surrogate_train: fewer usable rows (" + std::to_string(nr) +
                                    ") than a batch");
-    float *feat = nullptr, *tgt = nullptr;
-    uint32_t* dperm[2] = {nullptr, nullptr};
-    uint32_t* hperm[2] = {nullptr, nullptr};
     int rc = KWGPU_OK;
+    const size_t pbytes = (size_t)M * nr * sizeof(uint32_t);
+    const size_t losses = (size_t)tp->epochs * M;
     auto cleanup = [&]() {
         (void)hipStreamSynchronize(st);
-        (void)hipFree(feat);
-        (void)hipFree(tgt);
-        for (int k = 0; k < 2; ++k) {
-            (void)hipFree(dperm[k]);
-            (void)hipHostFree(hperm[k]);
-        }
+        if (s->feat_cap * (F + 1) * sizeof(float) + 2 * s->perm_cap * sizeof(uint32_t) +
+                s->eloss_cap * sizeof(float) >
+            kTrainKeep)
+            free_train(s);
     };
-    const size_t pbytes = (size_t)M * nr * sizeof(uint32_t);
-    if (hipMalloc(&feat, n * F * sizeof(float)) || hipMalloc(&tgt, n * sizeof(float)) ||
-        hipMalloc(&dperm[0], pbytes) || hipMalloc(&dperm[1], pbytes) ||
-        hipHostMalloc((void**)&hperm[0], pbytes, hipHostMallocDefault) ||
-        hipHostMalloc((void**)&hperm[1], pbytes, hipHostMallocDefault) || ensure_scratch(s, B)) {
-        cleanup();
+    if (!ensure_train(s, n, nr, losses) || ensure_scratch(s, B))
         return kwgpu::ctx_fail(ctx, KWGPU_ERR_NOMEM, "kwgpu_surrogate_train: allocation");
-    }
-    hipLaunchKernelGGL(features_kernel, dim3(nblk((n + 1) / 2, kPairsPerWave)), dim3(64), 0, st, d_opts, n, g,
-                       d_premium, feat, tgt);
+    float *const feat = s->feat, *const tgt = s->tgt;
+    uint32_t *const *dperm = s->dperm, *const *hperm = s->hperm;
+    hipLaunchKernelGGL(features_kernel, dim3(nblk((n + 1) / 2, kPairsPerWave)), dim3(64), 0, st,
+                       d_opts, n, g, d_premium, feat, tgt);
     // every member steps at once (one launch per layer for the whole ensemble), each on
     // its own shuffle of the rows
     std::vector<std::mt19937_64> rng;
@@ -1542,22 +1584,32 @@ int train_rows(kwgpu_ctx* ctx, kwgpu_surrogate* s, const kwgpu_option* d_opts,
                        (size_t)M * kP);
     hipLaunchKernelGGL(zero_f, dim3(nblk((size_t)M * kP, 256)), dim3(256), 0, st, s->m2,
                        (size_t)M * kP);
+    hipLaunchKernelGGL(zero_f, dim3(nblk(losses, 256)), dim3(256), 0, st, s->eloss, losses);
+    // an order from its pinned buffer to the device
+    auto upload = [&](int k) -> hipError_t {
+        hipError_t e = hipMemcpyAsync(dperm[k], hperm[k], pbytes, hipMemcpyHostToDevice, st);
+        return e ? e : hipEventRecord(s->ev_perm[k], st);
+    };
     draw(hperm[0]);
-    if (hipError_t e = hipMemcpyAsync(dperm[0], hperm[0], pbytes, hipMemcpyHostToDevice, st)) {
+    if (hipError_t e = upload(0)) {
         cleanup();
         return kwgpu::ctx_fail(ctx, KWGPU_ERR_HIP, std::string("permutation: ") + hipGetErrorString(e));
     }
     long step = 0;
-    std::vector<float> lsum(M);
     for (int ep = 0; ep < tp->epochs && rc == KWGPU_OK; ++ep) {
         const uint32_t* didx = dperm[ep & 1];
-        // the next epoch's order, drawn while this one runs: its host buffer was last
-        // copied from before the previous epoch's end, which was waited for
+        // the next epoch's order, drawn while this one runs, once the copy of the order
+        // that its host buffer held is done
         std::thread next;
-        if (ep + 1 < tp->epochs) next = std::thread(draw, hperm[(ep + 1) & 1]);
-        hipLaunchKernelGGL(zero_f, dim3(1), dim3(64), 0, st, s->loss, (size_t)M);
+        const int kn = (ep + 1) & 1;
+        if (ep + 1 < tp->epochs)
+            next = std::thread([&, kn, ep] {
+                if (ep > 0) (void)hipEventSynchronize(s->ev_perm[kn]);
+                draw(hperm[kn]);
+            });
         for (size_t b = 0; b < steps_per_epoch; ++b, ++step) {
-            hipError_t e = gradients(s, 0, M, B, feat, tgt, didx + b * B, (long)nr, st);
+            hipError_t e = gradients(s, 0, M, B, feat, tgt, didx + b * B, (long)nr,
+                                     s->eloss + (size_t)ep * M, st);
             const double frac = step / total;
             const float lr = (float)(tp->lr_final + 0.5 * (tp->lr - tp->lr_final) *
                                                          (1.0 + std::cos(M_PI * frac)));
@@ -1580,18 +1632,16 @@ int train_rows(kwgpu_ctx* ctx, kwgpu_surrogate* s, const kwgpu_option* d_opts,
         if (next.joinable()) next.join();
         if (rc == KWGPU_OK && ep + 1 < tp->epochs) {
             // the other device buffer was last read by the previous epoch (stream order)
-            if (hipError_t e = hipMemcpyAsync(dperm[(ep + 1) & 1], hperm[(ep + 1) & 1], pbytes,
-                                              hipMemcpyHostToDevice, st))
-                rc = kwgpu::ctx_fail(ctx, KWGPU_ERR_HIP, hipGetErrorString(e));
+            if (hipError_t e = upload(kn)) rc = kwgpu::ctx_fail(ctx, KWGPU_ERR_HIP, hipGetErrorString(e));
         }
-        if (hipError_t e = hipStreamSynchronize(st)) {
-            if (rc == KWGPU_OK) rc = kwgpu::ctx_fail(ctx, KWGPU_ERR_HIP, hipGetErrorString(e));
-            break;
-        }
-        (void)hipMemcpy(lsum.data(), s->loss, M * sizeof(float), hipMemcpyDeviceToHost);
-        if (loss_out)
-            for (int m = 0; m < M; ++m)
-                loss_out[(size_t)ep * M + m] = lsum[m] / (float)(steps_per_epoch * B);
+    }
+    if (rc == KWGPU_OK) {
+        std::vector<float> lsum(losses);
+        hipError_t e = hipStreamSynchronize(st);
+        if (!e) e = hipMemcpy(lsum.data(), s->eloss, losses * sizeof(float), hipMemcpyDeviceToHost);
+        if (e) rc = kwgpu::ctx_fail(ctx, KWGPU_ERR_HIP, hipGetErrorString(e));
+        if (loss_out && !e)
+            for (size_t k = 0; k < losses; ++k) loss_out[k] = lsum[k] / (float)(steps_per_epoch * B);
     }
     cleanup();
     return rc;
