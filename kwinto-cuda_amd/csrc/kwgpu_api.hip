@@ -195,8 +195,21 @@ bool windowed_fits(int cap, int precision, double theta) {
 // ... but not for a uniform batch of short marches, whose windows are their whole grids, nor
 // for few PDEs of over 1024 points: some window then needs the two-wave march anyway, and the
 // batch takes its time (600 at 2048 x 512: 393 us windowed, 387 us not; 1500: 426 and 747).
+// Listing the windows and eliminating their pinned rows takes 20 to 30 us, which a march of
+// few point-steps does not give back: 8000 at 256 x 100 97 us windowed, 87 not; 3000 at 512 x
+// 160 135 and 122; 3000 at 1024 x 160 (4.9e8 point-steps) 185 and 173; 8000 at 1024 x 66 (5.3e8)
+// 194 and 213; 14317 at 256 x 160 (5.8e8) 192 and 216. Up to kLoneMax PDEs nothing is listed:
+// 2048 at 256 x 66 48 and 45 us, at 256 x 100 56 and 57, at 384 x 66 47 and 52; with a wave or
+// less to a SIMD the widest windows, which need 16 rows a lane either way, set the batch's time
+// (173 at 1024 x 256 112 and 103 us).
+constexpr int kLongMarch = 256;
 bool uniform_windowed(size_t m, int x_dim, int t_dim) {
-    return t_dim - 1 >= kwgpu::kWindowMinSteps && (x_dim <= 1024 || m > kwgpu::kLoneMax / 2);
+    const int steps = t_dim - 1;
+    if (steps < kwgpu::kWindowMinSteps) return false;
+    if (x_dim > 1024) return m > kwgpu::kLoneMax / 2;
+    if (m <= kwgpu::kLoneMax / 2) return x_dim <= 896;
+    if (m <= kwgpu::kLoneMax) return x_dim > 256 || steps >= 99;
+    return steps >= kLongMarch || (double)m * x_dim * steps >= 5e8;
 }
 
 Choice choice_for(const kwgpu_ctx* c, int cap, int precision, int layout, double theta) {
