@@ -153,12 +153,16 @@ int kwgpu_fd1d_price_device(kwgpu_ctx* ctx, const kwgpu_option* d_opts, size_t n
  * tight serving loops and harnesses that forbid hipMalloc). Same pricing, per-option
  * grids included, on device-resident options, prices and status, asynchronous on
  * `stream`; here params->x_dims / params->t_dims, when set, are HOST arrays of n sizes.
- * The PDE order, the sizes and the bucket counters of the batch live in a fixed device
+ * The PDE order, the sizes, the bucket counters and the records of the windowed march (of
+ * uniform batches too) live in a fixed device
  * scratch array of the library (24 MiB per device, held until the process ends): at most
  * 1048576 options (more returns KWGPU_ERR_INVALID), wave layout only (x_dim <= 2048, else
  * KWGPU_ERR_UNSUPPORTED). No graph and no side stream: the grid-size buckets run one
  * after another on `stream`. Calls on one context are ordered; calls from different
- * contexts on one GPU share the scratch and race when they overlap.
+ * contexts on one GPU share the scratch and race when they overlap. While `stream` is being
+ * captured a batch of one grid size is recorded without any scratch (its march carries whole
+ * grids where a windowed one would need it), so the graph's replays may overlap other
+ * calls; a batch of per-option grids, which uploads its sizes, cannot be captured.
  */
 int kwgpu_fd1d_price_device_noalloc(kwgpu_ctx* ctx, const kwgpu_option* d_opts, size_t n,
                                     const kwgpu_fd1d_params* params, double* d_prices,

@@ -242,14 +242,20 @@ kwgpu::WindowScratch window_scratch(const kwgpu_ctx* c) {
     return {rec, (uint32_t*)(rec + c->wrecs), counts};
 }
 
-// A stream under capture takes no scratch of the context: the captured launch may be
-// replayed beside the context's other solves and after its buffers have grown. (The
-// stand-in runtime of the host tests has no such call.)
+// A stream under capture takes no scratch, of the context or of the device: the captured
+// launch may be replayed beside any other solve and after the context's buffers have grown.
+// (The stand-in runtime of the host tests may have no such call.)
 extern "C" hipError_t hipStreamIsCapturing(hipStream_t, hipStreamCaptureStatus*) __attribute__((weak));
 bool capturing(hipStream_t s) {
     hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
     if (!hipStreamIsCapturing || hipStreamIsCapturing(s, &st) != hipSuccess) return false;
     return st != hipStreamCaptureStatusNone;
+}
+
+// Whether a uniform batch whose choice is the windowed march takes it on stream s.
+bool takes_windows(size_t m, int x_dim, int t_dim, hipStream_t s) {
+    const bool scratch = m > (size_t)kwgpu::kLoneMax || x_dim > 1024;
+    return uniform_windowed(m, x_dim, t_dim) && !(scratch && capturing(s));
 }
 
 uint64_t fnv(uint64_t h, const void* p, size_t n) {
@@ -436,10 +442,9 @@ int run_fd_on(kwgpu_ctx* c, FdBatch b, const int32_t* pde_x, const int32_t* pde_
         const int cap = bucket_of(b.x_dim, precision, layout);
         Choice ch = choice_for(c, cap, precision, layout, theta);
         if (ch.variant == kWindowed) {
-            const bool scratch = b.m > kwgpu::kLoneMax || b.x_dim > 1024;
-            if (uniform_windowed(b.m, b.x_dim, b.t_dim) && !(scratch && capturing(s))) {
+            if (takes_windows(b.m, b.x_dim, b.t_dim, s)) {
                 const int big = b.x_dim > 1024 ? b.m : 0;
-                if (scratch)
+                if (b.m > kwgpu::kLoneMax || big)
                     if (int rc = ensure_window(c, b.m, b.m, big)) return rc;
                 if (hipError_t e = kwgpu::launch_fd1d_windowed(b, window_scratch(c), big, s))
                     return hip_fail(c, e, "kwgpu: windowed kernel launch");
@@ -1190,8 +1195,9 @@ int kwgpu_fd1d_price_device_noalloc(kwgpu_ctx* c, const kwgpu_option* d_opts, si
     if (!hx && !ht) {
         const int cap = bucket_of(p->x_dim, p->precision, p->layout);
         Choice ch = choice_for(c, cap, p->precision, p->layout, p->theta);
-        if (ch.variant == kWindowed && !uniform_windowed(n, p->x_dim, p->t_dim))
+        if (ch.variant == kWindowed && !takes_windows(n, p->x_dim, p->t_dim, s))
             ch = Choice{kwgpu::default_wave_variant(cap), true};
+        if (capturing(s)) ch.persist = false;  // a persistent grid's work counter is scratch
         plan.push_back(Bucket{cap, ch, 0, n, p->x_dim, p->precision, p->x_dim > 1024 ? (int)n : 0});
     } else {
         const Slots slots(c, p->layout, p->theta);
@@ -1232,7 +1238,9 @@ int kwgpu_fd1d_price_device_noalloc(kwgpu_ctx* c, const kwgpu_option* d_opts, si
     if (plan.size() > (size_t)kNoAllocCounters)
         return fail(c, KWGPU_ERR_INVALID, "kwgpu_fd1d_price_device_noalloc: too many buckets");
     // a fill kernel, not a memset, clears the counters the persistent grids take work from
-    if ((e = kwgpu::launch_zero_counters(d_counters, (int)plan.size(), s)))
+    bool persist = false;
+    for (const Bucket& k : plan) persist |= k.ch.persist;
+    if (persist && (e = kwgpu::launch_zero_counters(d_counters, (int)plan.size(), s)))
         return hip_fail(c, e, "kwgpu_fd1d_price_device_noalloc: counter reset");
     for (size_t i = 0; i < plan.size(); ++i) {
         const Bucket& k = plan[i];

@@ -1,0 +1,63 @@
+"""Which kernels a call launches, on the CPU: the library's host code against a stand-in HIP
+runtime that records the launches (tests/hostmock/route_mock.cpp, routes.cpp). No kernel runs."""
+from __future__ import annotations
+
+import os
+import pathlib
+import re
+import subprocess
+
+import pytest
+
+ROOT = pathlib.Path(__file__).resolve().parents[1]
+SRC = ROOT / "kwinto-cuda_amd" / "csrc"
+MOCK = pathlib.Path(__file__).resolve().parent / "hostmock"
+HIPCC = "/opt/rocm/bin/hipcc"
+UNITS = ["kwgpu_api", "fd1d_wave", "fd1d_lane", "bs", "surrogate"]
+LISTED = ["zero_counters", "plan_windows", "list_windows", "fd1d_windowed"]
+
+
+@pytest.fixture(scope="module")
+def routes(tmp_path_factory):
+    """routes(request, ...): the kernels that each request launches, a list of names each."""
+    if not os.path.exists(HIPCC):
+        pytest.skip("ROCm compilers not installed")
+    d = tmp_path_factory.mktemp("routes")
+    host = [HIPCC, "-O1", "-std=c++17", "-fPIC", "--offload-host-only", f"-I{ROOT / 'include'}",
+            f"-I{SRC}", f"-I{MOCK}"]
+    src = [SRC / f"{u}.hip" for u in UNITS] + [MOCK / "route_mock.cpp", MOCK / "routes.cpp"]
+    jobs = [subprocess.Popen(host + ["-c", str(s), "-o", str(d / (s.stem + ".o"))],
+                             stderr=subprocess.PIPE, text=True) for s in src]
+    for p, s in zip(jobs, src):
+        err = p.communicate(timeout=600)[1]
+        assert p.returncode == 0, f"{s}: {err}"
+    objs = [str(d / (s.stem + ".o")) for s in src]
+    # each unit refers to its (absent) device code object by a generated name
+    nm = subprocess.run(["nm", "-u", *objs], capture_output=True, text=True, check=True).stdout
+    names = sorted(set(re.findall(r"__hip_fatbin_\w+", nm)))
+    (d / "fatbins.cpp").write_text("".join(f'extern "C" {{ char {n}[16]; }}\n' for n in names))
+    subprocess.run(["g++", *objs, str(d / "fatbins.cpp"), "-o", str(d / "routes")], check=True)
+
+    def run(*requests):
+        r = subprocess.run([str(d / "routes")], input="\n".join(requests) + "\n", text=True,
+                           capture_output=True, timeout=120)
+        assert r.returncode == 0, r.stderr
+        return [re.split(r",(?! )", ln) if ln else [] for ln in r.stdout.split("\n")[:-1]]
+    return run
+
+
+def test_capture_takes_no_shared_scratch(routes, tmp_path):
+    """A call captured into a graph may be replayed beside any other: it may only launch
+    kernels that keep nothing in the context's or the device's scratch (work counters,
+    windows' records and lists)."""
+    sizes = ["%s %d %d %d" % (c, n, x, t) for c in ("price", "noalloc") for n, x, t in (
+        (64, 512, 128), (2048, 1024, 256), (2049, 1024, 256), (2400, 256, 66), (16384, 512, 512),
+        (600, 2048, 256), (1500, 1025, 90), (4000, 2048, 257))]
+    free, held = routes("capture 0", *sizes), routes("capture 1", *sizes)
+    assert any("plan_windows" in k for k in free)
+    # tuned to the 16-row variants on persistent grids
+    (tmp_path / "tune").write_text("256 0 2 1\n512 0 5 1\n1024 0 8 1\n2048 0 9 1\n")
+    tuned = routes(f"tune {tmp_path / 'tune'}", "capture 1", *sizes)
+    for call, k in list(zip(sizes, held[1:])) + list(zip(sizes, tuned[2:])):
+        assert len(k) == 1 and k[0].split("<")[0] in ("fd1d_wave", "fd1d_lone"), (call, k)
+        assert k[0] == "fd1d_lone" or k[0].split(", ")[4] == "false", (call, k)  # persistent
