@@ -220,7 +220,7 @@ int kwgpu_fd1d_autotune(kwgpu_ctx* ctx, const kwgpu_option* d_opts, size_t n,
 
 /* Saves / loads the context's autotuned choices (text, one "bucket precision variant
  * persistent" line each). Loading skips lines of an unknown precision, variants that
- * do not hold their bucket and lane-layout choices for FP32-mixed. */
+ * do not exist or do not hold their bucket and lane-layout choices for FP32-mixed. */
 int kwgpu_tune_save(kwgpu_ctx* ctx, const char* path);
 int kwgpu_tune_load(kwgpu_ctx* ctx, const char* path);
 

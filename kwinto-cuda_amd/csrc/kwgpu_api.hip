@@ -343,7 +343,7 @@ int launch_buckets(kwgpu_ctx* c, const FdBatch& b, const std::vector<Bucket>& pl
         if (k.ch.variant == kWindowed) {
             if ((e = kwgpu::launch_fd1d_windowed(bb, window_scratch(c), k.big, ss)))
                 return hip_fail(c, e, "kwgpu: windowed kernel launch");
-        } else if (k.ch.variant < 0) {
+        } else if (k.ch.variant == kLane) {
             double* ws = (double*)c->ws.p + ws_off;
             ws_off += kwgpu::lane_workspace_doubles(bb.m, k.max_x);
             if (int rc = lane_launch(c, bb, k.max_x, k.prec, ss, ws)) return rc;
@@ -452,7 +452,7 @@ int run_fd_on(kwgpu_ctx* c, FdBatch b, const int32_t* pde_x, const int32_t* pde_
             }
             ch.variant = kwgpu::default_wave_variant(cap);
         }
-        if (ch.variant < 0) {
+        if (ch.variant == kLane) {
             const size_t need = kwgpu::lane_workspace_doubles(b.m, b.x_dim) * sizeof(double);
             if (c->ws.cap < need) drop_graph(c);  // a captured graph may hold the old buffer
             if (ensure(c->ws, need) != hipSuccess)
@@ -1522,7 +1522,7 @@ int kwgpu_tune_load(kwgpu_ctx* c, const char* path) {
             c->serial[prec] = v != 0;
             continue;
         }
-        if (v == kWindowed && !windowed_fits(cap, prec, 0.5)) continue;
+        if (v < kWindowed || (v == kWindowed && !windowed_fits(cap, prec, 0.5))) continue;
         if (v >= kwgpu::wave_variant_count() || (v >= 0 && kwgpu::wave_variant(v).capacity() != cap)) continue;
         if (v < 0 && prec != KWGPU_FP64) continue;
         c->tuned[{cap, prec}] = Choice{v, per != 0};

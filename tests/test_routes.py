@@ -61,3 +61,19 @@ def test_capture_takes_no_shared_scratch(routes, tmp_path):
     for call, k in list(zip(sizes, held[1:])) + list(zip(sizes, tuned[2:])):
         assert len(k) == 1 and k[0].split("<")[0] in ("fd1d_wave", "fd1d_lone"), (call, k)
         assert k[0] == "fd1d_lone" or k[0].split(", ")[4] == "false", (call, k)  # persistent
+
+
+@pytest.mark.parametrize("variant", [-3, -7, -100])
+def test_tune_file_with_an_unknown_march(routes, tmp_path, variant):
+    """A tune file's march numbers below those that exist are skipped, as variants that do not
+    hold their bucket are: no lane kernel runs without its workspace."""
+    f = tmp_path / "tune"
+    f.write_text("".join(f"{cap} 0 {variant} 0\n" for cap in (128, 256, 512, 1024, 2048)))
+    calls = ["price 100 128 90", "price 3000 512 400", "uneven 300 90 100,256,700,2048",
+             "noalloc 3000 512 400", "noalloc_uneven 300 90 100,256,700,2048", "host 50 256 90"]
+    plain, tuned = routes(*calls), routes(f"tune {f}", *calls)[1:]
+    assert plain == tuned
+    # the lane layout itself (-1) is still taken from a file, with its workspace
+    f.write_text("512 0 -1 0\n")
+    for k in routes(f"tune {f}", "price 3000 512 400", "uneven 300 90 100,256,512,2048")[1:]:
+        assert any("fd1d_lane" in x for x in k) and "null workspace" not in k
