@@ -42,30 +42,36 @@ constexpr int kWindowMinSteps = 64;
 
 // log of the critical spot of an American put with unit strike, rate r > 0 and yield q, in
 // Barone-Adesi & Whaley's approximation: the root of
-//     f(S) = (1 - S) - E(S) + (1 - e^{-qT} Phi(-d1(S))) S / lambda
-// by three Newton steps from their starting value between the perpetual critical spot and
-// min(1, r / q). In FP32: the result only places a cut that is checked afterwards. Over
-// 320000 options (vol 2-150 %, T 0.005-30 years) 36 are off by more than 0.02; a bisection
-// to the last digit costs some 20 evaluations of f and was half the planning time.
+//     f(S) = (1 - S) - E(S) + (1 - e^{-qT} Phi(-d1(S))) S / lambda,
+// E the European put. With m2 = 1 - e^{-rT} Phi(-d2) and n1 = 1 - e^{-qT} Phi(-d1) it is that of
+//     log m2 - log n1 = x + log(1 - 1 / lambda),   x = log S,
+// where nothing cancels at small rates, whose root lies up to five standard deviations from the
+// strike. Convex and falling on the root's left, so three Newton steps from a start that lies
+// mostly there: to 0.005 sigma sqrt(T) in 99 of 100 options of vol 2-200 %, T 0.005-20 years
+// and rates down to 1e-6. (Newton steps in S from the starting value of their paper were off
+// by more than 0.5 at a tenth of the rates below 1 %; with the margin of then nearly every cut was
+// passed at rates under 1e-4 and half of them under 1e-3: 8192 options of vol 80-150 % and
+// rates under 1e-4 at 512 x 512 took 1891 us, on whole grids 685, and so 628.) In FP32: the
+// result only places a cut that is checked afterwards. No number where n1 is not positive, as
+// it can be at q < 0.
 KWGPU_HD float critical_log_spot(float t, float z, float r, float q) {
-    const float z2 = z * z, st = z * sqrtf(t), n = 2.0f * (r - q) / z2 - 1.0f;
-    const float lam = 0.5f * (-n - sqrtf(n * n - 8.0f * r / (z2 * expm1f(-r * t))));
+    const float z2 = z * z, rt = sqrtf(t), st = z * rt, n = 2.0f * (r - q) / z2 - 1.0f;
+    const float er1 = -expm1f(-r * t), eq1 = -expm1f(-q * t), er = 1.0f - er1, eq = 1.0f - eq1;
+    const float lam = 0.5f * (-n - sqrtf(n * n + 8.0f * r / (z2 * er1)));
     const float perp = 0.5f * (-n - sqrtf(n * n + 8.0f * r / z2));
-    const float eq = expf(-q * t), er = expf(-r * t), drift = (r - q + 0.5f * z2) * t;
-    const float lowest = perp / (perp - 1.0f), top = q > r ? r / q : 1.0f;
-    const float h = ((r - q) * t - 2.0f * st) / (1.0f - lowest);
-    float s = lowest + (top - lowest) * expf(h < 0.0f ? h : 0.0f);
-    s = fminf(fmaxf(s, 1e-3f), top);
+    const float c = logf(1.0f - 1.0f / lam), drift = (r - q + 0.5f * z2) * t;
+    const float top = q > r ? logf(r / q) : 0.0f, gain = q < 0.0f ? r - q : r;
+    float x = fmaxf(logf(perp / (perp - 1.0f)), top - st * sqrtf(2.0f * logf(1.0f + 0.3f * z / (gain * rt))));
     for (int it = 0; it < 3; ++it) {
-        const float d1 = (logf(s) + drift) / st;
-        const float n1 = 1.0f - 0.5f * eq * erfcf(d1 * 0.70710678f);  // 1 - e^{-qT} Phi(-d1)
-        const float n2 = 0.5f * er * erfcf((d1 - st) * 0.70710678f);
-        const float f = (1.0f - s) - (n2 - s * (1.0f - n1)) + n1 * s / lam;
-        const float df = n1 * (1.0f / lam - 1.0f) +
-                         eq * 0.39894228f * expf(-0.5f * d1 * d1) / (lam * st);
-        s = fminf(fmaxf(s - f / df, 0.5f * s), fminf(top, 2.0f * s));
+        const float d1 = (x + drift) / st, d2 = d1 - st;
+        const float n1 = eq1 + 0.5f * eq * erfcf(-d1 * 0.70710678f);
+        const float m2 = er1 + 0.5f * er * erfcf(-d2 * 0.70710678f);
+        if (!(n1 > 0.0f)) return NAN;
+        const float f = logf(m2 / n1) - x - c;
+        const float df = 0.39894228f * (er * expf(-0.5f * d2 * d2) / m2 - eq * expf(-0.5f * d1 * d1) / n1) / st - 1.0f;
+        x = fminf(fmaxf(x - f / df, x - 0.7f * st), top);
     }
-    return logf(s);
+    return x;
 }
 
 // The window of option o on an N-point grid marched `steps` steps at theta = 1/2. `far`:
@@ -75,21 +81,26 @@ KWGPU_HD float critical_log_spot(float t, float z, float r, float q) {
 // error of e^-36 = 2e-16. Where the steps are few Crank-Nicolson's tails are heavier than
 // the Gaussian's: at 64 steps the exponent 36 loses 2 n (y^3/3 + ...), y = 36 / (2 n), 0.9.
 //
-// In the money the cut lies min(0.075, 0.24 sigma sqrt(T)) in log S and 2 rows past the
-// approximate critical spot. Measured on 7400 marches (vol 1-200 %, T 0.005-30 years, rates
-// -3-25 %, 1024 and 2048 points) the boundary ended at most 0.070 past it, and 0.23 sigma
-// sqrt(T): where the rate is near 0 the approximation lies too near the strike (half of the
-// options: under 0.004). A cut that is too near costs a second march after the first, which
-// a whole launch may wait for (0.5 ms of 2.2 for one option of 16384); the margin costs about
-// 10 rows of 1024. The cut needs
+// In the money the cut lies 0.25 sigma sqrt(T) / (1 + sqrt(a / 0.06)), a = r sqrt(T) / sigma, in
+// log S and 2 rows past the approximate critical spot. The boundary ends past that spot by more
+// the smaller a is: over 2256 marches (1024 x 512, vol 2-200 %, T 0.005-20 years, rates 1e-5 to
+// 25 %) by at most 0.20 sigma sqrt(T) and 2 rows at a < 1e-5, 0.14 at 1e-3, 0.09 at 0.1 and 0.02
+// at 1. Of 50000 cuts on 129 to 2048 points (rates 1e-7 to 50 %, yields below and above them by
+// any factor) 27 were passed. A cut that is too near costs a second march after
+// the first, which a whole launch may wait for (0.5 ms of 2.2 for one option of 16384); the
+// margin costs about 6 rows of 1024. The cut needs
 //   * kPinnedRows rows to forget the approximate value they are started from: with
 //     a = theta dt (sigma^2 / 2) / dx^2 at the cut, an error shrinks by about
 //     e^{-1/sqrt(a)} per row, and a <= 150 leaves 1e-9 of an error of O(dt^2);
+//   * the mesh to see the early exercise: a put's payoff falls behind at r in the money, and the
+//     differences are off there by about sigma^2 dx^2 S / 4; where that is more than r, no row
+//     stays pinned;
 //   * early exercise to be worth something: while q > r the boundary never comes nearer than
 //     log(r / q) to the strike, and past 4.5 sigma sqrt(T) the premium is below about 1e-9 of
 //     the price. Such an option keeps the rows its European twin keeps, and with them the
 //     same arithmetic, so that rounding cannot price it below the twin (on 32768 options at
-//     1024 x 1024 the two had differed by up to 9e-11, the smallest such ratio 5.1);
+//     1024 x 1024 the two had differed by up to 9e-11, the smallest such ratio 5.1). At a < 1e-3 the
+//     approximation is off by up to 1.3 sigma sqrt(T) from a ratio of 0.5 on;
 //   * for a call, the unprojected edge row to be forgotten as well: its value can be
 //     e^{scale sigma sqrt(T)}, 22 sigma sqrt(T) decades, and a row with a < 0.1 takes off
 //     at least one.
@@ -117,9 +128,10 @@ KWGPU_HD Window window_of(const kwgpu_option& o, int N, int steps, double densit
     // the put that the option is in xi
     const double r = o.w < 0 ? o.r : o.q, q = o.w < 0 ? o.q : o.r;
     if (!o.e || !(r > 0.0)) return w;
-    if (q > r && log(q / r) > 4.5 * s) return w;
+    const double a0 = r * o.t / s;  // r sqrt(T) / sigma
+    if (q > r && log(q / r) > (a0 < 1e-3 ? 0.5 : 4.5) * s) return w;
     const double xb = (double)critical_log_spot((float)o.t, (float)o.z, (float)r, (float)q) -
-                      fmin(0.075, 0.24 * s);
+                      0.25 * s / (1.0 + sqrt(a0 / 0.06));
     if (!(xb > -6.9)) return w;  // nor when it is no number
     const double at = (asinh(xb / density) + Y) * per;
     const int lo = (int)floor(at) - 2;
@@ -127,6 +139,7 @@ KWGPU_HD Window window_of(const kwgpu_option& o, int N, int steps, double densit
     const double dx = sqrt(xb * xb + density * density) * h;
     const double a1 = 0.25 * s2 / steps;  // a at dx = 1
     if (!(a1 <= 150.0 * dx * dx)) return w;
+    if (!(r > 0.25 * o.z * o.z * dx * dx * exp(xb))) return w;
     if (!(o.w < 0)) {
         const double xa = sqrt(a1 / 0.1) * per;  // about where a = 0.1
         const double from = xa > -xb ? xa : -xb;

@@ -1,0 +1,64 @@
+"""The in-the-money cut of the windowed march (csrc/fd1d_plan.h) over the rates at which it can be
+put too near the strike: an option whose exercise boundary passes its cut is marched twice.
+On the CPU, with the serial marches of tests/cpp/window_test.cpp."""
+from __future__ import annotations
+
+import pathlib
+import subprocess
+
+import numpy as np
+import pytest
+
+from kwgpu.workloads import OPTION_DTYPE
+
+ROOT = pathlib.Path(__file__).resolve().parents[1]
+TOL = 1e-11  # as in test_window.py
+
+
+@pytest.fixture(scope="module")
+def cases(tmp_path_factory):
+    """cases(options, x_dim, t_dim): per option lo, end, pinned, inside, the price on the window
+    as it is and the price on the whole grid."""
+    exe = str(tmp_path_factory.mktemp("cases") / "window_cases")
+    subprocess.run(["g++", "-O3", "-std=c++17", f"-I{ROOT / 'include'}",
+                    str(ROOT / "tests" / "cpp" / "window_cases.cpp"), "-o", exe], check=True)
+
+    def run(o, x_dim, t_dim, *mesh):
+        text = "\n".join(" ".join(repr(float(o[c][i])) if c not in "ew" else str(int(o[c][i]))
+                                  for c in ("t", "k", "z", "r", "q", "s", "e", "w"))
+                         for i in range(len(o)))
+        out = subprocess.run([exe, str(x_dim), str(t_dim), *map(str, mesh)], input=text, text=True,
+                             capture_output=True, check=True, timeout=300).stdout
+        return np.array([[float(v) for v in ln.split()] for ln in out.splitlines()])
+    return run
+
+
+def draw(n, seed, rate, vol):
+    """American puts and calls whose early exercise is worth something: `rate` is a put's rate
+    and a call's yield, log-uniform."""
+    g = np.random.default_rng(seed)
+    o = np.zeros(n, OPTION_DTYPE)
+    o["t"] = np.exp(g.uniform(np.log(0.01), np.log(10.0), n))
+    o["k"] = 100.0
+    o["z"] = g.uniform(*vol, n)
+    o["s"] = 100 * np.exp(g.uniform(-1.0, 1.0, n) * np.minimum(1.0, 3 * o["z"] * np.sqrt(o["t"])))
+    o["e"] = 1
+    o["w"] = np.where(g.random(n) < 0.5, -1, 1)
+    earns = np.exp(g.uniform(*np.log(rate), n))
+    pays = np.select([np.arange(n) % 3 == 0, np.arange(n) % 3 == 1], [0.0, earns * g.random(n)],
+                     g.uniform(-0.01, 0.05, n))
+    o["r"] = np.where(o["w"] < 0, earns, pays)
+    o["q"] = np.where(o["w"] < 0, pays, earns)
+    return o
+
+
+@pytest.mark.parametrize("rate", [(1e-5, 1e-4), (1e-4, 1e-3), (1e-3, 1e-2), (1e-2, 0.25)])
+@pytest.mark.parametrize("vol", [(0.03, 0.3), (0.3, 0.8), (0.8, 1.6)])
+@pytest.mark.parametrize("x_dim,t_dim,n", [(512, 300, 400), (1024, 66, 400)])
+def test_few_boundaries_pass_their_cut(cases, x_dim, t_dim, n, rate, vol):
+    c = cases(draw(n, x_dim + int(1e6 * rate[0]), rate, vol), x_dim, t_dim)
+    cut = c[:, 0] > 0
+    assert cut.sum() > 0.1 * n
+    assert np.sum(cut & (c[:, 2] == 0)) <= 0.02 * cut.sum()
+    ok = (c[:, 2] == 1) & (c[:, 3] == 1)
+    assert np.max(np.abs(c[ok, 4] - c[ok, 5]) / np.maximum(100.0, c[ok, 5])) <= TOL
