@@ -81,29 +81,32 @@ KWGPU_HD float critical_log_spot(float t, float z, float r, float q) {
 // error of e^-36 = 2e-16. Where the steps are few Crank-Nicolson's tails are heavier than
 // the Gaussian's: at 64 steps the exponent 36 loses 2 n (y^3/3 + ...), y = 36 / (2 n), 0.9.
 //
-// In the money the cut lies 0.25 sigma sqrt(T) / (1 + sqrt(a / 0.06)), a = r sqrt(T) / sigma, in
-// log S and 2 rows past the approximate critical spot. The boundary ends past that spot by more
-// the smaller a is: over 2256 marches (1024 x 512, vol 2-200 %, T 0.005-20 years, rates 1e-5 to
-// 25 %) by at most 0.20 sigma sqrt(T) and 2 rows at a < 1e-5, 0.14 at 1e-3, 0.09 at 0.1 and 0.02
-// at 1. Of 50000 cuts on 129 to 2048 points (rates 1e-7 to 50 %, yields below and above them by
-// any factor) 27 were passed. A cut that is too near costs a second march after
-// the first, which a whole launch may wait for (0.5 ms of 2.2 for one option of 16384); the
-// margin costs about 6 rows of 1024. The cut needs
+// In the money the cut lies 0.18 sigma sqrt(T) / (1 + sqrt(a / 6)), a = r sqrt(T) / sigma, in log S
+// and 2 rows past the approximate critical spot. The boundary ends past that spot by more the
+// smaller a is: over 5000 marches on 2048 points laid close to the strike (vol 0.3-150 %, T 0.001-20
+// years, rates 1e-4 to 90 %) by a row and at most 0.16 sigma sqrt(T) at a < 0.01, 0.12 at 0.2, 0.09
+// at 2 and 0.02 beyond 10. A cut that is too near costs a second march after the first, which a
+// whole launch may wait for (0.5 ms of 2.2 for one option of 16384); the margin costs about 8
+// rows of 1024. The cut needs
 //   * kPinnedRows rows to forget the approximate value they are started from: with
 //     a = theta dt (sigma^2 / 2) / dx^2 at the cut, an error shrinks by about
 //     e^{-1/sqrt(a)} per row, and a <= 150 leaves 1e-9 of an error of O(dt^2);
-//   * the mesh to see the early exercise: a put's payoff falls behind at r in the money, and the
-//     differences are off there by about sigma^2 dx^2 S / 4; where that is more than r, no row
-//     stays pinned;
 //   * early exercise to be worth something: while q > r the boundary never comes nearer than
 //     log(r / q) to the strike, and past 4.5 sigma sqrt(T) the premium is below about 1e-9 of
 //     the price. Such an option keeps the rows its European twin keeps, and with them the
 //     same arithmetic, so that rounding cannot price it below the twin (on 32768 options at
 //     1024 x 1024 the two had differed by up to 9e-11, the smallest such ratio 5.1). At a < 1e-3 the
 //     approximation is off by up to 1.3 sigma sqrt(T) from a ratio of 0.5 on;
-//   * for a call, the unprojected edge row to be forgotten as well: its value can be
-//     e^{scale sigma sqrt(T)}, 22 sigma sqrt(T) decades, and a row with a < 0.1 takes off
-//     at least one.
+//   * the rows past it to be pinned in the scheme too: a payoff falls behind there at r (a call's:
+//     at r S) less what waiting earns and what the differences are off by. A put's error is largest
+//     near the strike; a call's grows with S and dx, and from xc on, where it reaches r / 2, the
+//     rows are not pinned and carry more than the payoff;
+//   * those rows of a call, and its unprojected edge row, to be forgotten: their values are
+//     e^{x - |xb|} of the cut's, a row with a < 0.1 takes off at least a decade, and 20 more leave
+//     nothing. (Without these two, 1 of 2500 cuts of calls in a search over long maturities, coarse
+//     grids and yields far below the rate held although they should not have: deep in the money
+//     prices were off by up to 2 %. With them 277000 cuts of that search and 565000 windows of a
+//     wider one on the CPU are at most 3e-15 of max(K, price) from the whole grid, none passed.)
 KWGPU_HD Window window_of(const kwgpu_option& o, int N, int steps, double density, double scale,
                           double far) {
     Window w{0, N};
@@ -131,7 +134,7 @@ KWGPU_HD Window window_of(const kwgpu_option& o, int N, int steps, double densit
     const double a0 = r * o.t / s;  // r sqrt(T) / sigma
     if (q > r && log(q / r) > (a0 < 1e-3 ? 0.5 : 4.5) * s) return w;
     const double xb = (double)critical_log_spot((float)o.t, (float)o.z, (float)r, (float)q) -
-                      0.25 * s / (1.0 + sqrt(a0 / 0.06));
+                      0.18 * s / (1.0 + sqrt(a0 / 6.0));
     if (!(xb > -6.9)) return w;  // nor when it is no number
     const double at = (asinh(xb / density) + Y) * per;
     const int lo = (int)floor(at) - 2;
@@ -139,11 +142,26 @@ KWGPU_HD Window window_of(const kwgpu_option& o, int N, int steps, double densit
     const double dx = sqrt(xb * xb + density * density) * h;
     const double a1 = 0.25 * s2 / steps;  // a at dx = 1
     if (!(a1 <= 150.0 * dx * dx)) return w;
-    if (!(r > 0.25 * o.z * o.z * dx * dx * exp(xb))) return w;
-    if (!(o.w < 0)) {
-        const double xa = sqrt(a1 / 0.1) * per;  // about where a = 0.1
-        const double from = xa > -xb ? xa : -xb;
-        if (!((Y - asinh(from / density)) * per >= 22.0 * s + 20.0)) return w;
+    // the differences of the payoff's exponential, at spacing d = h sqrt(x^2 + density^2) that
+    // grows by h^2 |x| a row, are off by c h^2 of it; half as much again for higher orders
+    const float xf = (float)xb, rf = (float)r, den = (float)density, d2 = den * den;
+    const float up = fmaxf((float)mu, 0.0f), z2 = (float)(o.z * o.z), h2 = 1.5f * (float)(h * h);
+    const float idle = fmaxf((float)q, 0.0f);  // what waiting earns of S
+    if (o.w < 0) {
+        const float u = fmaxf(-xf, 1.0f), v = fmaxf(-xf, 2.0f);  // largest |x| e^x, x^2 e^x past the cut
+        const float off = h2 * ((z2 / 6 + up / 2) * u * expf(-u) +
+                                fmaxf(-(float)mu, 0.0f) / 6 * (v * v * expf(-v) + d2 * expf(xf)));
+        if (!(rf > idle * expf(xf) + off)) return w;
+    } else {
+        const float a = z2 / 6 + up / 2, b = z2 / 24 + up / 6;  // c = a x + b (x^2 + density^2)
+        if (!(rf > idle * expf(xf) + h2 * (b * (xf * xf + d2) - a * xf))) return w;
+        const float xc = 0.5f * (sqrtf(fmaxf(0.0f, a * a - 4 * b * (b * d2 - 0.5f * rf / h2))) - a) / b;
+        if (!(0.5f * rf > idle * expf(-xc))) return w;
+        const float n = (float)per, xa = sqrtf((float)a1 / 0.1f) * n;  // about where a = 0.1
+        const float from = asinhf(fmaxf(xa, -xf) / den), edge = (float)(scale * s), end = fminf(xc, edge);
+        if (!((asinhf(end / den) - from) * n >= (end + xf) / 2.3f + 20.0f &&
+              ((float)Y - from) * n >= (edge + xf) / 2.3f + 20.0f))
+            return w;
     }
     w.lo = lo;
     return w;

@@ -62,3 +62,25 @@ def test_few_boundaries_pass_their_cut(cases, x_dim, t_dim, n, rate, vol):
     assert np.sum(cut & (c[:, 2] == 0)) <= 0.02 * cut.sum()
     ok = (c[:, 2] == 1) & (c[:, 3] == 1)
     assert np.max(np.abs(c[ok, 4] - c[ok, 5]) / np.maximum(100.0, c[ok, 5])) <= TOL
+
+
+@pytest.mark.parametrize("x_dim,t_dim", [(256, 66), (400, 90), (512, 130), (777, 70), (1024, 66)])
+def test_calls_of_long_maturity_and_low_yield(cases, x_dim, t_dim):
+    """Far in the money a call's payoff grows with the spot, and so does what the differences are
+    off by there: past some row the scheme never exercises, and a cut must not take those rows for
+    pinned. Spots deep in the money, near the boundary, and at the strike."""
+    g = np.random.default_rng(x_dim)
+    n = 600
+    o = np.zeros(n, OPTION_DTYPE)
+    s = g.uniform(0.8, 1.8, n)
+    o["z"] = g.uniform(0.25, 0.7, n)
+    o["t"] = (s / o["z"]) ** 2
+    o["k"], o["e"], o["w"] = 100.0, 1, 1
+    o["r"] = g.uniform(1.0, 3.5, n) / o["t"]
+    o["q"] = o["r"] * np.exp(-g.uniform(2.0, 4.4, n) * s)
+    o["s"] = 100 * np.where(np.arange(n) % 4 == 0, 1.0, np.exp(g.uniform(3.0, 4.9, n) * s))
+    c = cases(o, x_dim, t_dim)
+    cut = c[:, 0] > 0
+    assert np.sum(cut & (c[:, 2] == 0)) <= 0.02 * n
+    ok = (c[:, 2] == 1) & (c[:, 3] == 1)
+    assert np.max(np.abs(c[ok, 4] - c[ok, 5]) / np.maximum(100.0, c[ok, 5])) <= TOL
