@@ -112,13 +112,24 @@ KWGPU_HD Window window_of(const kwgpu_option& o, int N, int steps, double densit
     Window w{0, N};
     const double s = o.z * sqrt(o.t), s2 = s * s;
     const double mu = o.r - o.q - 0.5 * o.z * o.z;
-    // the domain: a march long enough to pay for a second set-up, no overflow anywhere on
-    // the mesh, a drift within a few standard deviations, ordinary rates
+    // the domain: a march long enough to pay for a second set-up, a drift within a few
+    // standard deviations, ordinary rates
     if (!(steps >= kWindowMinSteps && N >= 128 && s > 0.0 && scale * s <= 150.0 && scale >= 10.0 &&
           fabs(mu) * o.t <= 3.0 * s && fabs(o.r) <= 1.0 && fabs(o.q) <= 1.0 && far < 1e6))
         return w;
+    // ... and no overflow anywhere on the whole mesh, which a march reports and a window that
+    // leaves those rows out cannot: a solution starts at up to e^150 (above), grows with the
+    // rates by up to e^21 (20 in 64 steps or more), and at a mesh edge, whose one-sided drift may
+    // run inward, by e^{1.1 |mu| T / dx} while a step's share is at most 1: e^480 of the e^709 that
+    // FP64 holds (largest of 520000 marches: 1e72)
+    if (!(fabs(o.r) * o.t <= 20.0 && fabs(o.q) * o.t <= 20.0)) return w;
     const double Y = asinh(scale * s / density), h = 2.0 * Y / (N - 1);  // mesh step in y
     const double per = 1.0 / h;
+    {
+        const float x = (float)(scale * s), dx = sqrtf(x * x + (float)(density * density)) * (float)h;
+        const float drift = (float)(fabs(mu) * o.t) / dx;
+        if (!(drift <= (float)steps && drift <= 280.0f)) return w;
+    }
     {
         const double u = far > 0.0 ? far : 0.0;
         const double b = 0.5 * (u + sqrt(u * u + 4.0 * 18.0 * s2));

@@ -142,7 +142,8 @@ __device__ __forceinline__ void pinned_edge(const FdBatch& b, const PdeParams& P
 // One wave's (W = 2: one workgroup's) work: the options ids[slot] .. (or slot itself without
 // ids), at most `slots`, each on its window (from rec[p], or lo_all when rec is null). Bit k
 // of the result: segment k's option has to be solved again on its whole grid (what was
-// written for it does not stand).
+// written for it does not stand): its boundary passed the cut, its price is asked for outside
+// the window, or a value is not finite.
 template <int M, int L, int W = 1>
 __device__ __forceinline__ unsigned solve_window(const FdBatch& b, const uint32_t* ids,
                                                  const int* rec, int lo_all, int slot0, int slots,
@@ -201,10 +202,13 @@ __device__ __forceinline__ unsigned solve_window(const FdBatch& b, const uint32_
         double2* qpv = reinterpret_cast<double2*>(qp);
 #pragma unroll
         for (int i = 0; i < M; ++i) {
-            // every row but the grid's last is projected: row N - 1 is a put's last position
-            // and a call's first
+            // every row but one is projected. On a whole grid that is row N - 1, a put's last
+            // position and a call's first; behind a cut it is the window's last, whose value is
+            // about 0 either way: the projection turns a NaN into the payoff, so the row left
+            // without it is what carries one on to the end
             const int at = d.j0 + i;
-            const bool proj = d.P.american && at < d.N && at != (d.P.call ? 0 : d.N - 1);
+            const bool proj = d.P.american && at < d.N &&
+                              at != (d.P.call && edge.lo == 0 ? 0 : min(edge.lo + LT * M, d.N) - 1);
             qpv[i * NT + t.gl] = make_double2(Q[i], proj ? xv[i] : -INFINITY);
         }
         if constexpr (W == 2) qpv[M * NT + t.gl] = make_double2(aw, bw);
@@ -225,7 +229,9 @@ __device__ __forceinline__ unsigned solve_window(const FdBatch& b, const uint32_
     bool bad = false;
 #pragma unroll
     for (int i = 0; i < M; ++i) bad |= d.j0 + i < d.N && !isfinite(xv[i]);
-    const bool seg_bad = segments(bad) >> t.seg & 1;
+    const unsigned nonfinite = segments(bad);
+    const bool seg_bad = nonfinite >> t.seg & 1;
+    again |= nonfinite & segments(lo > 0 || LT * M < d.N);  // the whole grid decides
     group_sync<W>();
 #pragma unroll
     for (int i = 0; i < M; ++i) qp[t.seg * LT * M + t.ls * M + i] = xv[i];

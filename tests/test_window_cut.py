@@ -84,3 +84,67 @@ def test_calls_of_long_maturity_and_low_yield(cases, x_dim, t_dim):
     assert np.sum(cut & (c[:, 2] == 0)) <= 0.02 * n
     ok = (c[:, 2] == 1) & (c[:, 3] == 1)
     assert np.max(np.abs(c[ok, 4] - c[ok, 5]) / np.maximum(100.0, c[ok, 5])) <= TOL
+
+
+def extreme(n, seed):
+    """Maturities and rates at which the march on a whole grid can overflow, the drift small: cost
+    of carry near half the variance. Sizes too: x points and t points."""
+    g = np.random.default_rng(seed)
+    o = np.zeros(n, OPTION_DTYPE)
+    s = 3.0 * np.exp(g.uniform(np.log(1e-3), 0.0, n))
+    o["t"] = np.exp(g.uniform(np.log(100.0), np.log(1000.0), n))
+    o["k"] = o["s"] = 100.0
+    o["z"] = s / np.sqrt(o["t"])
+    o["r"] = g.uniform(-0.99, -0.2, n)
+    o["q"] = o["r"] - 0.5 * o["z"] ** 2 - 2.9 * s / o["t"] * g.uniform(-1, 1, n)
+    o["e"] = np.arange(n) % 4 != 0
+    o["w"] = np.where(g.random(n) < 0.5, -1, 1)
+    return o, g.integers(129, 1024, n), g.integers(66, 500, n)
+
+
+def test_no_window_where_the_whole_grid_overflows(cases):
+    o, xd, td = extreme(400, 1)
+    over = 0
+    for i in range(len(o)):
+        lo, end, _, _, _, whole = cases(o[i:i + 1], xd[i], td[i])[0]
+        if not np.isfinite(whole):
+            over += 1
+            assert (lo, end) == (0, xd[i]), (o[i], xd[i], td[i])
+    assert over >= 40
+
+
+@pytest.mark.gpu
+def test_overflow_is_reported(ctx, tmp_path):
+    """A march that overflows reports it, whichever launch form its batch takes: the statuses are
+    those of the whole-grid kernels (the oracle eliminates serially, and overflows for nearly
+    the same options)."""
+    import torch
+
+    import kwgpu
+    import oracle
+    print("overflow", flush=True)
+    o, xd, td = extreme(1200, 2)
+    whole = kwgpu.Context(0)
+    (tmp_path / "tune").write_text("256 0 2 0\n512 0 5 0\n1024 0 8 0\n2048 0 9 0\n")
+    whole.tune_load(str(tmp_path / "tune"))
+    for cap in (1024, 512):  # a wave an option; with one grid of over 1024 points among them
+        m = 1200 if cap == 1024 else 500
+        x = np.minimum(xd[:m], cap).astype(np.int32)
+        if cap == 512:
+            x[0] = 1500
+        t = td[:m].astype(np.int32)
+        d_o = torch.from_numpy(o[:m].view(np.uint8).copy()).cuda()
+        d_x, d_t = torch.from_numpy(x).cuda(), torch.from_numpy(t).cuda()
+        prm = kwgpu.params(x_dims=d_x.data_ptr(), t_dims=d_t.data_ptr())
+        st = []
+        for c in (ctx, whole):
+            d_p = torch.zeros(m, dtype=torch.float64, device="cuda")
+            d_s = torch.full((m,), -1, dtype=torch.int32, device="cuda")
+            torch.cuda.synchronize()
+            c.fd1d_price_device(d_o.data_ptr(), m, d_p.data_ptr(), d_s.data_ptr(), prm)
+            c.synchronize()
+            st.append(d_s.cpu().numpy())
+        assert np.array_equal(st[0], st[1])
+        bad = ~np.isfinite(oracle.fd1d_price_uneven(o[:m], x, t)[0])
+        assert bad.sum() > 50 and np.mean(st[0][bad] == kwgpu.STATUS_NONFINITE) > 0.95
+    whole.close()
