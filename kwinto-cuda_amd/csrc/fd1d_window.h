@@ -312,8 +312,10 @@ __global__ __launch_bounds__(256) void plan_windows(FdBatch b, int* rec, int* co
         const int N = b.x_dims ? b.x_dims[oi] : b.x_dim;
         const int td = b.t_dims ? b.t_dims[oi] : b.t_dim;
         Window w{0, N};
-        if (!b.off || b.off[p + 1] - b.off[p] <= kFarOptions)
-            w = window_of(b.opts[oi], N, td - 1, b.density, b.scale, far_xi(b, p, oi, 0, 1));
+        const int pw = b.like ? (int)b.like[p] : p;
+        if (!b.off || b.off[pw + 1] - b.off[pw] <= kFarOptions)
+            w = window_of(b.opts[b.like ? b.rep[pw] : oi], N, td - 1, b.density, b.scale,
+                          far_xi(b, pw, oi, 0, 1));
         const int c = window_class(w.end - w.lo);
         rec[p] = w.lo | c << 16;
         atomicAdd(&n[c], 1);
@@ -376,9 +378,10 @@ __device__ __forceinline__ LoneWindow lone_window(const FdBatch& b, int slot) {
     const uint32_t oi = b.rep ? b.rep[p] : (uint32_t)p;
     const int N = b.x_dims ? b.x_dims[oi] : b.x_dim;
     const int td = b.t_dims ? b.t_dims[oi] : b.t_dim;
-    double far = far_xi(b, p, oi, threadIdx.x & 63, 64);
+    const int pw = b.like ? (int)b.like[p] : p;
+    double far = far_xi(b, pw, oi, threadIdx.x & 63, 64);
     for (int k = 32; k > 0; k >>= 1) far = fmax(far, __shfl_xor(far, k));
-    const Window w = window_of(b.opts[oi], N, td - 1, b.density, b.scale, far);
+    const Window w = window_of(b.opts[b.like ? b.rep[pw] : oi], N, td - 1, b.density, b.scale, far);
     return {__builtin_amdgcn_readfirstlane(w.lo), __builtin_amdgcn_readfirstlane(w.end - w.lo), N};
 }
 

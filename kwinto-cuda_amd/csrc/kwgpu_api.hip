@@ -276,7 +276,7 @@ uint64_t fnv_fields(uint64_t h, const T&... v) {
 uint64_t fnv_batch(uint64_t h, const FdBatch& b) {
     return fnv_fields(h, b.opts, b.rep, b.off, b.list, b.order, b.x_dims, b.t_dims, b.m, b.x_dim,
                       b.t_dim, b.density, b.scale, b.theta, b.prices, b.status, b.ws, b.ws_stride,
-                      b.ws_rows);
+                      b.ws_rows, b.like);
 }
 
 uint64_t fnv_bucket(uint64_t h, const Bucket& k) {
@@ -732,7 +732,8 @@ int fd_price_host(kwgpu_ctx* c, const kwgpu_option* opts, size_t n, const kwgpu_
     const size_t at_opts = carve(n * sizeof(kwgpu_option)), at_rep = carve(m * sizeof(uint32_t)),
                  at_off = carve((m + 1) * sizeof(uint32_t)), at_list = carve(n * sizeof(uint32_t)),
                  at_x = uneven ? carve(n * sizeof(int32_t)) : 0,
-                 at_t = uneven ? carve(n * sizeof(int32_t)) : 0, in_bytes = bytes,
+                 at_t = uneven ? carve(n * sizeof(int32_t)) : 0,
+                 at_like = combine ? carve(m * sizeof(uint32_t)) : 0, in_bytes = bytes,
                  at_prices = carve(n * sizeof(double)), at_status = carve(n * sizeof(int32_t));
     hipError_t e;
     if ((e = ensure(c->in, in_bytes)) != hipSuccess ||
@@ -760,6 +761,15 @@ int fd_price_host(kwgpu_ctx* c, const kwgpu_option* opts, size_t n, const kwgpu_
             pde_t[k] = ht[rep[k]];
         }
     }
+    if (combine) {
+        // both legs on the European one's window, so that they march the same rows in the same
+        // lanes and round alike: each on its own, their difference's error was ten times as large
+        uint32_t* like = (uint32_t*)(h + at_like);
+        std::vector<uint32_t> pde(n);
+        for (size_t k = 0; k < m; ++k)
+            for (uint32_t i = off[k]; i < off[k + 1]; ++i) pde[list[i]] = (uint32_t)k;
+        for (size_t k = 0; k < m; ++k) like[k] = rep[k] < n / 2 ? pde[rep[k] + n / 2] : (uint32_t)k;
+    }
     if ((e = hipMemcpyAsync(d, h, in_bytes, hipMemcpyHostToDevice, s))) {
         (void)hipStreamSynchronize(s);
         return hip_fail(c, e, "kwgpu: upload");
@@ -778,6 +788,7 @@ int fd_price_host(kwgpu_ctx* c, const kwgpu_option* opts, size_t n, const kwgpu_
     b.theta = p->theta;
     b.prices = (double*)d_out;
     b.status = (int32_t*)(d_out + (at_status - at_prices));
+    if (combine) b.like = (const uint32_t*)(d + at_like);
     if (uneven) {
         b.x_dims = (const int32_t*)(d + at_x);
         b.t_dims = (const int32_t*)(d + at_t);

@@ -30,6 +30,8 @@ struct FdBatch {
     double* ws;             // lane layout workspace (null for the wave layout)
     long long ws_stride;    // slots per workspace row (>= m)
     int ws_rows;            // rows per workspace array (>= every x_dim in the batch)
+    const uint32_t* like;   // per PDE, with rep and off: the PDE whose option and spots decide its
+                            // window; null = itself
 };
 
 // Limits of the FP32-mixed march. Both depend only on the PDE (T, sigma, r, q) and the
