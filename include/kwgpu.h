@@ -219,7 +219,8 @@ int kwgpu_fd1d_autotune(kwgpu_ctx* ctx, const kwgpu_option* d_opts, size_t n,
                         char* report, size_t report_len);
 
 /* Saves / loads the context's autotuned choices (text, one "bucket precision variant
- * persistent" line each). Loading skips lines of an unknown precision, variants that
+ * persistent" line each; before a windowed choice's line, -2, the fastest whole-grid variant's,
+ * which the bucket's batches without windows take). Loading skips lines of an unknown precision, variants that
  * do not exist or do not hold their bucket and lane-layout choices for FP32-mixed. */
 int kwgpu_tune_save(kwgpu_ctx* ctx, const char* path);
 int kwgpu_tune_load(kwgpu_ctx* ctx, const char* path);

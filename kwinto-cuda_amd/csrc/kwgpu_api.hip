@@ -33,6 +33,9 @@ constexpr int kLane = -1, kWindowed = -2;
 struct Choice {
     int variant = kLane;
     bool persist = true;
+    // beside kWindowed: the tuned whole-grid variant, for batches that take no windows (none: -1)
+    int whole = -1;
+    bool whole_persist = true;
 };
 
 // One launch of an uneven batch: PDEs order[begin, begin + count) of one bucket.
@@ -212,16 +215,22 @@ bool uniform_windowed(size_t m, int x_dim, int t_dim) {
     return steps >= kLongMarch || (double)m * x_dim * steps >= 5e8;
 }
 
+// The whole-grid march in place of windowed choice `ch`.
+Choice whole_choice(const Choice& ch, int cap) {
+    return ch.whole >= 0 ? Choice{ch.whole, ch.whole_persist}
+                         : Choice{kwgpu::default_wave_variant(cap), true};
+}
+
 Choice choice_for(const kwgpu_ctx* c, int cap, int precision, int layout, double theta) {
     Choice ch;
     if (cap == kLaneCap) return ch;  // lane layout
     const bool windowed = windowed_fits(cap, precision, theta);
     auto it = c->tuned.find({cap, precision});
-    if (it != c->tuned.end() && !(layout == KWGPU_LAYOUT_WAVE_REG && it->second.variant == kLane) &&
-        !(it->second.variant == kWindowed && !windowed))
-        return it->second;
-    ch.variant = windowed ? kWindowed : kwgpu::default_wave_variant(cap);
-    ch.persist = !windowed;
+    if (it != c->tuned.end() && !(layout == KWGPU_LAYOUT_WAVE_REG && it->second.variant == kLane))
+        return it->second.variant == kWindowed && !windowed ? whole_choice(it->second, cap) : it->second;
+    if (!windowed) return whole_choice(ch, cap);
+    ch.variant = kWindowed;
+    ch.persist = false;
     return ch;
 }
 
@@ -450,7 +459,7 @@ int run_fd_on(kwgpu_ctx* c, FdBatch b, const int32_t* pde_x, const int32_t* pde_
                     return hip_fail(c, e, "kwgpu: windowed kernel launch");
                 return KWGPU_OK;
             }
-            ch.variant = kwgpu::default_wave_variant(cap);
+            ch = whole_choice(ch, cap);
         }
         if (ch.variant == kLane) {
             const size_t need = kwgpu::lane_workspace_doubles(b.m, b.x_dim) * sizeof(double);
@@ -1246,7 +1255,7 @@ int kwgpu_fd1d_price_device_noalloc(kwgpu_ctx* c, const kwgpu_option* d_opts, si
         const int cap = bucket_of(p->x_dim, p->precision, p->layout);
         Choice ch = choice_for(c, cap, p->precision, p->layout, p->theta);
         if (ch.variant == kWindowed && !takes_windows(n, p->x_dim, p->t_dim, s))
-            ch = Choice{kwgpu::default_wave_variant(cap), true};
+            ch = whole_choice(ch, cap);
         if (capturing(s)) ch.persist = false;  // a persistent grid's work counter is scratch
         plan.push_back(Bucket{cap, ch, 0, n, p->x_dim, p->precision, p->x_dim > 1024 ? (int)n : 0});
     } else {
@@ -1473,7 +1482,17 @@ int kwgpu_fd1d_autotune(kwgpu_ctx* c, const kwgpu_option* d_opts, size_t n,
         const Cand* best = &cands[0];
         for (const auto& cd : cands)
             if (cd.ms < 0.98f * best->ms) best = &cd;
-        c->tuned[{cap, prec}] = best->ch;
+        Choice pick = best->ch;
+        if (pick.variant == kWindowed) {
+            const Cand* whole = nullptr;
+            for (const auto& cd : cands)
+                if (cd.ch.variant >= 0 && (!whole || cd.ms < 0.98f * whole->ms)) whole = &cd;
+            if (whole) {
+                pick.whole = whole->ch.variant;
+                pick.whole_persist = whole->ch.persist;
+            }
+        }
+        c->tuned[{cap, prec}] = pick;
         char buf[256];
         js += first_bucket ? "" : ", ";
         first_bucket = false;
@@ -1551,8 +1570,11 @@ int kwgpu_tune_save(kwgpu_ctx* c, const char* path) {
     if (!c || !path) return KWGPU_ERR_INVALID;
     FILE* f = std::fopen(path, "w");
     if (!f) return fail(c, KWGPU_ERR_INVALID, std::string("cannot write ") + path);
-    for (const auto& [k, ch] : c->tuned)
+    for (const auto& [k, ch] : c->tuned) {
+        if (ch.variant == kWindowed && ch.whole >= 0)  // the line before its own
+            std::fprintf(f, "%d %d %d %d\n", k.first, k.second, ch.whole, ch.whole_persist ? 1 : 0);
         std::fprintf(f, "%d %d %d %d\n", k.first, k.second, ch.variant, ch.persist ? 1 : 0);
+    }
     for (const auto& [prec, serial] : c->serial)  // bucket -1: the bucket schedule
         std::fprintf(f, "%d %d %d %d\n", -1, prec, serial ? 1 : 0, 0);
     std::fclose(f);
@@ -1575,7 +1597,12 @@ int kwgpu_tune_load(kwgpu_ctx* c, const char* path) {
         if (v < kWindowed || (v == kWindowed && !windowed_fits(cap, prec, 0.5))) continue;
         if (v >= kwgpu::wave_variant_count() || (v >= 0 && kwgpu::wave_variant(v).capacity() != cap)) continue;
         if (v < 0 && prec != KWGPU_FP64) continue;
-        c->tuned[{cap, prec}] = Choice{v, per != 0};
+        Choice& ch = c->tuned[{cap, prec}];
+        if (v == kWindowed)  // a whole-grid choice before it stands for batches without windows
+            ch = ch.variant >= 0 ? Choice{v, per != 0, ch.variant, ch.persist}
+                                 : Choice{v, per != 0, ch.whole, ch.whole_persist};
+        else
+            ch = Choice{v, per != 0};
     }
     std::fclose(f);
     drop_graph(c);

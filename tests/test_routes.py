@@ -77,3 +77,18 @@ def test_tune_file_with_an_unknown_march(routes, tmp_path, variant):
     f.write_text("512 0 -1 0\n")
     for k in routes(f"tune {f}", "price 3000 512 400", "uneven 300 90 100,256,512,2048")[1:]:
         assert any("fd1d_lane" in x for x in k) and "null workspace" not in k
+
+
+def test_tuned_whole_grid_march_beside_windows(routes, tmp_path):
+    """Where a bucket is tuned to the windowed march, its calls that take no windows (short or small
+    uniform batches, Greeks, capture) keep the tuned whole-grid variant; so they do after a save
+    and a load."""
+    f, g = tmp_path / "tune", tmp_path / "saved"
+    f.write_text("512 0 7 0\n512 0 -2 0\n256 0 4 1\n256 0 -2 0\n")
+    calls = ["price 2400 512 66", "noalloc 2400 512 66", "price 400 512 40", "greeks 40 512 90", "price 3000 512 512"]
+    loaded = routes(f"tune {f}", f"save {g}", *calls, "capture 1", "price 3000 512 512")[2:]
+    again = routes(f"tune {g}", *calls, "capture 1", "price 3000 512 512")[1:]
+    assert loaded == again
+    for k in (*loaded[:4], loaded[6]):
+        assert any(x.startswith("fd1d_wave<8, 64, 1") for x in k), k
+    assert "fd1d_windowed" in loaded[4]
