@@ -256,7 +256,8 @@ def bench_uneven(ctx, torch, stream, n, steps, log):
                      "roofline_frac": flops / (ms * 1e-3) / 1e12 / peak,
                      "autotuned": {str(k): v for k, v in chosen.items()},
                      "autotune_trials": trials,
-                     "bucket_schedule": tune.get("schedule")}
+                     "bucket_schedule": tune.get("schedule"),
+                     "windowed_together": tune.get("windowed_together")}
         log(f"bench: uneven {name} {ms:.3f} ms/step")
     d = np.abs(prices["fp32_mixed"] - prices["fp64"])
     out["fp32_mixed"]["max_abs_err_vs_fp64_fd"] = float(d.max())

@@ -210,7 +210,9 @@ int kwgpu_fd1d_greeks(kwgpu_ctx* ctx, const kwgpu_option* opts, size_t n,
  * option: 4, 2 or 1 options per wave, or two waves per option), with a static and with
  * a persistent grid, and in FP64 also the lane layout and (theta 1/2, over 128 points) the
  * windowed march, which such grids take untuned; keeps the fastest per (bucket,
- * precision) in the context, which later calls use. `report` (may be NULL) receives a
+ * precision) in the context, which later calls use. The windowed march takes all its buckets
+ * in one launch, so a batch of several buckets is also timed with every bucket windowed that
+ * can be, and keeps that where it is faster ("windowed_together" in the report). `report` (may be NULL) receives a
  * JSON object with every timing. Device pointers as for kwgpu_fd1d_price_device (the
  * sampled options' prices are written); synchronous.
  */

@@ -92,3 +92,27 @@ def test_tuned_whole_grid_march_beside_windows(routes, tmp_path):
     for k in (*loaded[:4], loaded[6]):
         assert any(x.startswith("fd1d_wave<8, 64, 1") for x in k), k
     assert "fd1d_windowed" in loaded[4]
+
+
+def test_per_option_grids_take_the_windowed_forms(routes):
+    """The forms that test_window_forms.py and test_window_again.py are written for."""
+    lone, lone_big, listed, big, small = routes(
+        "uneven 64 130 512,512", "uneven 64 130 512,1500", "uneven 2400 130 512", "uneven 1400 130 512,2048",
+        "uneven 300 90 60,100")
+    assert "fd1d_lone" in lone and "plan_windows" not in lone
+    assert "fd1d_lone_big" in lone_big and "fd1d_window_again" in lone_big
+    assert [k for k in LISTED if k in listed] == LISTED
+    assert "fd1d_windowed_big" in big and "fd1d_window_again" in big
+    assert not any("window" in k or "lone" in k for k in small)
+
+
+def test_rule_for_uniform_batches(routes):
+    """Which uniform batches take the windowed march, at the lines of the rule."""
+    calls = {"price 1024 896 65": True, "price 1024 897 65": False, "price 1025 256 65": False,
+             "price 1025 257 65": True, "price 2048 256 99": False, "price 2048 256 100": True,
+             "price 2049 512 256": False, "price 2049 512 257": True, "price 512 1100 65": False,
+             "price 1024 1025 400": False, "price 1025 1025 65": True, "price 64 512 64": False,
+             "price 64 512 65": True, "price 64 128 400": False, "price 64 129 400": True,
+             "price 2049 2049 65": False, "greeks 300 512 512": False}
+    for call, k in zip(calls, routes(*calls)):
+        assert any("lone" in x or "windowed" in x for x in k) == calls[call], (call, k)
