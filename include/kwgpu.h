@@ -139,6 +139,14 @@ int kwgpu_fd1d_price(kwgpu_ctx* ctx, const kwgpu_option* opts, size_t n,
                      const kwgpu_fd1d_params* params, double* prices, int32_t* status);
 
 /*
+ * The same call with the same inputs gives the same bits. With the batch that an option is in
+ * its FP64 price can move by rounding (a few 1e-12 relative): the number of options, stream
+ * capture and the furthest spot among the options of its PDE decide which rows of the grid are
+ * marched and how a kernel splits them. A context keeps up to 16 MiB of pinned host memory for
+ * the host entry points' copies; larger calls copy from and to the caller's arrays.
+ */
+
+/*
  * Same pricing on device-resident buffers, one PDE per option (no compression),
  * asynchronous on `stream` (a hipStream_t; NULL = the context's stream).
  * d_status may be NULL. This is the throughput path.
@@ -253,7 +261,8 @@ void* kwgpu_stream(kwgpu_ctx* ctx);
  * FD pricer's values at those nodes.
  * The three 256x256 layers run on BF16 MFMA with FP32 accumulation (forward and
  * backward); the 8-wide input layer and the 1-wide output layer run in FP32; Adam
- * keeps FP32 master weights.
+ * keeps FP32 master weights. A surrogate keeps up to 64 MiB of training buffers between
+ * fits.
  * --------------------------------------------------------------------------------- */
 typedef struct kwgpu_surrogate kwgpu_surrogate;
 
