@@ -9,10 +9,7 @@ rounds a solve whose rows sum terms up to a few hundred times their result, 1.1e
 
 On the GPU, against the oracle to 1e-8: grids around the row counts that the march is built
 for, in both launch forms (one option to a wave; listed by class, with several to a wave),
-with options whose exercise boundary goes past their window's cut and are solved again.
-(Of these uniform batches the ones of few point-steps, and 64 options on 1000 points and above, take
-the whole-grid kernels by the rule of choice; and the boundaries of PAST_THE_CUT stay within the cuts as
-they are placed now. test_window_forms.py and test_window_again.py reach the forms themselves.)"""
+with options whose exercise boundary goes past their window's cut and are solved again."""
 from __future__ import annotations
 
 import os

@@ -1,7 +1,8 @@
 """Every launch form of the windowed march over the row counts that it is built for. Per-option grid
 sizes always take the windowed march (test_window.py's uniform batches mostly do not: those of
 few point-steps take the whole-grid kernels, which test_routes.py and the last test here hold);
-the oracle is met to 1e-8, as there. And the windowed bucket of an uneven batch beside others."""
+the oracle is met to 1e-8, as there. (Its PAST_THE_CUT boundaries stay within the cuts as they are
+placed now; test_window_again.py has options that pass theirs.) And the windowed bucket of an uneven batch beside others."""
 from __future__ import annotations
 
 import numpy as np
